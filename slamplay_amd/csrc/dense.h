@@ -30,10 +30,10 @@
 #include "mfma.h"
 #include "pair_block.h"
 #include "solver.h"
+#include "tile_chol.h"
 
 namespace mba {
 
-constexpr int kTile = 32;
 constexpr int kJs = 36;  // per-observation stride of Jc~ (18, by columns), Jp~ (6), Hp (6), I - G (3)
 static_assert(kJs == RecLayout<kRecDense>::stride, "the dense record is pair_block's kRecDense");
 
@@ -123,60 +123,28 @@ __device__ __forceinline__ typename Mfma<F>::acc tile_mma_nt(const F* __restrict
     return c;
 }
 
-// Factors the tile held in T (lower triangle used) with one wave and writes L (lower triangle of
-// diagonal tile k of A) and X = L^-1 (Dinv[k], row-major, zero above the diagonal).  Lane r < 32
-// keeps row r in registers; the pivot and the entries l_cj of the scaled column j are the same
-// for every lane and are read from their lanes with v_readlane, so the factorization makes no
-// trip through LDS.  X is formed by columns: lane c < 32 solves L x = e_c by forward substitution
-// (x[m] = 0 for m < c follows by itself) with L broadcast from LDS.  Returns false (and writes
-// nothing) when a pivot is not positive and finite.  Only wave 0 may call it; lanes 32..63 repeat
-// the work of lanes 0..31 and store nothing.
+// Factors the tile held in T (lower triangle used) with one wave and writes X = L^-1 (Dinv[k],
+// row-major, zero above the diagonal); L itself is not kept, nothing reads a factored diagonal tile.
+// Lane r < 32 keeps row r of the tile in registers, lane 32 + i row i of the identity: the column
+// operations that turn the tile into L (column j scaled by 1 / l_jj, column c less l_cj times column j)
+// turn the identity below it into L^-T, whose row i is column i of X, so the inverse costs no
+// instructions of its own.  The pivot and the entries l_cj of the scaled column are read from their
+// lanes with v_readlane: no trip through LDS and no serial sum.  Entries above the tile's diagonal are
+// updated with the rest and never read by another lane.  Returns false (and writes nothing) when a
+// pivot is not positive and finite.  Only one whole wave may call it.
 template <typename F>
-__device__ __forceinline__ bool potrf_tile_wave(F (*T)[kTile + 1], F* dl, F* __restrict__ A, int ld, int k,
-                                                F* __restrict__ Dinv) {
+__device__ __forceinline__ bool potrf_tile_wave(F (*T)[kTile + 1], F* __restrict__ X) {
     const int l = threadIdx.x & 63, r = l & 31;
     F a[kTile];
 #pragma unroll
-    for (int c = 0; c < kTile; ++c) a[c] = T[r][c];
-    bool bad = false;
-#pragma unroll
-    for (int j = 0; j < kTile; ++j) {
-        const F d = read_lane(a[j], j);
-        const bool nonpos = !(d > (F)0) || !isfinite((double)d);
-        bad |= nonpos;
-        const F dd = nonpos ? (F)1 : d, inv = inv_sqrt(dd), ljj = dd * inv;
-        a[j] = r > j ? a[j] * inv : (r == j ? ljj : (F)0);
-        if (l == 0) dl[j] = inv;
-#pragma unroll
-        for (int c = j + 1; c < kTile; ++c) {
-            const F lcj = read_lane(a[j], c);
-            if (r >= c) a[c] -= a[j] * lcj;
-        }
+    for (int c = 0; c < kTile; ++c) {
+        const F t = T[r][c];
+        a[c] = l < kTile ? t : (r == c ? (F)1 : (F)0);
     }
-    if (bad) return false;
+    if (!potrf_stacked<F>(a)) return false;
+    if (l >= kTile)
 #pragma unroll
-    for (int c = 0; c < kTile; ++c) T[r][c] = c <= r ? a[c] : (F)0;
-    wave_sync_lds();
-    const size_t o = (size_t)(kTile * k) * ld + kTile * k;
-    for (int idx = l; idx < kTile * kTile; idx += 64) {
-        const int rr = idx / kTile, cc = idx % kTile;
-        if (cc <= rr) A[o + (size_t)rr * ld + cc] = T[rr][cc];
-    }
-    F x[kTile];
-#pragma unroll
-    for (int m = 0; m < kTile; ++m) {
-        F p0 = 0, p1 = 0;
-#pragma unroll
-        for (int q = 0; q + 1 < m; q += 2) {
-            p0 += T[m][q] * x[q];
-            p1 += T[m][q + 1] * x[q + 1];
-        }
-        if (m & 1) p0 += T[m][m - 1] * x[m - 1];
-        x[m] = ((m == r) ? (F)1 - (p0 + p1) : -(p0 + p1)) * dl[m];
-    }
-    if (l < kTile)
-#pragma unroll
-        for (int m = 0; m < kTile; ++m) Dinv[(size_t)k * kTile * kTile + m * kTile + r] = x[m];
+        for (int m = 0; m < kTile; ++m) X[m * kTile + r] = a[m];
     return true;
 }
 
@@ -185,12 +153,11 @@ template <typename F>
 __global__ void __launch_bounds__(64) k_potrf_tile(F* __restrict__ A, int ld, int k, F* __restrict__ Dinv, LMState* st) {
     if (st->done || st->step_invalid) return;
     __shared__ F T[kTile][kTile + 1];
-    __shared__ F dl[kTile];
     const int l = threadIdx.x;
     const size_t o = (size_t)(kTile * k) * ld + kTile * k;
     for (int idx = l; idx < kTile * kTile; idx += 64) T[idx / kTile][idx % kTile] = A[o + (size_t)(idx / kTile) * ld + idx % kTile];
     __syncthreads();
-    if (!potrf_tile_wave<F>(T, dl, A, ld, k, Dinv) && l == 0) st->step_invalid = 1;
+    if (!potrf_tile_wave<F>(T, Dinv + (size_t)k * kTile * kTile) && l == 0) st->step_invalid = 1;
 }
 
 // Step k of the factorization in one launch, one workgroup per lower tile (i, j) of the trailing
@@ -209,7 +176,6 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
     constexpr int PP = kTile + 16 / (int)sizeof(F);  // LDS row pitch: rows start 16-byte aligned
     __shared__ __align__(16) F P[2][kTile * PP];     // L_ik, L_jk
     __shared__ F T[kTile][kTile + 1];
-    __shared__ F dl[kTile];
     const int b = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
     int ii = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
     while ((ii + 1) * (ii + 2) / 2 <= b) ++ii;
@@ -219,15 +185,23 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
     const int si = w >> 1, sj = w & 1;
     const bool next_diag = b == 0;
     const F* Xk = Dinv + (size_t)k * kTile * kTile;
+    F* Aij = A + (size_t)(kTile * i) * ld + kTile * j;
+    // the tile's own entries are requested before the panel products (a load after the barrier waits
+    // for memory once more)
+    typename Mfma<F>::acc c = {0, 0, 0, 0};
+    const bool own = !(i == j && si < sj);
+    if (own)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = Aij[(size_t)(16 * si + Mfma<F>::row(l, e)) * ld + 16 * sj + (l & 15)];
     // panel tiles of rows i and j (one of them when i == j)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         if (t == 1 && i == j) break;
         const F* Ark = A + (size_t)(kTile * (t == 0 ? i : j)) * ld + kTile * k;
-        typename Mfma<F>::acc c = {0, 0, 0, 0};
-        c = tile_mma_nt<F>(Ark, ld, Xk, kTile, si, sj, c, (F)1);
+        typename Mfma<F>::acc p = {0, 0, 0, 0};
+        p = tile_mma_nt<F>(Ark, ld, Xk, kTile, si, sj, p, (F)1);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) P[t][(16 * si + Mfma<F>::row(l, e)) * PP + 16 * sj + (l & 15)] = c[e];
+        for (int e = 0; e < 4; ++e) P[t][(16 * si + Mfma<F>::row(l, e)) * PP + 16 * sj + (l & 15)] = p[e];
     }
     __syncthreads();
     if (j == k + 1) {
@@ -237,11 +211,7 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
             Aki[(size_t)cc * ld + rr] = P[0][rr * PP + cc];
         }
     }
-    F* Aij = A + (size_t)(kTile * i) * ld + kTile * j;
-    if (!(i == j && si < sj)) {
-        typename Mfma<F>::acc c;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = Aij[(size_t)(16 * si + Mfma<F>::row(l, e)) * ld + 16 * sj + (l & 15)];
+    if (own) {
         c = tile_mma_nt<F>(P[0], PP, i == j ? P[0] : P[1], PP, si, sj, c, (F)-1);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -254,7 +224,7 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
     }
     if (!next_diag) return;
     __syncthreads();
-    if (w == 0 && !potrf_tile_wave<F>(T, dl, A, ld, k + 1, Dinv) && l == 0) st->step_invalid = 1;
+    if (w == 0 && !potrf_tile_wave<F>(T, Dinv + (size_t)(k + 1) * kTile * kTile) && l == 0) st->step_invalid = 1;
 }
 
 // After the factorization: L_ik = (tile (k, i))' into the lower tile (i, k), i > k (one workgroup per
