@@ -15,9 +15,9 @@
 // products run on the matrix cores (v_mfma_f64_16x16x4f64, v_mfma_f32_16x16x4f32), and the
 // trailing update also factors the next diagonal tile, so a step is two launches.  The panel is
 // also stored transposed in the upper tiles (the factorization reads only the lower ones; in FP64
-// the factor overwrites S).  The triangular solves work on diagonal blocks of four tiles whose
-// inverses are formed after the factorization, one launch per block and sweep, with the rows
-// below (above) the block updated by many workgroups at once.  In mixed precision the factor is
+// the factor overwrites S).  The triangular solves work on diagonal blocks of sixteen tiles whose
+// inverses are formed after the factorization: two launches per block and sweep, each a
+// matrix-vector product over many workgroups.  In mixed precision the factor is
 // FP32 and the step is refined in FP64 against the FP64 S (refine_steps iterations of
 // r = b - S y, y += S_f^-1 r).
 #pragma once
@@ -103,9 +103,9 @@ __global__ void k_convert_S(const double* __restrict__ S, F* __restrict__ A, siz
 
 // ---------------------------------------------------------------------------------------------
 // 32 x 32 tile products on the matrix cores.  A 16 x 16 block of the product X Y' of two 32-column
-// tiles is one wave's eight v_mfma 16x16x4 steps: in step s, lane l supplies X[row0 + l%16][8q + s]
-// and Y[col0 + l%16][8q + s] (q = l/16), so each lane reads 8 consecutive values of one row and the
-// four lanes of a row cover it; every k in [0, 32) enters exactly once.  Accumulator element i of
+// tiles is one wave's eight v_mfma 16x16x4 steps: lane l supplies eight values of row row0 + l%16 of X
+// and of row col0 + l%16 of Y (Mfma::load_row), the four lanes of a row cover it and every k in [0, 32)
+// enters exactly once.  Accumulator element i of
 // lane l is entry (row(l, i), l%16) of the block; the FP64 and FP32 instructions order rows
 // differently.
 
@@ -116,8 +116,8 @@ __device__ __forceinline__ typename Mfma<F>::acc tile_mma_nt(const F* __restrict
                                                              int ldy, int si, int sj, typename Mfma<F>::acc c, F sign) {
     const int l = threadIdx.x & 63, q = l >> 4, r = l & 15;
     F xv[8], yv[8];
-    Mfma<F>::load8(X + (size_t)(16 * si + r) * ldx + 8 * q, xv);
-    Mfma<F>::load8(Y + (size_t)(16 * sj + r) * ldy + 8 * q, yv);
+    Mfma<F>::load_row(X + (size_t)(16 * si + r) * ldx, q, xv);
+    Mfma<F>::load_row(Y + (size_t)(16 * sj + r) * ldy, q, yv);
 #pragma unroll
     for (int s = 0; s < 8; ++s) c = Mfma<F>::mma(sign * xv[s], yv[s], c);
     return c;
@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(64) k_potrf_tile(F* __restrict__ A, int ld, in
     const int l = threadIdx.x;
     const size_t o = (size_t)(kTile * k) * ld + kTile * k;
     for (int idx = l; idx < kTile * kTile; idx += 64) T[idx / kTile][idx % kTile] = A[o + (size_t)(idx / kTile) * ld + idx % kTile];
-    __syncthreads();
+    lds_barrier();
     if (!potrf_tile_wave<F>(T, Dinv + (size_t)k * kTile * kTile) && l == 0) st->step_invalid = 1;
 }
 
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) P[t][(16 * si + Mfma<F>::row(l, e)) * PP + 16 * sj + (l & 15)] = p[e];
     }
-    __syncthreads();
+    lds_barrier();
     if (j == k + 1) {
         F* Aki = A + (size_t)(kTile * k) * ld + kTile * i;
         for (int idx = threadIdx.x; idx < kTile * kTile; idx += 256) {
@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, i
         }
     }
     if (!next_diag) return;
-    __syncthreads();
+    lds_barrier();
     if (w == 0 && !potrf_tile_wave<F>(T, Dinv + (size_t)(k + 1) * kTile * kTile) && l == 0) st->step_invalid = 1;
 }
 
@@ -241,221 +241,237 @@ __global__ void __launch_bounds__(256) k_panel_down(F* __restrict__ A, int ld, c
     const F* Aki = A + (size_t)(kTile * k) * ld + kTile * i;
     F* Aik = A + (size_t)(kTile * i) * ld + kTile * k;
     for (int idx = threadIdx.x; idx < kTile * kTile; idx += 256) T[idx / kTile][idx % kTile] = Aki[(size_t)(idx / kTile) * ld + idx % kTile];
-    __syncthreads();
+    lds_barrier();
     for (int idx = threadIdx.x; idx < kTile * kTile; idx += 256) Aik[(size_t)(idx / kTile) * ld + idx % kTile] = T[idx % kTile][idx / kTile];
 }
 
 // ---------------------------------------------------------------------------------------------
-// Blocked triangular solves over many workgroups.  The factor is cut into diagonal blocks of
-// kSolveBlk tiles (128 rows); after the factorization k_block_inverse forms each block's inverse
-// X = L_KK^-1 from the kept tile inverses (X_ii = Dinv_i, X_ij = -Dinv_i sum_{j<=k<i} L_ik X_kj),
-// so a block of either sweep is one matrix-vector product.  Forward sweep, launch K: workgroup 0
-// applies block K-1's solution to block K's rows and solves block K (y_K = X_K z_K); the other
-// workgroups apply block K-1's solution to one tile row each below block K.  The backward sweep
-// runs the same way upwards with the transposed panel (upper tiles) and x_K = X_K' z_K.  One sweep
-// is one launch per block; every workgroup streams rows of the factor with one wave per row.
-constexpr int kSolveBlk = 4;
+// Triangular solves.  The factor is cut into diagonal blocks of kSolveBlk tiles (512 rows); after the
+// factorization k_block_inverse forms each block's inverse X = L_KK^-1, so a block of either sweep is
+// one matrix-vector product with X (or X') and one with the panel below (above) it, both spread over
+// the chip at one wave per kSweepRows rows.  A system of at most 512 unknowns is solved by two
+// launches; 2250 unknowns by 18 (with 128-row blocks, whose product and panel one workgroup formed one
+// after the other, the sweeps were 36 launches of 10-12 us: 405 us per solve against 80 us).
+constexpr int kSolveBlk = 16;
 constexpr int kSolveRows = kSolveBlk * kTile;
 
 // Tiles of block K: [kSolveBlk K, min(kSolveBlk (K + 1), nt)).
-__device__ __forceinline__ int solve_block_tiles(int K, int nt) { return min(kSolveBlk, nt - kSolveBlk * K); }
+__host__ __device__ __forceinline__ int solve_block_tiles(int K, int nt) {
+    return nt - kSolveBlk * K < kSolveBlk ? nt - kSolveBlk * K : kSolveBlk;
+}
 
-// One workgroup per (block K, column tile j): column j of X = L_KK^-1, i.e. X_jj = Dinv_j and
-// X_ij = -Dinv_i sum_{j<=k<i} L_ik X_kj for i = j+1, ... in order, with the column's tiles, the
-// current factor tile and the partial sum staged in LDS (FP64).  X is stored row-major and, for the
-// backward sweep, transposed (XT), so both sweeps read rows.
+// One workgroup per (block K, 16 columns of X = L_KK^-1): with j their tile, X_jj = Dinv_j and
+// X_ij = -Dinv_i sum_{j<=k<i} L_ik X_kj for i = j+1, ... in order, in FP64 on the matrix cores.  The
+// columns found so far are kept in LDS transposed (rows of X_kj' are the products' second operand);
+// wave (row half si = w % 2, quarter w / 2) forms a 16 x 16 block of the sum over every fourth k, the
+// quarters are added, and the first two waves multiply by Dinv_i.  L_ik is requested while row i - 1 is
+// finished.  What bounds it is one CU's rate of reading L (measured in a copy with clock stamps: with 32
+// columns a workgroup, whose column halves read L twice, issuing the loads took 40% of the time), hence
+// the narrow columns: the five blocks of 2250 rows 97 -> 54 us in FP64, 75 -> 45 us in FP32.  X is stored row-major and transposed (XT), so
+// both sweeps read rows; tiles above the diagonal are neither written nor read.
+constexpr int kInvPitch = kTile + 2;
+constexpr int kInvThreads = 512;
+constexpr int kInvCols = 16;
+inline size_t block_inverse_lds(int nt) {
+    return ((size_t)(std::min(nt, kSolveBlk) + 1) * kInvCols * kInvPitch + 6 * 256) * sizeof(double);
+}
+
+// A lane's eight operands of a 32-column row stored in F, in the columns Mfma<double>::load_row takes.
 template <typename F>
-__global__ void __launch_bounds__(256) k_block_inverse(const F* __restrict__ A, int ld, const F* __restrict__ Dinv,
-                                                        F* __restrict__ Binv, F* __restrict__ BinvT, int nt,
-                                                        const LMState* st) {
+__device__ __forceinline__ void load_row_f64(const F* __restrict__ row, int q, F (&v)[8]) {
+    const R2v<F>* p = reinterpret_cast<const R2v<F>*>(row) + q;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const R2v<F> t = p[4 * i];
+        v[2 * i] = t.x;
+        v[2 * i + 1] = t.y;
+    }
+}
+
+template <typename F>
+__global__ void __launch_bounds__(kInvThreads) k_block_inverse(const F* __restrict__ A, int ld, const F* __restrict__ Dinv,
+                                                               F* __restrict__ Binv, F* __restrict__ BinvT, int nt,
+                                                               const LMState* st) {
     if (st->done || st->step_invalid) return;
-    __shared__ double Xc[kSolveBlk][kTile][kTile + 1];
-    __shared__ double Lt[kTile][kTile + 1];
-    __shared__ double Tt[kTile][kTile + 1];
-    const int K = blockIdx.x / kSolveBlk, j = blockIdx.x % kSolveBlk;
-    const int bt = solve_block_tiles(K, nt), t0 = kSolveBlk * K;
-    const int tid = threadIdx.x;
+    extern __shared__ __align__(16) double inv_lds[];
+    using M = Mfma<double>;
+    constexpr int kHalves = kTile / kInvCols, kQuarters = 4;
+    const int K = blockIdx.x / (kSolveBlk * kHalves), col = blockIdx.x % (kSolveBlk * kHalves);
+    const int j = col / kHalves, bt = solve_block_tiles(K, nt), t0 = kSolveBlk * K;
+    if (j >= bt) return;
+    constexpr int TS = kInvCols * kInvPitch;  // doubles of a tile's 16 columns in LDS
+    double* part = inv_lds;                   // partial sums of quarters 1-3, by lane
+    double* Tt = inv_lds + 6 * 256;           // the sum, transposed
+    double* Xc = Tt + TS;                     // X_ij' for i = j, j + 1, ...
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, q = l >> 4, c16 = l & 15;
+    const int si = w & 1, quarter = w >> 1, cs = kInvCols * col;  // first column within the block
     F* X = Binv + (size_t)K * kSolveRows * kSolveRows;
     F* XT = BinvT + (size_t)K * kSolveRows * kSolveRows;
-    // this workgroup's column: zero above the diagonal tile (and the whole column past the block)
-    for (int e = tid; e < kSolveRows * kTile; e += 256) {
-        const int r = e / kTile, c = kTile * j + e % kTile;
-        if (r < kTile * j || j >= bt || r >= kTile * bt) {
-            X[(size_t)r * kSolveRows + c] = (F)0;
-            XT[(size_t)c * kSolveRows + r] = (F)0;
-        }
+    {
+        const int r = tid / kInvCols, c = tid % kInvCols;
+        const F v = Dinv[(size_t)(t0 + j) * kTile * kTile + r * kTile + cs % kTile + c];
+        X[(size_t)(kTile * j + r) * kSolveRows + cs + c] = v;
+        Xc[c * kInvPitch + r] = (double)v;
     }
-    if (j >= bt) return;
-    auto put = [&](int i, int r, int c, double v) {
-        Xc[i][r][c] = v;
-        X[(size_t)(kTile * i + r) * kSolveRows + kTile * j + c] = (F)v;
-        XT[(size_t)(kTile * j + c) * kSolveRows + kTile * i + r] = (F)v;
+    // this wave's operands of row i: L_ik for its k = j + quarter + 4 m
+    constexpr int kMine = kSolveBlk / kQuarters;
+    F lr[kMine][8];
+    auto request = [&](int i) {
+        const F* Lrow = A + (size_t)(kTile * (t0 + i) + 16 * si + c16) * ld + kTile * t0;
+#pragma unroll
+        for (int m = 0; m < kMine; ++m)
+            if (j + quarter + kQuarters * m < i) load_row_f64<F>(Lrow + kTile * (j + quarter + kQuarters * m), q, lr[m]);
     };
-    for (int e = tid; e < kTile * kTile; e += 256)
-        put(j, e / kTile, e % kTile, (double)Dinv[(size_t)(t0 + j) * kTile * kTile + e]);
-    __syncthreads();
+    if (j + 1 < bt) request(j + 1);
+    lds_barrier();
     for (int i = j + 1; i < bt; ++i) {
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int k = j; k < i; ++k) {
-            const F* Lik = A + (size_t)(kTile * (t0 + i)) * ld + kTile * (t0 + k);
-            for (int e = tid; e < kTile * kTile; e += 256) Lt[e / kTile][e % kTile] = (double)Lik[(size_t)(e / kTile) * ld + e % kTile];
-            __syncthreads();
+        F dv[8];  // the row of Dinv_i the last product needs
+        if (quarter == 0) load_row_f64<F>(Dinv + (size_t)(t0 + i) * kTile * kTile + (16 * si + c16) * kTile, q, dv);
+        typename M::acc c = {0, 0, 0, 0};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int e = tid + 256 * q, r = e / kTile, c = e % kTile;
-                double sum = 0.0;
-#pragma unroll 8
-                for (int m = 0; m < kTile; ++m) sum += Lt[r][m] * Xc[k][m][c];
-                acc[q] += sum;
+        for (int m = 0; m < kMine; ++m) {
+            const int k = j + quarter + kQuarters * m;
+            if (k < i) {
+                double xv[8];
+                M::load_row(Xc + (size_t)(k - j) * TS + c16 * kInvPitch, q, xv);
+#pragma unroll
+                for (int s = 0; s < 8; ++s) c = M::mma((double)lr[m][s], xv[s], c);
             }
-            __syncthreads();
         }
+        if (i + 1 < bt) request(i + 1);
+        if (quarter > 0)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int e = tid + 256 * q;
-            Tt[e / kTile][e % kTile] = acc[q];
-        }
-        const F* Di = Dinv + (size_t)(t0 + i) * kTile * kTile;
-        for (int e = tid; e < kTile * kTile; e += 256) Lt[e / kTile][e % kTile] = (double)Di[e];
-        __syncthreads();
+            for (int e = 0; e < 4; ++e) part[((quarter - 1) * 2 + si) * 256 + e * 64 + l] = c[e];
+        lds_barrier();
+        if (quarter == 0)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int e = tid + 256 * q, r = e / kTile, c = e % kTile;
-            double sum = 0.0;
-#pragma unroll 8
-            for (int m = 0; m < kTile; ++m) sum += Lt[r][m] * Tt[m][c];
-            put(i, r, c, -sum);
+            for (int e = 0; e < 4; ++e) {
+                double t = c[e];
+#pragma unroll
+                for (int h = 0; h < 3; ++h) t += part[(h * 2 + si) * 256 + e * 64 + l];
+                Tt[c16 * kInvPitch + 16 * si + M::row(l, e)] = t;
+            }
+        lds_barrier();
+        if (quarter == 0) {
+            double tv[8];
+            M::load_row(Tt + c16 * kInvPitch, q, tv);
+            typename M::acc x = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) x = M::mma(-(double)dv[s], tv[s], x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 16 * si + M::row(l, e);
+                X[(size_t)(kTile * i + r) * kSolveRows + cs + c16] = (F)x[e];
+                Xc[(size_t)(i - j) * TS + c16 * kInvPitch + r] = x[e];
+            }
         }
-        __syncthreads();
+        lds_barrier();
+    }
+    const int rows = kTile * (bt - j);
+    for (int e = tid; e < kInvCols * rows; e += kInvThreads) {
+        const int cc = e / rows, r = e % rows;
+        XT[(size_t)(cs + cc) * kSolveRows + kTile * j + r] = (F)Xc[(size_t)(r / kTile) * TS + cc * kInvPitch + r % kTile];
     }
 }
 
-// Row dot products out(rr, dot(M[r0 + rr][c0 .. c0 + ncols), v)) for rr < nrows of a row-major M
-// (leading dimension ldm), ncols <= 128, v in double.  One wave per row: lane l takes columns l and
-// l + 64, the wave sums; a wave takes kRowBatch rows at a time with all their loads in flight
-// before the first sum, so the rows do not wait on each other's loads.
-constexpr int kRowBatch = 16;
+// Dot products of kSweepRows consecutive rows with v, by one wave: s[g] = sum_{c in [c0, c1)}
+// M[row0 + g][c] v[c] (every lane gets the sums).  Lane l takes columns c0 + l, + 64, ...; the loads of
+// 256 columns of all rows are in flight together, with clamped columns (v = 0 there) and rows
+// instead of branches around the loads.
+constexpr int kSweepRows = 4;
 
-template <typename F, typename Out>
-__device__ __forceinline__ void rows_dot(const F* __restrict__ M, size_t ldm, int r0, int nrows, int c0, int ncols,
-                                         const double* __restrict__ v, Out out) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const double v0 = lane < ncols ? v[lane] : 0.0, v1 = lane + 64 < ncols ? v[lane + 64] : 0.0;
-    // column and row indices are clamped into the block instead of branching around the loads (a
-    // branch per load makes every load wait for its own result); clamped columns carry v = 0 and
-    // clamped rows are not written
-    const int ca = min(lane, ncols - 1), cb = min(lane + 64, ncols - 1);
-    const int nw = blockDim.x >> 6;
-    for (int rb = wave * kRowBatch; rb < nrows; rb += nw * kRowBatch) {
-        F x0[kRowBatch], x1[kRowBatch];
+template <typename F>
+__device__ __forceinline__ void sweep_dot(const F* __restrict__ M, size_t ldm, int row0, int last_row, int c0, int c1,
+                                          const double* __restrict__ v, int v_end, double (&s)[kSweepRows]) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int g = 0; g < kRowBatch; ++g) {
-            const F* row = M + (size_t)(r0 + min(rb + g, nrows - 1)) * ldm + c0;
-            x0[g] = row[ca];
-            x1[g] = row[cb];
-        }
-        double s[kRowBatch];
+    for (int g = 0; g < kSweepRows; ++g) s[g] = 0.0;
+    for (int cb = c0; cb < c1; cb += 256) {
+        F m[kSweepRows][4];
+        double x[4];
 #pragma unroll
-        for (int g = 0; g < kRowBatch; ++g) {
-            double a = (double)x0[g] * v0;
-            a += (double)x1[g] * v1;
-            s[g] = a;
+        for (int u = 0; u < 4; ++u) {
+            const int c = cb + lane + 64 * u, cc = min(c, c1 - 1);
+            const double t = v[min(cc, v_end - 1)];
+            x[u] = c < c1 && c < v_end ? t : 0.0;
+#pragma unroll
+            for (int g = 0; g < kSweepRows; ++g) m[g][u] = M[(size_t)min(row0 + g, last_row) * ldm + cc];
         }
 #pragma unroll
-        for (int g = 0; g < kRowBatch; ++g) s[g] = wave_sum(s[g]);
-        if (lane == 0)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int g = 0; g < kRowBatch; ++g)
-                if (rb + g < nrows) out(rb + g, s[g]);
+            for (int g = 0; g < kSweepRows; ++g) s[g] = fma((double)m[g][u], x[u], s[g]);
     }
+#pragma unroll
+    for (int g = 0; g < kSweepRows; ++g) s[g] = wave_sum(s[g]);
 }
 
-// z[r0 + rr] -= M[r0 + rr][c0 ..] v for rr < nrows.
+// Forward sweep, block K: y_K = X_K rhs_K (rhs: b for block 0, which has n entries; z afterwards).
 template <typename F>
-__device__ __forceinline__ void rows_minus_mv(const F* __restrict__ M, size_t ldm, int r0, int nrows, int c0,
-                                              int ncols, const double* __restrict__ v, double* __restrict__ z) {
-    rows_dot<F>(M, ldm, r0, nrows, c0, ncols, v, [&](int rr, double s) { z[r0 + rr] -= s; });
-}
-
-// Forward sweep, launch K (see above).  z has ld entries; launch 0 copies b into z first.  The
-// diagonal workgroup keeps block K's right-hand side in LDS between its two products.
-constexpr int kSolveThreads = 512;
-
-template <typename F>
-__global__ void __launch_bounds__(kSolveThreads) k_trsv_fwd(const F* __restrict__ A, int ld, const F* __restrict__ Binv,
-                                                            int nt, int K, const double* __restrict__ b, int n,
-                                                            double* __restrict__ z, const LMState* st) {
+__global__ void __launch_bounds__(kWG) k_fwd_solve(const F* __restrict__ Binv, int nt, int K, const double* __restrict__ rhs,
+                                                   int n, double* __restrict__ y, const LMState* st) {
     if (st->done || st->step_invalid) return;
-    __shared__ double v[kSolveRows];
-    __shared__ double zk[kSolveRows];
-    const int t = threadIdx.x, g = blockIdx.x;
-    const int kb = kSolveRows * K;                       // first row of block K
-    const int rows_k = kTile * solve_block_tiles(K, nt);  // rows of block K
-    const int pb = kb - kSolveRows;                      // block K-1 (always full when K > 0)
-    if (g > 0) {
-        // one tile row below block K
-        const int r0 = kb + rows_k + kTile * (g - 1);
-        if (K == 0) {
-            for (int r = t; r < kTile; r += blockDim.x) z[r0 + r] = r0 + r < n ? b[r0 + r] : 0.0;
-            return;
-        }
-        for (int c = t; c < kSolveRows; c += blockDim.x) v[c] = z[pb + c];
-        __syncthreads();
-        rows_minus_mv<F>(A, (size_t)ld, r0, kTile, pb, kSolveRows, v, z);
-        return;
-    }
-    for (int r = t; r < rows_k; r += blockDim.x) zk[r] = K == 0 ? (r < n ? b[r] : 0.0) : z[kb + r];
-    if (K > 0)
-        for (int c = t; c < kSolveRows; c += blockDim.x) v[c] = z[pb + c];
-    __syncthreads();
-    if (K > 0) {
-        rows_dot<F>(A, (size_t)ld, kb, rows_k, pb, kSolveRows, v, [&](int rr, double s) { zk[rr] -= s; });
-        __syncthreads();
-    }
-    // y_K = X_K z_K
-    const F* X = Binv + (size_t)K * kSolveRows * kSolveRows;
-    rows_dot<F>(X, (size_t)kSolveRows, 0, rows_k, 0, rows_k, zk, [&](int r, double s) { z[kb + r] = s; });
+    const int rows = kTile * solve_block_tiles(K, nt), kb = kSolveRows * K;
+    const int r0 = kSweepRows * (blockIdx.x * kWaves + (threadIdx.x >> 6));
+    if (r0 >= rows) return;
+    double s[kSweepRows];
+    sweep_dot<F>(Binv + (size_t)K * kSolveRows * kSolveRows, kSolveRows, r0, rows - 1, 0, kTile * (r0 / kTile + 1), rhs + kb,
+                 n - kb, s);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int g = 0; g < kSweepRows; ++g) y[kb + r0 + g] = s[g];
 }
 
-// Backward sweep, launch K (blocks from the last down to 0): x_K = X_K' (z_K - U_{K,K+1} x_{K+1});
-// rows above block K get block K+1's solution applied.  Block K's result also goes to x (added to
-// it when accumulate != 0), rows below n excluded.
+// Rows below block K: z = rhs - L_{.K} y_K (rhs: b for block 0, z itself afterwards).
 template <typename F>
-__global__ void __launch_bounds__(kSolveThreads) k_trsv_bwd(const F* __restrict__ A, int ld, const F* __restrict__ BinvT,
-                                                            int nt, int K, double* __restrict__ z, double* __restrict__ x,
-                                                            int n, int accumulate, const LMState* st) {
+__global__ void __launch_bounds__(kWG) k_fwd_rows(const F* __restrict__ A, int ld, int K, const double* rhs, int n,
+                                                  const double* __restrict__ y, double* z, const LMState* st) {
     if (st->done || st->step_invalid) return;
-    __shared__ double v[kSolveRows];
-    __shared__ double zk[kSolveRows];
-    const int t = threadIdx.x, g = blockIdx.x;
-    const int nb = (nt + kSolveBlk - 1) / kSolveBlk;
-    const int kb = kSolveRows * K, rows_k = kTile * solve_block_tiles(K, nt);
-    const bool has_next = K + 1 < nb;
-    const int nbk = has_next ? kSolveRows * (K + 1) : 0;                      // first row of block K+1
-    const int cols_next = has_next ? kTile * solve_block_tiles(K + 1, nt) : 0;  // its rows
-    if (g > 0) {
-        if (!has_next) return;
-        const int r0 = kTile * (g - 1);  // a tile row above block K
-        for (int c = t; c < cols_next; c += blockDim.x) v[c] = z[nbk + c];
-        __syncthreads();
-        rows_minus_mv<F>(A, (size_t)ld, r0, kTile, nbk, cols_next, v, z);
-        return;
-    }
-    for (int r = t; r < rows_k; r += blockDim.x) zk[r] = z[kb + r];
-    if (has_next)
-        for (int c = t; c < cols_next; c += blockDim.x) v[c] = z[nbk + c];
-    __syncthreads();
-    if (has_next) {
-        rows_dot<F>(A, (size_t)ld, kb, rows_k, nbk, cols_next, v, [&](int rr, double s) { zk[rr] -= s; });
-        __syncthreads();
-    }
-    // x_K = X_K' z_K (rows of the transposed inverse)
-    const F* XT = BinvT + (size_t)K * kSolveRows * kSolveRows;
-    rows_dot<F>(XT, (size_t)kSolveRows, 0, rows_k, 0, rows_k, zk, [&](int r, double s) {
-        z[kb + r] = s;
-        const int row = kb + r;
-        if (row < n) x[row] = accumulate ? x[row] + s : s;
-    });
+    const int kb = kSolveRows * K;
+    const int r0 = kb + kSolveRows + kSweepRows * (blockIdx.x * kWaves + (threadIdx.x >> 6));
+    if (r0 >= ld) return;
+    double s[kSweepRows];
+    sweep_dot<F>(A + kb, ld, r0, ld - 1, 0, kSolveRows, y + kb, kSolveRows, s);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int g = 0; g < kSweepRows; ++g) z[r0 + g] = (r0 + g < n ? rhs[r0 + g] : 0.0) - s[g];
+}
+
+// Backward sweep, block K: t_K = X_K' y_K, also into x (added to it when accumulate != 0; rows below
+// n only).
+template <typename F>
+__global__ void __launch_bounds__(kWG) k_bwd_solve(const F* __restrict__ BinvT, int nt, int K, const double* __restrict__ y,
+                                                   double* __restrict__ t, double* __restrict__ x, int n, int accumulate,
+                                                   const LMState* st) {
+    if (st->done || st->step_invalid) return;
+    const int rows = kTile * solve_block_tiles(K, nt), kb = kSolveRows * K;
+    const int r0 = kSweepRows * (blockIdx.x * kWaves + (threadIdx.x >> 6));
+    if (r0 >= rows) return;
+    double s[kSweepRows];
+    sweep_dot<F>(BinvT + (size_t)K * kSolveRows * kSolveRows, kSolveRows, r0, rows - 1, kTile * (r0 / kTile), rows, y + kb, rows,
+                 s);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int g = 0; g < kSweepRows; ++g) {
+            const int row = kb + r0 + g;
+            t[row] = s[g];
+            if (row < n) x[row] = accumulate ? x[row] + s[g] : s[g];
+        }
+}
+
+// Rows above block K: y -= L_{K.}' t_K, from the transposed panels in the upper tiles.
+template <typename F>
+__global__ void __launch_bounds__(kWG) k_bwd_rows(const F* __restrict__ A, int ld, int nt, int K, const double* __restrict__ t,
+                                                  double* __restrict__ y, const LMState* st) {
+    if (st->done || st->step_invalid) return;
+    const int rows = kTile * solve_block_tiles(K, nt), kb = kSolveRows * K;
+    const int r0 = kSweepRows * (blockIdx.x * kWaves + (threadIdx.x >> 6));
+    if (r0 >= kb) return;
+    double s[kSweepRows];
+    sweep_dot<F>(A + kb, ld, r0, kb - 1, 0, rows, t + kb, rows, s);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int g = 0; g < kSweepRows; ++g) y[r0 + g] -= s[g];
 }
 
 // r = b - S y (FP64, S symmetric with its full n x n block stored); one wave per row.
@@ -488,11 +504,11 @@ struct DenseSchur {
     DevBuf<Real> js;
     DevBuf<int> blk_a, blk_b, blk_off;
     DevBuf<int2> pairs;
-    DevBuf<double> S, r, z;
+    DevBuf<double> S, r, z, y;
     DevBuf<float> Af, Dinvf, Binvf, BinvTf;
     DevBuf<double> Dinvd, Binvd, BinvTd;
     int64_t device_bytes() const {
-        return js.bytes() + blk_a.bytes() * 3 + pairs.bytes() + S.bytes() + r.bytes() + z.bytes() + Af.bytes() +
+        return js.bytes() + blk_a.bytes() * 3 + pairs.bytes() + S.bytes() + r.bytes() + z.bytes() + y.bytes() + Af.bytes() +
                Dinvf.bytes() + Binvf.bytes() + BinvTf.bytes() + Dinvd.bytes() + Binvd.bytes() + BinvTd.bytes();
     }
 
@@ -519,33 +535,44 @@ struct DenseSchur {
         BA_TRY(S.alloc((size_t)ld * ld));
         BA_TRY(r.alloc(ld));
         BA_TRY(z.alloc(ld));
+        BA_TRY(y.alloc(ld));
         const size_t binv = (size_t)nb * kSolveRows * kSolveRows;
         if (f64) {
             BA_TRY(Dinvd.alloc((size_t)nt * kTile * kTile));
             BA_TRY(Binvd.alloc(binv));
             BA_TRY(BinvTd.alloc(binv));
+            BA_TRY(allow_dynamic_lds((const void*)k_block_inverse<double>, (int)block_inverse_lds(nt)));
         } else {
             BA_TRY(Af.alloc((size_t)ld * ld));
             BA_TRY(Dinvf.alloc((size_t)nt * kTile * kTile));
             BA_TRY(Binvf.alloc(binv));
             BA_TRY(BinvTf.alloc(binv));
+            BA_TRY(allow_dynamic_lds((const void*)k_block_inverse<float>, (int)block_inverse_lds(nt)));
         }
         BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }
 
-    // x = (L L')^-1 b (accumulate: x += ...) by the blocked sweeps: nb launches each way.
+    // x = (L L')^-1 b (accumulate: x += ...) by the blocked sweeps.
     template <typename F, typename SolverT>
     void solve(SolverT& sv, const F* A, const F* Binv, const F* BinvT, const double* b, double* x, int accumulate) {
-        auto& d = sv.d;
+        const LMState* st = sv.d.st;
+        const int per = kSweepRows * kWaves;  // rows of a workgroup
         for (int K = 0; K < nb; ++K) {
-            const int below = std::max(0, nt - kSolveBlk * (K + 1));
-            sv.launch("trsv_fwd", k_trsv_fwd<F>, 1 + below, kSolveThreads, A, ld, Binv, nt, K, b, n, z.p,
-                      (const LMState*)d.st);
+            const double* rhs = K == 0 ? b : z.p;
+            const int lim = K == 0 ? n : ld;
+            sv.launch("fwd_solve", k_fwd_solve<F>, div_up(kTile * solve_block_tiles(K, nt), per), kWG, Binv, nt, K, rhs, lim,
+                      y.p, st);
+            const int below = ld - kSolveRows * (K + 1);
+            if (below > 0)
+                sv.launch("fwd_rows", k_fwd_rows<F>, div_up(below, per), kWG, A, ld, K, rhs, lim, (const double*)y.p, z.p, st);
         }
-        for (int K = nb - 1; K >= 0; --K)
-            sv.launch("trsv_bwd", k_trsv_bwd<F>, 1 + kSolveBlk * K, kSolveThreads, A, ld, BinvT, nt, K, z.p, x, n,
-                      accumulate, (const LMState*)d.st);
+        for (int K = nb - 1; K >= 0; --K) {
+            sv.launch("bwd_solve", k_bwd_solve<F>, div_up(kTile * solve_block_tiles(K, nt), per), kWG, BinvT, nt, K,
+                      (const double*)y.p, z.p, x, n, accumulate, st);
+            if (K > 0)
+                sv.launch("bwd_rows", k_bwd_rows<F>, div_up(kSolveRows * K, per), kWG, A, ld, nt, K, (const double*)z.p, y.p, st);
+        }
     }
 
     template <typename F, typename SolverT>
@@ -557,8 +584,8 @@ struct DenseSchur {
             sv.launch("step", k_step_tiles<F>, m * (m + 1) / 2, 256, A, ld, k, Dinv, d.st);
         }
         if (nt > 1) sv.launch("panel_down", k_panel_down<F>, nt * (nt - 1) / 2, 256, A, ld, (const LMState*)d.st);
-        sv.launch("block_inverse", k_block_inverse<F>, nb * kSolveBlk, 256, (const F*)A, ld, (const F*)Dinv, Binv, BinvT,
-                  nt, (const LMState*)d.st);
+        sv.launch_shm("block_inverse", k_block_inverse<F>, nb * kSolveRows / kInvCols, kInvThreads, block_inverse_lds(nt), (const F*)A, ld,
+                      (const F*)Dinv, Binv, BinvT, nt, (const LMState*)d.st);
         solve<F>(sv, A, Binv, BinvT, (const double*)d.bc, d.px, 0);
         for (int it = 0; it < refine; ++it) {
             sv.launch("residual", k_residual, div_up(n, kWaves), kWG, (const double*)S.p, ld, (const double*)d.bc,

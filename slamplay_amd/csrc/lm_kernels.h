@@ -192,6 +192,15 @@ __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Workgroup barrier for threads that exchange data through LDS only.  __syncthreads also waits for
+// every global load and store the wave has in flight, so a load requested ahead of it is waited for
+// there; here those stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Wave reductions on the VALU: four butterfly steps inside each row of 16 lanes by DPP lane
 // permutations (partners lane ^ 1, lane ^ 2, the mirrored lane of the half-row and of the row), so
 // every lane of a row holds the row's total, then the four row totals read with v_readlane and added

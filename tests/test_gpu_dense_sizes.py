@@ -1,0 +1,26 @@
+"""The dense reduced system at the sizes where its kernels change path: one tile of 32 unknowns, exact
+tile multiples, one tile past a 512-row block of the triangular solves and of its second block."""
+import numpy as np
+import pytest
+
+import slamplay_amd as S
+from slamplay_amd import _capi as C
+
+pytestmark = pytest.mark.gpu
+
+FIXED = dict(max_num_iterations=3, function_tolerance=0.0, gradient_tolerance=0.0, parameter_tolerance=0.0)
+
+
+# 9 nc unknowns: 27 (1 tile), 36, 63 (2 tiles), 180, 189, 198 (6 and 7 tiles), 288 (9 exact), 297,
+# 513 (17 tiles: block 2 of one tile), 1026 (33 tiles: block 3 of one tile)
+@pytest.mark.parametrize("nc", [3, 4, 7, 20, 21, 22, 32, 33, 57, 114])
+def test_dense_sizes_match_oracle(oracle_mod, nc):
+    p = S.synthetic(2, seed=nc, num_cameras=nc, num_points=40 * nc, max_track=min(8, nc))
+    ref = oracle_mod.solve(p.num_cameras(), p.num_points(), p.camera_index(), p.point_index(), p.observations(),
+                           p.cameras(), p.points(), oracle_mod.default_options(**FIXED))
+    out = S.SolveBA(p, linear_solver=C.SOLVER_DENSE_SCHUR, **FIXED)
+    assert out["num_successful_steps"] == sum(t["step_is_successful"] for t in ref["trace"][1:])
+    # both sides solve the same damped FP64 systems: condition number (at most 1e7 in three steps from
+    # radius 1e4) times unit roundoff, per step
+    assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-8 * ref["final_cost"]
+    np.testing.assert_allclose(p.cameras(), ref["cams"], rtol=0, atol=1e-7 * np.abs(ref["cams"]).max())
