@@ -2,11 +2,11 @@
 // SPARSE_SCHUR step of test_bundle_adjustment_ceres.cpp:97 for problems up to a few hundred cameras).
 //
 //   S = U* - sum_points sum_{i,j in track} W~_i Vinv_p W~_j'     (9 nc x 9 nc, FP64)
-// with U*'s per-observation part folded into the (i, i) pairs: S_aa = D_a^2 + sum J~'(I - G)J~ - ...
-// is assembled without atomics: the host enumerates every ordered observation pair (i, j) of a
-// point with camera(i) <= camera(j) once per problem and groups the pairs by camera block (a, b);
-// one wave owns one 9x9 block and reduces its pair list in a fixed order (pair_block.h, the kernel
-// the batched windows use too).  A pair contributes Jc~_i' (Hp_i Jp~_j') Jc~_j with
+// is assembled without atomics.  The diagonal block of a camera that sees no point twice is the
+// Schur-Jacobi block k_rhs_cam forms anyway, D_a^2 + sum J~'(I - G)J~.  For the others the host enumerates
+// every ordered observation pair (i, j) of a point with camera(i) <= camera(j) once per problem and
+// groups the pairs by camera block (a, b); one workgroup owns one 9x9 block and reduces its pair list
+// in a fixed order (pair_block.h, the products the batched windows use too).  A pair contributes Jc~_i' (Hp_i Jp~_j') Jc~_j with
 // Hp_i = Jp~_i Vinv_p, i.e. a 2x2 middle factor.
 //
 // The factorization is a tiled right-looking Cholesky (32 x 32 tiles): per step, the diagonal
@@ -69,29 +69,41 @@ __global__ void __launch_bounds__(kWG) k_dense_store(Dev<Real> d, Real* __restri
     }
 }
 
-// S <- 0 with an identity tail on the padding diagonal.
-__global__ void k_fill_S(double* __restrict__ S, int n, int ld, const LMState* st) {
+// S <- the cameras' Schur-Jacobi blocks M_c (k_rhs_cam: D_c^2 plus every observation with itself) on the
+// diagonal, zero elsewhere, an identity tail on the padding diagonal.
+__global__ void k_fill_S(double* __restrict__ S, int n, int ld, const double* __restrict__ M, const LMState* st) {
     if (st->done || st->step_invalid) return;
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)ld * ld) return;
     const int r = (int)(i / ld), c = (int)(i % ld);
-    S[i] = (r == c && r >= n) ? 1.0 : 0.0;
+    double v = (r == c && r >= n) ? 1.0 : 0.0;
+    if (r < n && c < n && r / 9 == c / 9) v = M[81 * (size_t)(r / 9) + 9 * (r % 9) + c % 9];
+    S[i] = v;
 }
 
-// One 9x9 block of the reduced camera system per workgroup of one wave (the blocks' pair lists, the
-// 36-value records of k_dense_store): pair_block in pair_block.h.
-template <typename Real>
-__global__ void __launch_bounds__(64) k_schur_blocks(Dev<Real> d, const Real* __restrict__ js,
-                                                     const int* __restrict__ blk_a, const int* __restrict__ blk_b,
-                                                     const int* __restrict__ blk_off, const int2* __restrict__ pairs,
-                                                     double* __restrict__ S, int ld, int nblocks) {
+// One 9x9 block of the reduced camera system per workgroup of NW waves (the blocks' pair lists, the
+// 36-value records of k_dense_store): pair_block in pair_block.h.  Bound by the products' instructions
+// and LDS reads (about 200 per 16 pairs) once the blocks of neighbouring cameras run on one XCD: 325 ->
+// 198 us at 250 cameras and 4.2M pairs (blocks in key order over all XCDs, the cameras' own blocks
+// among them), 78 -> 40 us at 49 cameras, 62 -> 9 us for a stereo window of 8.
+template <typename Real, int NW>
+constexpr size_t schur_blocks_lds() {
+    return (size_t)NW * pair_stage_bytes<Real, kRecDense>() + (NW > 1 ? NW * 81 * sizeof(double) : 0);
+}
+
+template <typename Real, int NW>
+__global__ void __launch_bounds__(64 * NW) k_schur_blocks(Dev<Real> d, const Real* __restrict__ js,
+                                                          const int4* __restrict__ blk, const int2* __restrict__ pairs,
+                                                          double* __restrict__ S, int ld) {
     LMState* st = d.st;
     if (st->done || st->step_invalid) return;
-    __shared__ __align__(16) unsigned char stage[pair_stage_bytes<Real, kRecDense>()];
-    const int b = blockIdx.x;
-    if (b >= nblocks) return;
-    const int4 bk = make_int4(blk_a[b], blk_b[b], blk_off[b], blk_off[b + 1]);
-    pair_block<Real, kRecDense>(bk, pairs, js, d.dc2, S, ld, reinterpret_cast<Real*>(stage));
+    extern __shared__ __align__(16) unsigned char schur_lds_mem[];
+    const int4 bk = blk[blockIdx.x];
+    if (bk.x < 0) return;  // padding of an XCD's list
+    constexpr int kStage = pair_stage_bytes<Real, kRecDense>();
+    pair_block<Real, kRecDense, NW>(bk, pairs, js, d.dc2, S, ld,
+                                    reinterpret_cast<Real*>(schur_lds_mem + (size_t)(threadIdx.x >> 6) * kStage),
+                                    reinterpret_cast<double*>(schur_lds_mem + (size_t)NW * kStage));
 }
 
 template <typename F>
@@ -502,14 +514,56 @@ struct DenseSchur {
     int n = 0, ld = 0, nt = 0, nb = 0, nblocks = 0, refine = 0;
     bool f64 = true;  // factor in FP64 (FP64 solver, or a small system)
     DevBuf<Real> js;
-    DevBuf<int> blk_a, blk_b, blk_off;
+    DevBuf<int4> blk;
+    int schur_waves = 4;  // waves per block of the pair products
     DevBuf<int2> pairs;
     DevBuf<double> S, r, z, y;
     DevBuf<float> Af, Dinvf, Binvf, BinvTf;
     DevBuf<double> Dinvd, Binvd, BinvTd;
     int64_t device_bytes() const {
-        return js.bytes() + blk_a.bytes() * 3 + pairs.bytes() + S.bytes() + r.bytes() + z.bytes() + y.bytes() + Af.bytes() +
+        return js.bytes() + blk.bytes() + pairs.bytes() + S.bytes() + r.bytes() + z.bytes() + y.bytes() + Af.bytes() +
                Dinvf.bytes() + Binvf.bytes() + BinvTf.bytes() + Dinvd.bytes() + Binvd.bytes() + BinvTd.bytes();
+    }
+
+    // The blocks the pair kernel forms: those of two different cameras, and a camera's own block when it
+    // observes a point more than once (pairs x != y, which M_c does not hold; the pair kernel then
+    // writes the whole block).  In launch order: workgroup k runs on XCD k % 8; each XCD takes a
+    // contiguous eighth (by pairs) of the blocks sorted by groups of four cameras on either side, so
+    // that the records of eight cameras, read once per pair, are re-read from its own L2.
+    // Padding entries have camera -1.
+    std::vector<int4> block_list(const PairBlocks& pb, int nc) {
+        std::vector<int> take;
+        int64_t total = 0;
+        for (int i = 0; i < (int)pb.a.size(); ++i) {
+            bool t = pb.a[i] != pb.b[i];
+            for (int q = pb.off[i]; !t && q < pb.off[i + 1]; ++q) t = pb.i[q] != pb.j[q];
+            if (!t) continue;
+            take.push_back(i);
+            total += pb.off[i + 1] - pb.off[i];
+        }
+        constexpr int G = 4;
+        auto group = [&](int i) { return (int64_t)(pb.a[i] / G) * (nc / G + 1) + pb.b[i] / G; };
+        std::stable_sort(take.begin(), take.end(), [&](int x, int y) { return group(x) < group(y); });
+        std::vector<std::vector<int4>> xq(kXcds);
+        int64_t seen = 0;
+        for (int i : take) {
+            const int64_t n_i = pb.off[i + 1] - pb.off[i];
+            const int x = (int)std::min<int64_t>(kXcds - 1, (seen + n_i / 2) * kXcds / std::max<int64_t>(total, 1));
+            xq[x].push_back(make_int4(pb.a[i], pb.b[i], pb.off[i], pb.off[i + 1]));
+            seen += n_i;
+        }
+        size_t longest = 0;
+        for (const auto& q : xq) longest = std::max(longest, q.size());
+        std::vector<int4> out(longest * kXcds, make_int4(-1, -1, 0, 0));
+        for (int x = 0; x < kXcds; ++x)
+            for (size_t k = 0; k < xq[x].size(); ++k) out[k * kXcds + x] = xq[x][k];
+        // A workgroup of eight waves fills a CU's LDS with its staging areas, so it is taken only while
+        // every block still has a CU of its own (28 blocks of 380 pairs: 6.9 us against 7.8 with four
+        // waves and 15.9 with one; 1,130 blocks: 52 against 40).  Four waves otherwise: three such
+        // workgroups share a CU (1,130 blocks 70.8 -> 40 us and 8,856 blocks 205 -> 198 against one wave
+        // each; 193 with two).
+        schur_waves = (int)take.size() <= kCUs ? 8 : 4;
+        return out;
     }
 
     int create(const ba_problem_view* v, const Layout& L, const ba_options& o, hipStream_t s) {
@@ -523,11 +577,10 @@ struct DenseSchur {
         refine = f64 ? 0 : std::max(0, o.refine_steps);
         PairBlocks pb;
         build_pair_blocks(L, &pb);
-        const std::vector<int>&ba = pb.a, &bb = pb.b, &boff = pb.off, &pi = pb.i, &pj = pb.j;
-        nblocks = (int)ba.size();
-        BA_TRY(blk_a.upload(ba.data(), ba.size(), s));
-        BA_TRY(blk_b.upload(bb.data(), bb.size(), s));
-        BA_TRY(blk_off.upload(boff.data(), boff.size(), s));
+        const std::vector<int>&pi = pb.i, &pj = pb.j;
+        std::vector<int4> list = block_list(pb, nc);
+        nblocks = (int)list.size();
+        BA_TRY(blk.upload(list.data(), list.size(), s));
         std::vector<int2> pr(pi.size());
         for (size_t q = 0; q < pi.size(); ++q) pr[q] = make_int2(pi[q], pj[q]);
         BA_TRY(pairs.upload(pr.data(), pr.size(), s));
@@ -549,6 +602,7 @@ struct DenseSchur {
             BA_TRY(BinvTf.alloc(binv));
             BA_TRY(allow_dynamic_lds((const void*)k_block_inverse<float>, (int)block_inverse_lds(nt)));
         }
+        BA_TRY(allow_dynamic_lds((const void*)k_schur_blocks<Real, 8>, (int)schur_blocks_lds<Real, 8>()));
         BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }
@@ -594,6 +648,12 @@ struct DenseSchur {
         }
     }
 
+    template <int NW, typename SolverT>
+    void enqueue_schur(SolverT& sv) {
+        sv.launch_shm("schur_pairs", k_schur_blocks<Real, NW>, nblocks, 64 * NW, schur_blocks_lds<Real, NW>(), sv.d,
+                      (const Real*)js.p, (const int4*)blk.p, (const int2*)pairs.p, S.p, ld);
+    }
+
     template <typename SolverT>
     void enqueue_solve(SolverT& sv) {
         auto& d = sv.d;
@@ -603,10 +663,12 @@ struct DenseSchur {
                              k_dense_store<Real, kModelStereo>),
                   xcd_grid(nc), kWG, d, js.p);
         const size_t nn = (size_t)ld * ld;
-        sv.launch("fill_S", k_fill_S, (int)((nn + 255) / 256), 256, S.p, n, ld, (const LMState*)d.st);
-        if (nblocks)
-            sv.launch("schur_pairs", k_schur_blocks<Real>, nblocks, 64, d, (const Real*)js.p, (const int*)blk_a.p,
-                      (const int*)blk_b.p, (const int*)blk_off.p, (const int2*)pairs.p, S.p, ld, nblocks);
+        sv.launch("fill_S", k_fill_S, (int)((nn + 255) / 256), 256, S.p, n, ld, (const double*)d.M,
+                  (const LMState*)d.st);
+        if (schur_waves == 8)
+            enqueue_schur<8>(sv);
+        else
+            enqueue_schur<4>(sv);
         if (f64) {
             factor_and_solve<double>(sv, S.p, Dinvd.p, Binvd.p, BinvTd.p);
         } else {

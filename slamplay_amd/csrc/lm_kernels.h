@@ -36,6 +36,7 @@ namespace mba {
 constexpr int kWG = 256;    // threads per workgroup for every solver kernel
 constexpr int kWaves = kWG / 64;
 constexpr int kXcds = 8;    // MI355X: 8 XCDs, workgroups dispatched round-robin over them
+constexpr int kCUs = 256;   // MI355X: compute units
 
 // Block b runs on XCD b % 8; give XCD k the contiguous index range [k per, (k + 1) per) so that
 // neighbouring cameras (which share points) and neighbouring point chunks share one L2.

@@ -14,7 +14,8 @@
 // pairs, lane q of the row pair q, accumulating in registers (FP64); the 16 partial sums of an entry
 // are combined by a DPP butterfly inside the row.  The block's entries are written to S (row-major,
 // leading dimension ld, both triangles).  Every entry's sum runs in a fixed order (pair q, q + 16,
-// ... per lane, then the butterfly), whatever wave or launch takes the block.
+// ... per lane, then the butterfly), whatever wave or launch takes the block.  The dense solver, whose
+// blocks are few and long, gives a block to a workgroup of several waves instead (NW below).
 #pragma once
 
 #include "lm_kernels.h"
@@ -83,12 +84,28 @@ __device__ __forceinline__ void pair_store_round(Real* st_i, Real* st_j, int r, 
     *reinterpret_cast<R4<Real>*>((e < RL::ci ? st_i : st_j) + RL::pitch * k + 4 * RL::chunk(e)) = v;
 }
 
+// One entry (r, c) of block bk, the pairs' sum v, into S.
+__device__ __forceinline__ void pair_entry(const int4 bk, int r, int c, double v, const double* __restrict__ dc2, double* S,
+                                           int ld) {
+    const int ca = bk.x, cb = bk.y;
+    const double s = (ca == cb && r == c ? dc2[9 * ca + r] : 0.0) - v;
+    S[(size_t)(9 * ca + r) * ld + 9 * cb + c] = s;
+    if (ca != cb) S[(size_t)(9 * cb + c) * ld + 9 * ca + r] = s;
+}
+
 // Block bk = (camera a, camera b, first pair, end pair) of the pair list `pairs` (observation
 // indices (i, j) into the records js) into S; dc2 holds D^2 (added on the diagonal of a == b).
-template <typename Real, int LAYOUT>
-__device__ __forceinline__ void pair_block(const int4 bk, const int2* __restrict__ pairs, const Real* __restrict__ js,
-                                           const double* __restrict__ dc2, double* S, int ld, Real* stage) {
+// NW > 1: the workgroup's NW waves take the block's stages in turn (wave w the stages w, w + NW, ...; each
+// with its own staging area) and their sums are added in neighbouring pairs through sums (NW x 81 doubles of LDS); every wave of the workgroup must call it.
+template <typename Real, int LAYOUT, int NW = 1>
+__device__ __forceinline__ void pair_block(const int4 bk_all, const int2* __restrict__ pairs, const Real* __restrict__ js,
+                                           const double* __restrict__ dc2, double* S, int ld, Real* stage,
+                                           double* sums = nullptr) {
     using RL = RecLayout<LAYOUT>;
+    const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    int4 bk = bk_all;
+    bk.z = min(bk.z + kPairsPerStage * wave, bk.w);
+    constexpr int kStride = NW * kPairsPerStage;  // pairs between two stages of a wave
     constexpr int PS = kPairsPerStage;
     static_assert(PS == 16, "one pair per lane of a 16-lane row");
     const int lane = threadIdx.x & 63, q = lane & 15, h = lane >> 4;
@@ -101,16 +118,21 @@ __device__ __forceinline__ void pair_block(const int4 bk, const int2* __restrict
     for (int r = 0; r < 9; ++r)
 #pragma unroll
         for (int k = 0; k < 3; ++k) acc[r][k] = 0.0;
-    const int npairs = bk.w - bk.z;
-    const int nst = (npairs + PS - 1) / PS;
+    const int npairs = bk.w - bk.z;  // up to the block's end, the other waves' stages among them
+    const int nst = (npairs + kStride - 1) / kStride;
     int2 pr = make_int2(0, 0), pr_next = make_int2(0, 0);
     if (lane < min(PS, npairs)) pr = pairs[bk.z + lane];
-    if (nst > 1 && lane < min(PS, npairs - PS)) pr_next = pairs[bk.z + PS + lane];
+    if (nst > 1 && lane < min(PS, npairs - kStride)) pr_next = pairs[bk.z + kStride + lane];
     int m_ld = min(PS, npairs);
-    R4<Real> b0 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 0), b1 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 1),
-             b2 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 2), b3 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 3);
+    R4<Real> b0{}, b1{}, b2{}, b3{};
+    if (NW == 1 || nst > 0) {
+        b0 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 0);
+        b1 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 1);
+        b2 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 2);
+        b3 = pair_load_round<Real, LAYOUT>(js, pr, m_ld, 3);
+    }
     for (int stg = 0; stg < nst; ++stg) {
-        const int base = bk.z + stg * PS;
+        const int base = bk.z + stg * kStride;
         const int m = min(PS, bk.w - base);
         pair_store_round<Real, LAYOUT>(st_i, st_j, 0, b0);
         pair_store_round<Real, LAYOUT>(st_i, st_j, 1, b1);
@@ -122,8 +144,8 @@ __device__ __forceinline__ void pair_block(const int4 bk, const int2* __restrict
         // loads complete in order)
         int2 pr_far = make_int2(0, 0);
         if (stg + 1 < nst) {
-            if (stg + 2 < nst && lane < min(PS, bk.w - base - 2 * PS)) pr_far = pairs[base + 2 * PS + lane];
-            m_ld = min(PS, bk.w - base - PS);
+            if (stg + 2 < nst && lane < min(PS, bk.w - base - 2 * kStride)) pr_far = pairs[base + 2 * kStride + lane];
+            m_ld = min(PS, bk.w - base - kStride);
             b0 = pair_load_round<Real, LAYOUT>(js, pr_next, m_ld, 0);
             b1 = pair_load_round<Real, LAYOUT>(js, pr_next, m_ld, 1);
             b2 = pair_load_round<Real, LAYOUT>(js, pr_next, m_ld, 2);
@@ -177,7 +199,6 @@ __device__ __forceinline__ void pair_block(const int4 bk, const int2* __restrict
         pr = pr_next;
         pr_next = pr_far;
     }
-    const int ca = bk.x, cb = bk.y;
 #pragma unroll
     for (int r = 0; r < 9; ++r) {
 #pragma unroll
@@ -185,10 +206,24 @@ __device__ __forceinline__ void pair_block(const int4 bk, const int2* __restrict
             const double v = row16_sum(acc[r][k]);
             const int c = c0 + k;
             if (q == 0 && k < nc) {
-                const double s = (ca == cb && r == c ? dc2[9 * ca + r] : 0.0) - v;
-                S[(size_t)(9 * ca + r) * ld + 9 * cb + c] = s;
-                if (ca != cb) S[(size_t)(9 * cb + c) * ld + 9 * ca + r] = s;
+                if (NW == 1)
+                    pair_entry(bk, r, c, v, dc2, S, ld);
+                else
+                    sums[81 * wave + 9 * r + c] = v;
             }
+        }
+    }
+    if (NW > 1) {
+        lds_barrier();
+        for (int e = threadIdx.x; e < 81; e += 64 * NW) {
+            double v[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v[w] = sums[81 * w + e];
+#pragma unroll
+            for (int h = 1; h < NW; h *= 2)
+#pragma unroll
+                for (int w = 0; w + h < NW; w += 2 * h) v[w] += v[w + h];
+            pair_entry(bk, e / 9, e % 9, v[0], dc2, S, ld);
         }
     }
 }
