@@ -416,7 +416,7 @@ struct Solver final : SolverBase {
         d.st = st.p;
         d.trace = trace.p;
         d.trace_cap = trace_cap;
-        if (linear_solver == BA_SOLVER_DENSE_SCHUR) BA_TRY(dense.create(v, L, o, s));
+        if (linear_solver == BA_SOLVER_DENSE_SCHUR) BA_TRY(dense.create(L, cam_off.p, co_pt.p, o, s));
         BA_TRY(reset());
         return BA_OK;
     }

@@ -24,3 +24,31 @@ def test_dense_sizes_match_oracle(oracle_mod, nc):
     # radius 1e4) times unit roundoff, per step
     assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-8 * ref["final_cost"]
     np.testing.assert_allclose(p.cameras(), ref["cams"], rtol=0, atol=1e-7 * np.abs(ref["cams"]).max())
+
+
+# Pair lists of the reduced system: observations in random order, points seen twice by one camera (its own
+# block then has pairs of two observations), cameras without observations and pairs of cameras without a
+# common point (two separate halves).
+@pytest.mark.parametrize("nc,repeats", [(5, 0), (6, 1), (13, 7), (66, 40)])
+def test_dense_pair_lists_match_oracle(oracle_mod, nc, repeats):
+    rng = np.random.default_rng(nc)
+    half = S.synthetic(2, seed=nc, num_cameras=nc, num_points=30 * nc, max_track=min(6, nc))
+    ci, pi = half.camera_index(), half.point_index()
+    no, npt = ci.size, half.num_points()
+    obs = half.observations().reshape(-1, 2)
+    twice = rng.choice(no, repeats, replace=False)
+    order = rng.permutation(2 * no + repeats)
+    # the second half's cameras follow an unused one (index nc), its points follow the first half's
+    ci = np.concatenate([ci, ci + nc + 1, ci[twice]])[order]
+    pi = np.concatenate([pi, pi + npt, pi[twice]])[order]
+    ob = np.concatenate([obs, obs, obs[twice] + rng.normal(0, 0.3, (repeats, 2))])[order]
+    cams = half.cameras().reshape(-1, 9)
+    cams = np.concatenate([cams, cams[:1], cams])
+    pts = np.concatenate([half.points(), half.points()])
+    p = S.BALProblem.from_arrays(ci, pi, ob, cams, pts)
+    ref = oracle_mod.solve(p.num_cameras(), p.num_points(), p.camera_index(), p.point_index(), p.observations(),
+                           p.cameras(), p.points(), oracle_mod.default_options(**FIXED))
+    out = S.SolveBA(p, linear_solver=C.SOLVER_DENSE_SCHUR, **FIXED)
+    # as above: at most 1e7 in condition times unit roundoff, per step
+    assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-8 * ref["final_cost"]
+    np.testing.assert_allclose(p.cameras(), ref["cams"], rtol=0, atol=1e-7 * np.abs(ref["cams"]).max())
