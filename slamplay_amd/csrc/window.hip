@@ -242,6 +242,42 @@ __global__ void k_window_reset(const WinDesc* __restrict__ descs, char* __restri
     }
 }
 
+// Places the images of a lane's windows: window t's inputs from the staged copy into its region, the
+// rest of the region zeroed.  One upload and one launch per lane; a window used to take two copies and
+// a fill of its own, 20 us of runtime calls each (64 stereo windows: 4.5 ms).  gridDim.y workgroups per
+// window, 16 bytes per thread and turn (regions and staged inputs are 256-byte multiples).
+struct PlaceTask {
+    int64_t src, dst, in_bytes, total;
+};
+constexpr int kPlaceSplit = 16;
+__global__ void __launch_bounds__(256) k_window_place(const char* __restrict__ staged, char* __restrict__ arena,
+                                                      const PlaceTask* __restrict__ tasks) {
+    const PlaceTask t = tasks[blockIdx.x];
+    const int64_t n_in = t.in_bytes / 16, n = t.total / 16;
+    const uint4* src = reinterpret_cast<const uint4*>(staged + t.src);
+    uint4* dst = reinterpret_cast<uint4*>(arena + t.dst);
+    for (int64_t i = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.y * blockDim.x)
+        dst[i] = i < n_in ? src[i] : make_uint4(0, 0, 0, 0);
+}
+
+// The windows' parameters in the caller's order, packed: 9 K camera values, then 3 P point values at
+// out_off; inv holds each window's internal index of every caller point.
+struct PackTask {
+    int slot, K, P, pad;
+    int64_t inv_off, out_off;
+};
+__global__ void __launch_bounds__(256) k_window_pack(const WinDesc* __restrict__ descs, char* __restrict__ arena,
+                                                     const PackTask* __restrict__ tasks, const int* __restrict__ inv,
+                                                     double* __restrict__ out) {
+    const PackTask t = tasks[blockIdx.x];
+    const WinDesc D = descs[t.slot];
+    const double* cx = at<double>(arena, D.o_cam_x);
+    const double* px = at<double>(arena, D.o_pt_x);
+    double* o = out + t.out_off;
+    for (int k = threadIdx.x; k < 9 * t.K; k += 256) o[k] = cx[k];
+    for (int e = threadIdx.x; e < 3 * t.P; e += 256) o[9 * t.K + e] = px[4 * (size_t)inv[t.inv_off + e / 3] + e % 3];
+}
+
 // Gathers the LM states of the listed windows into out (one thread per window).
 __global__ void k_window_states(const WinDesc* __restrict__ descs, const char* __restrict__ arena,
                                 const int* __restrict__ work, int n_work, WinState* __restrict__ out) {
@@ -364,6 +400,36 @@ struct WindowEngine {
         hdesc[slot] = rebase(img.desc, base);
         BA_HIP(hipMemcpyAsync(ddesc.p + slot, &hdesc[slot], sizeof(WinDesc), hipMemcpyHostToDevice, s));
         work_slots.clear();  // the task lists depend on the windows' sizes: rebuild them
+        return BA_OK;
+    }
+
+    // Places the images of windows `slots` at consecutive offsets from the start of the arena
+    // (synchronous: the images may go afterwards).
+    int place_all(const std::vector<WindowImage>& imgs, const std::vector<int>& slots) {
+        if (slots.empty()) return BA_OK;
+        std::vector<PlaceTask> tasks;
+        int64_t base = 0, staged = 0;
+        for (int w : slots) {
+            const int64_t in = (int64_t)imgs[w].bytes.size();
+            tasks.push_back(PlaceTask{staged, base, in, imgs[w].total});
+            hdesc[w] = rebase(imgs[w].desc, base);
+            staged += in;
+            base += imgs[w].total;
+        }
+        if (base > arena_cap) return fail(BA_ERR_CAPACITY, "windows do not fit the arena");
+        std::vector<char> host((size_t)staged);
+        for (size_t i = 0; i < slots.size(); ++i)
+            std::memcpy(host.data() + tasks[i].src, imgs[slots[i]].bytes.data(), (size_t)tasks[i].in_bytes);
+        DevBuf<char> dstaged;
+        DevBuf<PlaceTask> dtasks;
+        BA_TRY(dstaged.upload(host.data(), host.size(), s));
+        BA_TRY(dtasks.upload(tasks.data(), tasks.size(), s));
+        BA_HIP(hipMemcpyAsync(ddesc.p, hdesc.data(), hdesc.size() * sizeof(WinDesc), hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_window_place, dim3((unsigned)slots.size(), kPlaceSplit), dim3(256), 0, s, (const char*)dstaged.p,
+                           arena.p, (const PlaceTask*)dtasks.p);
+        BA_HIP(hipGetLastError());
+        work_slots.clear();
+        BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }
 
@@ -667,14 +733,10 @@ struct Batch final : BatchBase {
             int64_t total = 0;
             for (int w : lane_order[l]) total += imgs[w].total;
             BA_TRY(eng->init(o, total, count, lane_streams[l]));
-            int64_t base = 0;
-            for (int w : lane_order[l]) {
-                BA_TRY(eng->place(imgs[w], w, base));
-                base += imgs[w].total;
-            }
-            BA_HIP(hipStreamSynchronize(eng->s));
+            BA_TRY(eng->place_all(imgs, lane_order[l]));
             lanes.push_back(std::move(eng));
         }
+        BA_TRY(prepare_packing());
         // the host images are only needed for their permutations from here on
         for (int w : small) std::vector<char>().swap(imgs[w].bytes);
         if (tune) return autotune();
@@ -746,6 +808,7 @@ struct Batch final : BatchBase {
     // Milliseconds of two LM iterations of every lane, launched together (host clock around the
     // launches and the waits); the windows are reset before and after.
     int time_iteration(double* ms) {
+        params_changed();
         const int nl = (int)lanes.size();
         for (int l = 0; l < nl; ++l) {
             BA_TRY(lanes[l]->reset(lane_order[l]));
@@ -815,6 +878,7 @@ struct Batch final : BatchBase {
 
     int run(ba_summary* summaries) override {
         BA_TRY(use_device(opt.device));
+        params_changed();
         const bool graphs = opt.launch_mode == 0;
         const int nl = (int)lanes.size();
         // one LM trial per launch sequence, the first after the initial linearization: under the
@@ -878,16 +942,87 @@ struct Batch final : BatchBase {
     }
 
     int reset() override {
+        params_changed();
         for (size_t l = 0; l < lanes.size(); ++l) BA_TRY(lanes[l]->reset(lane_order[l]));
         for (auto& sv : large_solvers) BA_TRY(sv->reset());
         for (auto& e : lanes) BA_HIP(hipStreamSynchronize(e->s));
         return BA_OK;
     }
 
+    // The first download after the windows' parameters changed fetches its window alone; the second
+    // one, so a caller that reads several, fetches all of them packed by one kernel per lane, and
+    // later ones read that copy until the parameters change again.  (512 windows one by one: 19.3 ms of
+    // copies, waits and host permutations of 38 us each.)
     int download(int w, double* cams, double* pts) override {
         if (w < 0 || w >= (int)imgs.size()) return fail(BA_ERR_INVALID_ARGUMENT, "window %d out of range", w);
         if (large_index[w] >= 0) return large_solvers[large_index[w]]->download(cams, pts);
-        return lanes[lane_of[w]]->download(w, imgs[w].pt_perm, cams, pts);
+        if (downloads++ == 0) return lanes[lane_of[w]]->download(w, imgs[w].pt_perm, cams, pts);
+        if (!fetched) BA_TRY(fetch_all());
+        const double* src = host_params.data() + pack[pack_of[w]].out_off;
+        if (cams) std::copy(src, src + 9 * (size_t)imgs[w].K, cams);
+        if (pts) std::copy(src + 9 * (size_t)imgs[w].K, src + 9 * (size_t)imgs[w].K + 3 * (size_t)imgs[w].P, pts);
+        return BA_OK;
+    }
+
+    // Results on the host: the pack tasks lane after lane (lane l's are [pack_first[l], pack_first[l + 1])).
+    std::vector<PackTask> pack;
+    std::vector<int> pack_of;  // window -> its task
+    std::vector<size_t> pack_first;
+    DevBuf<PackTask> dpack;
+    DevBuf<int> dinv;
+    DevBuf<double> dparams;
+    std::vector<double> host_params;
+    int64_t n_params = 0;
+    int downloads = 0;     // since the parameters last changed
+    bool fetched = false;  // host_params holds them
+
+    void params_changed() {
+        downloads = 0;
+        fetched = false;
+    }
+
+    int prepare_packing() {
+        pack.clear();
+        pack_of.assign(imgs.size(), -1);
+        pack_first.assign(1, 0);
+        std::vector<int> inv;
+        n_params = 0;
+        for (const auto& order : lane_order) {
+            for (int w : order) {
+                const WindowImage& im = imgs[w];
+                pack_of[w] = (int)pack.size();
+                pack.push_back(PackTask{w, im.K, im.P, 0, (int64_t)inv.size(), n_params});
+                n_params += 9 * (int64_t)im.K + 3 * (int64_t)im.P;
+                const size_t o = inv.size();
+                inv.resize(o + im.P);
+                for (int ip = 0; ip < im.P; ++ip) inv[o + im.pt_perm[ip]] = ip;
+            }
+            pack_first.push_back(pack.size());
+        }
+        if (pack.empty()) return BA_OK;
+        hipStream_t s = lanes[0]->s;
+        BA_TRY(dpack.upload(pack.data(), pack.size(), s));
+        BA_TRY(dinv.upload(inv.data(), inv.size(), s));
+        BA_HIP(hipStreamSynchronize(s));
+        return BA_OK;
+    }
+
+    int fetch_all() {
+        BA_TRY(use_device(opt.device));
+        if (!dparams.p) BA_TRY(dparams.alloc((size_t)n_params));
+        host_params.resize((size_t)n_params);
+        for (size_t l = 0; l < lanes.size(); ++l) {
+            const size_t n = pack_first[l + 1] - pack_first[l];
+            if (n)
+                hipLaunchKernelGGL(k_window_pack, dim3((unsigned)n), dim3(256), 0, lanes[l]->s, (const WinDesc*)lanes[l]->ddesc.p,
+                                   lanes[l]->arena.p, (const PackTask*)dpack.p + pack_first[l], (const int*)dinv.p, dparams.p);
+        }
+        BA_HIP(hipGetLastError());
+        for (auto& e : lanes) BA_TRY(e->sync("window results"));
+        BA_HIP(hipMemcpyAsync(host_params.data(), dparams.p, (size_t)n_params * sizeof(double), hipMemcpyDeviceToHost, lanes[0]->s));
+        BA_TRY(lanes[0]->sync("window results"));
+        fetched = true;
+        return BA_OK;
     }
 };
 

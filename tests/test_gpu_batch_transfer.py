@@ -1,0 +1,46 @@
+"""Batch results read one window at a time (the first download after a change fetches its window alone,
+later ones a packed copy of all): every order of reading gives the parameters the batch holds now."""
+import numpy as np
+import pytest
+
+import slamplay_amd as S
+
+pytestmark = pytest.mark.gpu
+
+FIXED = dict(max_num_iterations=3, function_tolerance=0.0, gradient_tolerance=0.0, parameter_tolerance=0.0)
+
+
+# windows of (cameras, points): a single one, a few (one of them beyond the batched kernels, 36
+# cameras, and one of 64 points, one chunk exactly), and enough for two lanes
+@pytest.mark.parametrize("sizes", [[(5, 30)], [(5, 65), (36, 200), (8, 64), (6, 200)], [(5 + i % 3, 40 + i) for i in range(66)]])
+def test_batch_downloads_follow_the_parameters(sizes):
+    probs = [S.synthetic(4, seed=i + 1, num_cameras=c, num_points=n, max_track=min(c, 6)) for i, (c, n) in enumerate(sizes)]
+    start = [(p.cameras().copy(), p.points().copy()) for p in probs]
+    n = len(probs)
+
+    def alone(w, run):
+        """Window w read as the only download after the change."""
+        b.reset()
+        if run:
+            b.run()
+        return b.download(w)
+
+    def same(x, y):
+        np.testing.assert_array_equal(x[0], y[0])
+        np.testing.assert_array_equal(x[1], y[1])
+
+    b = S.Batch(probs, **FIXED)
+    some = sorted({0, n // 2, n - 1})
+    solved = {w: alone(w, True) for w in some}
+    b.reset()
+    for w in range(n):
+        same(b.download(w), start[w])  # the second one fetches all
+    b.run()
+    for w in reversed(range(n)):
+        got = b.download(w)
+        if w in solved:
+            same(got, solved[w])
+    b.reset()
+    for w in some:
+        same(b.download(w), start[w])  # not the fetched solution
+    b.close()
