@@ -216,6 +216,19 @@ void build_pair_blocks(const Layout& L, PairBlocks* out) {
     o.off.push_back((int)cnt[nkey]);
 }
 
+// Parameters in the caller's layout: cameras 9 values each, points 3 values each in the caller's order
+// (orig[internal point] = caller point).
+__global__ void __launch_bounds__(kWG) k_params_out(const double* __restrict__ cam_x, int nc, const double* __restrict__ pt_x,
+                                                    const int* __restrict__ orig, int np, double* __restrict__ cams,
+                                                    double* __restrict__ pts) {
+    const int64_t e = (int64_t)blockIdx.x * kWG + threadIdx.x;
+    if (e < 9 * (int64_t)nc) cams[e] = cam_x[(e % 9) * nc + e / 9];
+    if (e < 3 * (int64_t)np) {
+        const int64_t ip = e / 3, i = e % 3;
+        pts[3 * (int64_t)orig[ip] + i] = pt_x[4 * ip + i];
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Threads per workgroup of k_jz_dir and k_jtx_dir (one workgroup per camera).  128 for k_jz_dir:
 // at its register use a CU then holds eight of them, so the 1,500 cameras of the 1.2M-observation
@@ -248,7 +261,7 @@ struct Solver final : SolverBase {
     DevBuf<double> cam_part, pt_part;
     DevBuf<LMState> st;
     DevBuf<ba_iteration> trace;
-    DevBuf<int> pt_orig;  // internal point -> caller point, uploaded on the first Normalize / Perturb
+    DevBuf<int> pt_orig;  // internal point -> caller point
     PrepScratch prep_w;
     LMState* st_host = nullptr;  // pinned
     double wait_timeout_s = 0.0;
@@ -313,6 +326,7 @@ struct Solver final : SolverBase {
         BA_TRY(chunk_off.upload(L.chunk_off.data(), L.chunk_off.size(), s));
         BA_TRY(chunk_len.upload(L.chunk_len.data(), L.chunk_len.size(), s));
         BA_TRY(slot_of.upload(L.slot_of.data(), L.slot_of.size(), s));
+        BA_TRY(pt_orig.upload(L.pt_perm.data(), L.pt_perm.size(), s));
         BA_TRY(co_uv64.upload(L.co_uv.data(), L.co_uv.size(), s));
         if (sizeof(Real) != sizeof(double)) {
             std::vector<Real> uvr(L.co_uv.begin(), L.co_uv.end());
@@ -443,7 +457,6 @@ struct Solver final : SolverBase {
 
     int prep_params(DeviceParams* p) {
         BA_TRY(use_device(device));
-        if (!pt_orig.p && L.np) BA_TRY(pt_orig.upload(L.pt_perm.data(), L.pt_perm.size(), s));
         *p = DeviceParams{cam_x.p, pt_x.p, pt_orig.p, L.nc, L.np};
         return BA_OK;
     }
@@ -465,18 +478,17 @@ struct Solver final : SolverBase {
         return BA_OK;
     }
 
+    // The caller's layouts are formed on the device (into the step buffers, which hold nothing between
+    // runs) and copied straight into the caller's arrays: 370 -> 200 us for 1,500 cameras and 100k points,
+    // against staging vectors and a permutation on the host.
     int download(double* cams, double* pts) override {
         const int nc = L.nc, np = L.np;
-        std::vector<double> cx(9 * (size_t)nc), px_(4 * (size_t)np);
-        if (nc) BA_HIP(hipMemcpyAsync(cx.data(), cam_x.p, cx.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-        if (np) BA_HIP(hipMemcpyAsync(px_.data(), pt_x.p, px_.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+        hipLaunchKernelGGL(k_params_out, dim3(std::max(1, div_up(std::max(9 * (int64_t)nc, 3 * (int64_t)np), kWG))), dim3(kWG),
+                           0, s, (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, dcam.p, dpt.p);
+        BA_HIP(hipGetLastError());
+        if (cams && nc) BA_HIP(hipMemcpyAsync(cams, dcam.p, 9 * (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (pts && np) BA_HIP(hipMemcpyAsync(pts, dpt.p, 3 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, s));
         BA_HIP(hipStreamSynchronize(s));
-        if (cams)
-            for (int c = 0; c < nc; ++c)
-                for (int i = 0; i < 9; ++i) cams[9 * (size_t)c + i] = cx[(size_t)i * nc + c];
-        if (pts)
-            for (int ip = 0; ip < np; ++ip)
-                for (int i = 0; i < 3; ++i) pts[3 * (size_t)L.pt_perm[ip] + i] = px_[4 * (size_t)ip + i];
         return BA_OK;
     }
 
