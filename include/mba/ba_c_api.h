@@ -197,7 +197,7 @@ int ba_summary_full_report(const ba_summary* summary, int32_t num_cameras, int32
  * that forbid hipMalloc).  Every pointer of `problem` and `cost` (one double) is DEVICE memory on
  * the current device; the kernels of ba_eval_cost are enqueued on `stream` (a hipStream_t, NULL for
  * the null stream) and the call returns without waiting.  Work space is a fixed per-GPU buffer of
- * the library (about 1.8 MB, held until the process ends): at most 4096 cameras and 2^24
+ * the library (about 0.4 MB, held until the process ends): at most 4096 cameras and 2^24
  * observations (BA_ERR_CAPACITY beyond).  Indices are not checked on the host; an out-of-range
  * index makes the cost NaN.  Calls that overlap on one GPU share the buffer and race. */
 int ba_eval_cost_noalloc(const ba_problem_view* problem, int32_t loss, double loss_scale, double* cost,
