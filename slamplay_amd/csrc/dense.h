@@ -210,8 +210,7 @@ __device__ __forceinline__ typename Mfma<F>::acc tile_mma_nt(const F* __restrict
 // Lane r < 32 keeps row r of the tile in registers, lane 32 + i row i of the identity: the column
 // operations that turn the tile into L (column j scaled by 1 / l_jj, column c less l_cj times column j)
 // turn the identity below it into L^-T, whose row i is column i of X, so the inverse costs no
-// instructions of its own.  The pivot and the entries l_cj of the scaled column are read from their
-// lanes with v_readlane: no trip through LDS and no serial sum.  Entries above the tile's diagonal are
+// instructions of its own (potrf_stacked).  Entries above the tile's diagonal are
 // updated with the rest and never read by another lane.  Returns false (and writes nothing) when a
 // pivot is not positive and finite.  Only one whole wave may call it.
 template <typename F>
@@ -219,10 +218,10 @@ __device__ __forceinline__ bool potrf_tile_wave(F (*T)[kTile + 1], F* __restrict
     const int l = threadIdx.x & 63, r = l & 31;
     F a[kTile];
 #pragma unroll
-    for (int c = 0; c < kTile; ++c) {
-        const F t = T[r][c];
-        a[c] = l < kTile ? t : (r == c ? (F)1 : (F)0);
-    }
+    for (int c = 0; c < kTile; ++c) a[c] = l == kTile + c ? (F)1 : (F)0;
+    if (l < kTile)
+#pragma unroll
+        for (int c = 0; c < kTile; ++c) a[c] = T[r][c];
     if (!potrf_stacked<F>(a)) return false;
     if (l >= kTile)
 #pragma unroll
@@ -569,6 +568,26 @@ __global__ void __launch_bounds__(kWG) k_residual(const double* __restrict__ S, 
     if (lane == 0) r[row] = b[row] - v;
 }
 
+// The whole factor and solve of a small reduced system by one workgroup (tile_chol.h): S's lower
+// triangle and b packed into LDS.  One launch in place of the tile steps, the block inverse and the sweeps.
+constexpr int kSmallThreads = 512;
+__global__ void __launch_bounds__(kSmallThreads) k_dense_small(const double* __restrict__ S, int ld, const double* __restrict__ b,
+                                                               double* __restrict__ x, int n, LMState* st) {
+    if (st->done || st->step_invalid) return;
+    extern __shared__ __align__(16) double small_lds[];
+    __shared__ int bad;
+    if (threadIdx.x == 0) bad = 0;
+    small_load<kSmallThreads>(S, ld, b, n, small_lds);
+    lds_barrier();
+    small_factor<kSmallThreads, false>(small_lds, n, &bad);
+    if (bad) {
+        if (threadIdx.x == 0) st->step_invalid = 1;
+        return;
+    }
+    small_backward<kSmallThreads, false>(small_lds, n);
+    for (int k = threadIdx.x; k < n; k += kSmallThreads) x[k] = small_lds[tri(n) + k];
+}
+
 __global__ void k_set_linear_iters(LMState* st, int iters) {
     if (st->done || st->step_invalid) return;
     st->pcg_iters = iters;
@@ -578,6 +597,10 @@ __global__ void k_set_linear_iters(LMState* st, int iters) {
 // microseconds there, and an FP32 factor of a small, nearly gauge-free system (a local window whose
 // trust region has grown) would need a Krylov solve on top to reach the FP64 step.
 constexpr int kDenseF64MaxN = 288;
+// Systems up to this size (22 cameras, 159 KB of LDS) are factored and solved by one workgroup: 26 us at 8
+// cameras and 71 at 22, against 35 and 85 for the tile steps, block inverse and sweeps; past it the
+// triangle does not fit the LDS.
+constexpr int kDenseSmallN = 198;
 
 template <typename Real>
 struct DenseSchur {
@@ -674,7 +697,9 @@ struct DenseSchur {
         BA_TRY(z.alloc(ld));
         BA_TRY(y.alloc(ld));
         const size_t binv = (size_t)nb * kSolveRows * kSolveRows;
-        if (f64) {
+        if (n <= kDenseSmallN) {
+            BA_TRY(allow_dynamic_lds((const void*)k_dense_small, (int)(small_system_doubles(n) * sizeof(double))));
+        } else if (f64) {
             BA_TRY(Dinvd.alloc((size_t)nt * kTile * kTile));
             BA_TRY(Binvd.alloc(binv));
             BA_TRY(BinvTd.alloc(binv));
@@ -753,7 +778,10 @@ struct DenseSchur {
             enqueue_schur<8>(sv);
         else
             enqueue_schur<4>(sv);
-        if (f64) {
+        if (n <= kDenseSmallN) {
+            sv.launch_shm("small_solve", k_dense_small, 1, kSmallThreads, small_system_doubles(n) * sizeof(double),
+                          (const double*)S.p, ld, (const double*)d.bc, d.px, n, d.st);
+        } else if (f64) {
             factor_and_solve<double>(sv, S.p, Dinvd.p, Binvd.p, BinvTd.p);
         } else {
             sv.launch("convert_S", k_convert_S<float>, (int)((nn + 255) / 256), 256, (const double*)S.p, Af.p, nn,

@@ -47,7 +47,7 @@ int64_t lds_per_block() {
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
 
-// Static LDS of k_wsolve (xv, colv, dinv, bad) plus slack for alignment.
+// LDS of k_wsolve beside the packed triangle: its right-hand side row and flag, and room for alignment.
 int64_t solve_static_lds() { return 3 * kWinMaxN * 8 + 16 + 256; }
 
 // Largest reduced system (9 K) k_wsolve can factor in LDS (0: none).
@@ -154,7 +154,7 @@ int build_window_image(const ba_problem_view* v, const ba_options& opt, WindowIm
     D.o_pv = take(96 * (int64_t)slots);
     D.o_js = take(kWinJs * sizeof(Real) * (int64_t)No);
     D.o_S = take(sizeof(double) * (int64_t)n * n);  // zero: blocks without common points are never written
-    D.o_L = take(sizeof(double) * (int64_t)n * (n + 1) / 2);  // the factor when it is not kept in LDS
+    D.o_L = take(sizeof(double) * (int64_t)small_system_doubles(n));  // the factor when it is not kept in LDS
     img->total = off;
     img->bytes.assign(input_bytes, 0);
     char* b = img->bytes.data();
@@ -536,7 +536,7 @@ struct WindowEngine {
     }
 
     // dynamic LDS of k_wsolve: the packed factor of the largest window factored in LDS
-    size_t solve_lds() const { return (size_t)work_nmax * (work_nmax + 1) / 2 * sizeof(double); }
+    size_t solve_lds() const { return (size_t)small_system_doubles(work_nmax) * sizeof(double); }
 
     template <int M>
     int enqueue_iteration_m() {

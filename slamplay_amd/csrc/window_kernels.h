@@ -12,7 +12,8 @@
 //   k_wschur      (window, block group) 9x9 blocks of S, each by one wave from LDS-staged
 //                 observation pairs;
 //   k_wsolve      (window) S copied as a packed lower triangle into LDS (or the window's global
-//                 buffer), right-looking FP64 Cholesky, blocked triangular solves;
+//                 buffer), FP64 Cholesky by 32-column tiles with the right-hand side as a last row,
+//                 backward sweep;
 //   k_wback_cam   (window, camera) u = J~_p'(r~ - J~_c y_c) into slot order (FP64);
 //   k_wback_pt    (window, point chunk) y_p = V*^-1 sum u, candidate points, |dx|^2, |x|^2;
 //   k_wcand_cam   (window, camera) candidate camera, model cost change, FP64 candidate cost;
@@ -31,15 +32,14 @@
 // share the launch, nor on the block sizes chosen for the launch.
 #pragma once
 
-#include "mfma.h"
 #include "pair_block.h"
+#include "tile_chol.h"
 #include "window.h"
 
 namespace mba {
 
 constexpr int kWinMaxN = 288;  // 9 * 32 cameras
 constexpr int kWinMaxK = kWinMaxN / 9;
-constexpr int kWinTb = 16;     // diagonal block of the triangular solves
 constexpr int kWinCamThreads = 256;  // block size of the per-camera kernels
 struct WinPtrs {
     int K, P, No, n_slots;
@@ -227,207 +227,6 @@ template <typename Real>
 constexpr int win_stage_bytes() {
     return pair_stage_bytes<Real, kRecWindow>();
 }
-
-// Packed lower-triangular storage: element (i, j), j <= i, at i (i + 1) / 2 + j (row i contiguous).
-__device__ __forceinline__ int tri(int i) { return i * (i + 1) / 2; }
-
-// In-place blocked right-looking Cholesky of the packed n x n matrix L (LDS, or the window's global
-// buffer); dinv receives 1 / L_jj.  Panels of kWinNb columns: wave 0 factors the panel's diagonal
-// block in registers (lane i holds row i; each column's entries move between lanes through LDS, no
-// barrier), then every thread solves its rows of the panel below the block against it
-// (x L11' = a, the entries of L11 read from LDS by all threads at once), so a panel costs two
-// barriers.  The trailing lower triangle is then updated with the panel by 16 x 16 tiles on the
-// matrix cores (one tile per wave at a time, K = 16 in four steps; entries past n or above the
-// diagonal are neither read nor written).  *bad is set when a pivot is not positive (the factor is
-// then meaningless and the caller rejects the step).  Every entry receives the same sequence of
-// operations as in a column-by-column right-looking factorization (its updates by the earlier
-// columns in order, then the scaling by 1 / sqrt(pivot)), fixed by the algorithm, not by the
-// workgroup size.
-constexpr int kWinNb = 16;
-
-template <typename F, int NT>
-__device__ __forceinline__ void win_panel(F* L, int n, int jb, int je, F* dinv, F* xch, int* bad) {
-    constexpr int NB = kWinNb, RS = (kWinMaxN - NB + NT - 1) / NT;
-    const int tid = threadIdx.x, nb = je - jb;
-    if (tid < 64) {
-        // the diagonal block: lane i < nb holds row jb + i; the pivot's reciprocal square root by
-        // the hardware estimate and Newton steps, each column's entries to the other lanes through
-        // xch (a wave's LDS operations complete in order)
-        const int i = tid;
-        F a[NB];
-#pragma unroll
-        for (int c = 0; c < NB; ++c) a[c] = (i < nb && c <= i) ? L[tri(jb + i) + jb + c] : (F)0;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            if (j < nb) {  // uniform
-                F djj = read_lane(a[j], j);
-                const bool nonpos = !(djj > (F)0);
-                if (nonpos) djj = (F)1;
-                const F inv = inv_sqrt(djj), d = djj * inv;
-                a[j] = i > j ? a[j] * inv : (i == j ? d : a[j]);
-                if (i == 0) {
-                    dinv[jb + j] = inv;
-                    if (nonpos) *bad = 1;
-                }
-                if (i < NB) xch[i] = a[j];
-                wave_sync_lds();
-#pragma unroll
-                for (int c = j + 1; c < NB; ++c) {
-                    if (c < nb) {  // uniform
-                        const F lcj = xch[c];
-                        if (i >= c && i < nb) a[c] = fma(-a[j], lcj, a[c]);
-                    }
-                }
-                wave_sync_lds();
-            }
-        }
-        if (i < nb)
-#pragma unroll
-            for (int c = 0; c < NB; ++c)
-                if (c <= i) L[tri(jb + i) + jb + c] = a[c];
-    }
-    __syncthreads();
-    // the panel's rows below the block: x_j = (a_j - sum_k<j x_k l_jk) / l_jj, k in order
-#pragma unroll
-    for (int s = 0; s < RS; ++s) {
-        const int row = je + tid + NT * s;
-        if (row < n) {
-            F a[NB];
-#pragma unroll
-            for (int c = 0; c < NB; ++c) a[c] = c < nb ? L[tri(row) + jb + c] : (F)0;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                if (j < nb) {
-#pragma unroll
-                    for (int k = 0; k < j; ++k) a[j] = fma(-a[k], L[tri(jb + j) + jb + k], a[j]);
-                    a[j] = a[j] * dinv[jb + j];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < NB; ++c)
-                if (c < nb) L[tri(row) + jb + c] = a[c];
-        }
-    }
-}
-
-template <typename F, int NT>
-__device__ __forceinline__ void win_cholesky(F* L, int n, F* dinv, F* xch, int* bad) {
-    constexpr int NW = NT / 64, NB = kWinNb;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int jb = 0; jb < n; jb += NB) {
-        const int je = min(jb + NB, n);
-        win_panel<F, NT>(L, n, jb, je, dinv, xch, bad);
-        __syncthreads();
-        if (je >= n) break;
-        // trailing update: L[r][c] -= sum_{k in [jb, je)} L[r][k] L[c][k] for je <= c <= r < n
-        const int m = n - je, T = (m + 15) / 16;
-        const int l16 = lane & 15, q = lane >> 4;
-        for (int tt = wave; tt < T * (T + 1) / 2; tt += NW) {
-            int ti = (int)((sqrtf(8.0f * tt + 1.0f) - 1.0f) * 0.5f);
-            while ((ti + 1) * (ti + 2) / 2 <= tt) ++ti;
-            while (ti * (ti + 1) / 2 > tt) --ti;
-            const int tk = tt - ti * (ti + 1) / 2;
-            const int r0 = je + 16 * ti, c0 = je + 16 * tk;
-            typename Mfma<F>::acc acc;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = r0 + Mfma<F>::row(lane, e), c = c0 + l16;
-                acc[e] = (r < n && c <= r) ? L[tri(r) + c] : (F)0;
-            }
-            const int ra = r0 + l16, cb = c0 + l16;
-#pragma unroll
-            for (int s4 = 0; s4 < NB / 4; ++s4) {
-                const int k = jb + 4 * s4 + q;
-                const F a = (ra < n && k < je) ? L[tri(ra) + k] : (F)0;
-                const F b = (cb < n && k < je) ? L[tri(cb) + k] : (F)0;
-                acc = Mfma<F>::mma(-a, b, acc);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = r0 + Mfma<F>::row(lane, e), c = c0 + l16;
-                if (r < n && c <= r) L[tri(r) + c] = acc[e];
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// x <- (L L')^-1 x for the LDS vector x (double), L the packed factor above.  Blocks of kWinTb
-// rows: the diagonal block by wave 0 (one row per lane), the rest of the vector by the workgroup.
-// Expects x complete on entry (after a barrier) and leaves it complete.
-template <typename F, int NT>
-__device__ __forceinline__ void win_chol_solve(const F* L, const F* dinv, int n, double* x) {
-    constexpr int TB = kWinTb;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // forward: L z = x
-    for (int kb = 0; kb < n; kb += TB) {
-        const int m = min(TB, n - kb);
-        if (wave == 0) {
-            // the lane's row of the diagonal block and the block's 1 / l_cc first, so that the
-            // serial chain below waits on no memory
-            double lr[TB], dv[TB];
-#pragma unroll
-            for (int c = 0; c < TB; ++c) {
-                lr[c] = (lane < m && c < lane) ? (double)L[tri(kb + lane) + kb + c] : 0.0;
-                dv[c] = c < m ? (double)dinv[kb + c] : 0.0;
-            }
-            double v = lane < m ? x[kb + lane] : 0.0;
-#pragma unroll
-            for (int c = 0; c < TB; ++c) {
-                if (c < m) {
-                    const double zc = read_lane(v, c) * dv[c];
-                    if (lane == c) v = zc;
-                    if (lane > c) v -= lr[c] * zc;
-                }
-            }
-            if (lane < m) x[kb + lane] = v;
-        }
-        __syncthreads();
-        for (int i = kb + m + tid; i < n; i += NT) {
-            const F* row = L + tri(i) + kb;
-            double s = 0.0;
-#pragma unroll
-            for (int c = 0; c < TB; ++c)
-                if (c < m) s += (double)row[c] * x[kb + c];
-            x[i] -= s;
-        }
-        __syncthreads();
-    }
-    // backward: L' y = z
-    const int last = ((n - 1) / TB) * TB;
-    for (int kb = last; kb >= 0; kb -= TB) {
-        const int m = min(TB, n - kb);
-        if (wave == 0) {
-            double lc[TB], dv[TB];
-#pragma unroll
-            for (int c = 0; c < TB; ++c) {
-                lc[c] = (c < m && lane < c) ? (double)L[tri(kb + c) + kb + lane] : 0.0;
-                dv[c] = c < m ? (double)dinv[kb + c] : 0.0;
-            }
-            double v = lane < m ? x[kb + lane] : 0.0;
-#pragma unroll
-            for (int c = TB - 1; c >= 0; --c) {
-                if (c < m) {
-                    const double yc = read_lane(v, c) * dv[c];
-                    if (lane == c) v = yc;
-                    if (lane < c) v -= lc[c] * yc;
-                }
-            }
-            if (lane < m) x[kb + lane] = v;
-        }
-        __syncthreads();
-        for (int i = tid; i < kb; i += NT) {
-            double s = 0.0;
-#pragma unroll
-            for (int c = 0; c < TB; ++c)
-                if (c < m) s += (double)L[tri(kb + c) + i] * x[kb + c];
-            x[i] -= s;
-        }
-        __syncthreads();
-    }
-}
-
-
 
 // ------------------------------------------------------------------------------------------------
 // Phase kernels.  ctask: (slot, camera) per workgroup; ptask: (slot, chunk) per 64-thread
@@ -773,52 +572,40 @@ __global__ void __launch_bounds__(NT) k_wschur(const WinDesc* __restrict__ descs
                           tk.w, &counter, reinterpret_cast<Real*>(smem + (size_t)wave * win_stage_bytes<Real>()));
 }
 
-// Per window: factor S (FP64) and solve for the camera step y_c (into yc).  The packed factor lives
-// in LDS when the window's reduced system has at most lds_n unknowns and in the window's own global
-// buffer (L2-resident at these sizes) otherwise; the arithmetic is the same either way.
+// Per window: factor S (FP64) and solve for the camera step y_c (into yc): tile_chol.h's small system.
+// The packed triangle lives in LDS when the window's reduced system has at most lds_n unknowns and in
+// the window's own global buffer (L2-resident at these sizes) otherwise; the arithmetic is the same
+// either way.  Latency-bound by its chain of tiles: a launch for 32 stereo windows of up to 10 keyframes
+// 73 -> 27 us, 20 keyframes 195-240 -> 85 us (against 16-column panels with the pivot columns exchanged
+// through LDS and both triangular sweeps by 16-row blocks).
+template <int NT, bool kGlobal>
+__device__ __forceinline__ void win_solve(const WinPtrs& w, const double* Sg, double* L, int* bad) {
+    const int n = 9 * w.K, tid = threadIdx.x;
+    if (tid == 0) *bad = 0;
+    small_load<NT>(Sg, n, w.bc, n, L);
+    small_barrier<kGlobal>();
+    small_factor<NT, kGlobal>(L, n, bad);
+    if (*bad) return;  // have_step stays 0: an invalid step
+    small_backward<NT, kGlobal>(L, n);
+    for (int k = tid; k < n; k += NT) w.yc[k] = L[tri(n) + k];
+    if (tid == 0) w.st->have_step = 1;
+}
+
 template <int NT>
 __global__ void __launch_bounds__(NT) k_wsolve(const WinDesc* __restrict__ descs, char* __restrict__ arena,
                                                const int* __restrict__ wtask, int ntask, int lds_n) {
     extern __shared__ __align__(32) unsigned char smem[];
-    __shared__ double xv[kWinMaxN], dinv[kWinMaxN], xch[kWinNb];
     __shared__ int bad;
     const int t = blockIdx.x;
     if (t >= ntask) return;
     const WinDesc D = descs[wtask[t]];
     const WinPtrs w = win_ptrs(D, arena);
-    WinState* st = w.st;
-    if (st->done || st->invalid) return;
-    const int K = w.K, n = 9 * K, tid = threadIdx.x;
+    if (w.st->done || w.st->invalid) return;
     const double* Sg = at<double>(arena, D.o_S);
-    double* S = n > lds_n ? at<double>(arena, D.o_L) : reinterpret_cast<double*>(smem);
-    const int ntri = n * (n + 1) / 2;
-    // packed copy of the lower triangle, eight loads in flight per thread
-    constexpr int U = 8;
-    for (int b0 = tid; b0 < ntri; b0 += U * NT) {
-        double v[U];
-        int ix[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int idx = min(b0 + u * NT, ntri - 1);
-            int i = (int)((sqrtf(8.0f * idx + 1.0f) - 1.0f) * 0.5f);
-            while (tri(i + 1) <= idx) ++i;
-            while (tri(i) > idx) --i;
-            ix[u] = idx;
-            v[u] = Sg[(size_t)i * n + (idx - tri(i))];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (b0 + u * NT < ntri) S[ix[u]] = v[u];
-    }
-    if (tid == 0) bad = 0;
-    __syncthreads();
-    win_cholesky<double, NT>(S, n, dinv, xch, &bad);
-    if (bad) return;  // have_step stays 0: an invalid step
-    for (int k = tid; k < n; k += NT) xv[k] = w.bc[k];
-    __syncthreads();
-    win_chol_solve<double, NT>(S, dinv, n, xv);
-    for (int k = tid; k < n; k += NT) w.yc[k] = xv[k];
-    if (tid == 0) st->have_step = 1;
+    if (9 * w.K > lds_n)
+        win_solve<NT, true>(w, Sg, at<double>(arena, D.o_L), &bad);
+    else
+        win_solve<NT, false>(w, Sg, reinterpret_cast<double*>(smem), &bad);
 }
 
 // Per (window, camera): u = J~_p'(r~ - J~_c y_c) into slot order.
