@@ -18,9 +18,9 @@ struct DeviceParams {
 
 // Scratch owned by the caller's handle, grown on demand and kept between calls.
 struct PrepScratch {
-    DevBuf<unsigned long long> sel_state;  // 4 selections x (prefix, mask, rank)
-    DevBuf<unsigned int> hist;             // digit counts of the four selections (256 each)
-    DevBuf<double> dist;                   // L1 distances to the median
+    DevBuf<unsigned long long> sel_state;  // 4 selections x (key, rank)
+    DevBuf<unsigned int> hist;             // digit counts of the four selections' two passes, collected keys
+    DevBuf<unsigned long long> keys;       // keys that share a selection's first digits (three selections at once)
     DevBuf<unsigned int> draws;            // glibc rand() outputs
     DevBuf<unsigned int> tables;           // jump-ahead matrices
     DevBuf<unsigned int> counts;           // accepted pairs per block, then their exclusive scan

@@ -89,48 +89,80 @@ const std::vector<uint32_t>& jump_tables() {
     return tables;
 }
 
-// One thread per chunk of kChunk draws: jump from the seed state to the chunk start, then run the
-// recurrence 31 draws at a time with the state in registers (s[j] += s[j+28] for the first three,
-// whose r_{i-3} is still the previous round's, s[j] += s[j-3] for the rest).  Each round's 64 x 31
-// draws of the workgroup go through LDS so that lanes store consecutive draws of one chunk.
-__global__ void __launch_bounds__(64) k_rand_generate(RandState start, const uint32_t* __restrict__ tables,
-                                                      int n_chunks, int64_t n_draws, uint32_t* __restrict__ out) {
-    __shared__ uint32_t tile[64][kDeg + 2];  // odd row stride: the per-thread row writes hit distinct banks
-    const int b = blockIdx.x * 64 + threadIdx.x;
-    const int lane_c = threadIdx.x / kDeg, lane_j = threadIdx.x < 2 * kDeg ? threadIdx.x - lane_c * kDeg : kDeg;
-    uint32_t s[kDeg];
+// A workgroup gives the draws of 64 consecutive chunks.  The first one's start state by the jumps of the
+// workgroup index's bits, in wave 0, one row of the 31 x 31 product per lane, while the other waves put
+// Q_0..Q_5 into LDS; the others by doubling, chunks n .. 2n - 1 from 0 .. n - 1 with Q_log2(n), the 31 n rows
+// spread over the threads.  Then one lane per chunk runs the recurrence 31 draws at a time with the state
+// in registers (s[j] += s[j+28] for the first three, whose r_{i-3} is still the previous round's,
+// s[j] += s[j-3] for the rest) into LDS, from where the workgroup stores its 15,872 words contiguously.
+// Bound by latency, not by what it writes: 818,000 draws (3.3 MB) take 15 us (132 with a whole product
+// per bit of the chunk index in every thread, 57 with one wave to a workgroup for all of this).
+constexpr int kBlockChunks = 64;
+constexpr int kBlockBits = 6;  // log2(kBlockChunks)
+constexpr int kChunkRow = kChunk + 1;  // odd row stride: the lanes' rows start in distinct banks
+constexpr int kStateRow = kDeg + 2;
+__global__ void __launch_bounds__(256) k_rand_generate(RandState start, const uint32_t* __restrict__ tables,
+                                                       int64_t n_draws, uint32_t* __restrict__ out) {
+    __shared__ uint32_t lds[kBlockChunks * kChunkRow];  // first the states and Q_0..Q_5, then the draws
+    static_assert(kBlockChunks * kStateRow + kBlockBits * kDeg * kDeg <= kBlockChunks * kChunkRow, "LDS of the start states");
+    uint32_t* const state = lds;
+    uint32_t* const Qs = lds + kBlockChunks * kStateRow;
+    const int t = threadIdx.x;
+    if (t >= 64) {
+        constexpr int n = kBlockBits * kDeg * kDeg, per = (n + 191) / 192;
+        uint32_t v[per];
 #pragma unroll
-    for (int j = 0; j < kDeg; ++j) s[j] = start.s[j];
-    for (int q = 0; q < kJumps && b < n_chunks && (b >> q); ++q) {
-        if (!((b >> q) & 1)) continue;
-        const uint32_t* Q = tables + (size_t)q * kDeg * kDeg;
-        uint32_t t[kDeg];
+        for (int i = 0; i < per; ++i) v[i] = tables[min(t - 64 + 192 * i, n - 1)];
 #pragma unroll
-        for (int i = 0; i < kDeg; ++i) {
+        for (int i = 0; i < per; ++i)
+            if (t - 64 + 192 * i < n) Qs[t - 64 + 192 * i] = v[i];
+    } else {
+        uint32_t mine = 0;  // entry t of the state
+#pragma unroll
+        for (int j = 0; j < kDeg; ++j) mine = t == j ? start.s[j] : mine;
+        for (int q = kBlockBits; q < kJumps && ((int)blockIdx.x >> (q - kBlockBits)); ++q) {
+            if (!(((int)blockIdx.x >> (q - kBlockBits)) & 1)) continue;
+            const uint32_t* Q = tables + (size_t)q * kDeg * kDeg + (t < kDeg ? t : 0) * kDeg;
+            uint32_t row[kDeg], acc = 0;
+#pragma unroll
+            for (int k = 0; k < kDeg; ++k) row[k] = Q[k];
+#pragma unroll
+            for (int k = 0; k < kDeg; ++k) acc += row[k] * (uint32_t)__builtin_amdgcn_readlane((int)mine, k);
+            mine = acc;
+        }
+        if (t < kDeg) state[t] = mine;
+    }
+    __syncthreads();
+    for (int q = 0; q < kBlockBits; ++q) {
+        const int n = 1 << q;
+        for (int e = t; e < kDeg * n; e += 256) {
+            const int m = e / kDeg, i = e - kDeg * m;
             uint32_t acc = 0;
 #pragma unroll
-            for (int k = 0; k < kDeg; ++k) acc += Q[i * kDeg + k] * s[k];
-            t[i] = acc;
+            for (int k = 0; k < kDeg; ++k) acc += Qs[q * kDeg * kDeg + i * kDeg + k] * state[m * kStateRow + k];
+            state[(m + n) * kStateRow + i] = acc;
         }
-#pragma unroll
-        for (int j = 0; j < kDeg; ++j) s[j] = t[j];
+        __syncthreads();
     }
-    for (int round = 0; round < kChunk / kDeg; ++round) {
+    uint32_t s[kDeg];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) s[j] += s[j + 28];
+    for (int j = 0; j < kDeg; ++j) s[j] = state[(t & 63) * kStateRow + j];
+    __syncthreads();
+    if (t < 64)
+        for (int round = 0; round < kChunk / kDeg; ++round) {
 #pragma unroll
-        for (int j = 3; j < kDeg; ++j) s[j] += s[j - 3];
+            for (int j = 0; j < 3; ++j) s[j] += s[j + 28];
 #pragma unroll
-        for (int j = 0; j < kDeg; ++j) tile[threadIdx.x][j] = s[j] >> 1;
-        __syncthreads();
-        // lanes 0-30 and 31-61 store the 31 draws of two chunks per instruction
-        if (lane_j < kDeg)
-            for (int c = lane_c; c < 64; c += 2) {
-                const int64_t bb = (int64_t)blockIdx.x * 64 + c;
-                const int64_t o = bb * kChunk + (int64_t)round * kDeg + lane_j;
-                if (bb < n_chunks && o < n_draws) out[o] = tile[c][lane_j];
-            }
-        __syncthreads();
+            for (int j = 3; j < kDeg; ++j) s[j] += s[j - 3];
+#pragma unroll
+            for (int j = 0; j < kDeg; ++j) lds[t * kChunkRow + round * kDeg + j] = s[j] >> 1;
+        }
+    __syncthreads();
+    const int64_t first = (int64_t)blockIdx.x * (kBlockChunks * kChunk);
+    const int n = (int)std::min<int64_t>(n_draws - first, kBlockChunks * kChunk);
+    for (int e = t; e < n; e += 256) {
+        const int c = e / kChunk;
+        out[first + e] = lds[c * kChunkRow + e - c * kChunk];
     }
 }
 
@@ -249,19 +281,21 @@ __device__ __forceinline__ void center_translation(const double aa[3], const dou
 }
 
 // BALProblem.cpp:305-336, points: X += n * sigma with the normals of the caller's point order
+// (both kernels leave the parameters alone when the stream gave too few normals: the host then draws a
+// longer one, and otherwise never waits between the draws and their use)
 __global__ void k_perturb_points(double* __restrict__ pt, const int* __restrict__ pt_orig, int np,
-                                 const double* __restrict__ normals, double sigma) {
+                                 const double* __restrict__ normals, double sigma, const int* __restrict__ got, int need) {
     const int ip = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ip >= np) return;
+    if (ip >= np || *got < need) return;
     const int64_t o = 3 * (int64_t)pt_orig[ip];
     for (int j = 0; j < 3; ++j) pt[4 * (int64_t)ip + j] += normals[o + j] * sigma;
 }
 
 // cameras: angle-axis += n * rs with the centre held, t recomputed, then t += n * ts
 __global__ void k_perturb_cams(double* __restrict__ cam, int nc, const double* __restrict__ normals, int64_t first,
-                               double rs, double ts) {
+                               double rs, double ts, const int* __restrict__ got, int need) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
+    if (c >= nc || (need > 0 && *got < need)) return;
     const int per = (rs > 0.0 ? 3 : 0) + (ts > 0.0 ? 3 : 0);
     int64_t k = first + (int64_t)per * c;
     double aa[3], t[3], center[3];
@@ -285,8 +319,16 @@ __global__ void k_perturb_cams(double* __restrict__ cam, int nc, const double* _
 
 // ---------------------------------------------------------------------------------------------
 // Upper median (nth_element at n/2, BALProblem.cpp:71-76) by radix selection over the IEEE bit
-// patterns mapped to order-preserving keys, 8 bits per pass from the top.  Selection k (0..2: a
-// point axis, 3: the L1 distances) keeps (prefix, mask, rank) in sel[3k..3k+2].
+// patterns mapped to order-preserving keys, from the top.  Selection k: 0..2 a point axis, 3 the L1
+// distances.  Two histograms of 11 bits over all keys (every block picks the digits found so far from
+// the previous counts itself, so a pass is one launch), then the keys that share those 22 bits -- a
+// thousandth of the range around the median, a few hundred of 100,000 -- are collected and one block
+// finishes on them (on all keys, if all are alike).  Bound by launches, 5 us each: four a selection, 43 us
+// for both selections of 100,000 points; eight passes of eight bits, with a launch each to pick the
+// digit, took 93 us.
+constexpr int kSelBits = 11;
+constexpr int kSelBins = 1 << kSelBits;
+constexpr int kSelShift0 = 64 - kSelBits, kSelShift1 = kSelShift0 - kSelBits;
 __device__ __forceinline__ unsigned long long order_key(double x) {
     const unsigned long long u = (unsigned long long)__double_as_longlong(x);
     return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
@@ -297,78 +339,128 @@ __device__ __forceinline__ double key_value(unsigned long long k) {
     return __longlong_as_double((long long)u);
 }
 
-__global__ void __launch_bounds__(256) k_sel_init(unsigned long long* __restrict__ sel, unsigned long long rank,
-                                                  unsigned int* __restrict__ hist) {
-    const int k = threadIdx.x;
-    if (k < 4) {
-        sel[3 * k] = 0;
-        sel[3 * k + 1] = 0;
-        sel[3 * k + 2] = rank;
-    }
-    for (int i = k; i < 4 * 256; i += 256) hist[i] = 0;
+// hist: [selection][pass 0, 1][kSelBins]; count: collected keys per selection
+__global__ void __launch_bounds__(256) k_sel_init(unsigned int* __restrict__ hist, unsigned int* __restrict__ count) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 4 * 2 * kSelBins) hist[i] = 0;
+    if (i < 4) count[i] = 0;
 }
 
-__global__ void __launch_bounds__(kSelBlock) k_sel_hist(const double* __restrict__ pt, const double* __restrict__ dist,
-                                                        int np, const unsigned long long* __restrict__ sel,
-                                                        int first, int shift, unsigned int* __restrict__ hist) {
-    __shared__ unsigned int h[256];
-    const int k = first + (int)blockIdx.y;
-    const unsigned long long prefix = sel[3 * k], mask = sel[3 * k + 1];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    for (int i = blockIdx.x * kSelBlock + threadIdx.x; i < np; i += gridDim.x * kSelBlock) {
-        const double x = k < 3 ? pt[4 * (int64_t)i + k] : dist[i];
-        const unsigned long long key = order_key(x);
-        if ((key & mask) == prefix) atomicAdd(&h[(key >> shift) & 255], 1u);
+// The bin of counts h (kSelBins of them) that holds rank *r, by a block of 256 threads: its number is
+// returned in every thread and *r becomes the rank inside it.
+__device__ __forceinline__ unsigned int sel_pick(const unsigned int* __restrict__ h, unsigned long long* r) {
+    constexpr int per = kSelBins / 256;
+    __shared__ unsigned long long wsum[4], rank_in;
+    __shared__ unsigned int digit;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    unsigned int v[per];
+    unsigned long long x = 0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+        v[i] = h[per * t + i];
+        x += v[i];
     }
-    __syncthreads();
-    // integer counts: the sum does not depend on the order the blocks add in
-    if (h[threadIdx.x]) atomicAdd(&hist[256 * k + threadIdx.x], h[threadIdx.x]);
-}
-
-// digit counts scanned; the thread whose bin holds the rank records it, and the counts are cleared
-// for the next pass
-__global__ void __launch_bounds__(256) k_sel_pick(unsigned long long* __restrict__ sel, unsigned int* __restrict__ hist,
-                                                  int first, int shift) {
-    __shared__ unsigned int wsum[4];
-    const int k = first + (int)blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const unsigned int tot = hist[256 * k + t];
-    hist[256 * k + t] = 0;
-    unsigned int x = tot;
+    const unsigned long long own = x;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const unsigned int y = __shfl_up(x, d, 64);
+        const unsigned long long y = __shfl_up(x, d, 64);
         if (lane >= d) x += y;
     }
+    __syncthreads();  // the shared words of an earlier pick have been read
     if (lane == 63) wsum[wave] = x;
     __syncthreads();
-    unsigned int off = 0;
-    for (int w = 0; w < wave; ++w) off += wsum[w];
-    const unsigned long long incl = off + x, excl = incl - tot;
-    const unsigned long long r = sel[3 * k + 2];
-    __syncthreads();  // every thread has read the rank before it is replaced
-    if (excl <= r && r < incl) {
-        sel[3 * k] |= (unsigned long long)t << shift;
-        sel[3 * k + 1] |= 255ull << shift;
-        sel[3 * k + 2] = r - excl;
+    unsigned long long excl = x - own;
+    for (int w = 0; w < wave; ++w) excl += wsum[w];
+    if (excl <= *r && *r < excl + own) {
+        unsigned long long left = *r - excl;
+        int i = 0;
+        while (i + 1 < per && left >= v[i]) left -= v[i++];
+        digit = per * t + i;
+        rank_in = left;
+    }
+    __syncthreads();
+    *r = rank_in;
+    return digit;
+}
+
+// BALProblem.cpp:274-281: L1 distance of a point to the per-axis medians
+__device__ __forceinline__ double norm_dist(const double* __restrict__ p, const double m[3]) {
+    return fabs(p[0] - m[0]) + fabs(p[1] - m[1]) + fabs(p[2] - m[2]);
+}
+
+// Pass 0 or 1 of selections first .. first + gridDim.y - 1, or (PASS 2) the collection of the keys that
+// share both digits.  sel[k] receives the selection's key so far and its rank among the collected ones.
+// Selection 3 forms the distances from the points and the medians in sel[0..2].
+template <int PASS>
+__global__ void __launch_bounds__(kSelBlock) k_sel_pass(const double* __restrict__ pt, int np, int first,
+                                                        unsigned long long* __restrict__ sel, unsigned int* __restrict__ hist,
+                                                        unsigned int* __restrict__ count, unsigned long long* __restrict__ keys) {
+    __shared__ unsigned int h[PASS < 2 ? kSelBins : 1];
+    const int k = first + (int)blockIdx.y, t = threadIdx.x;
+    unsigned int* hk = hist + 2 * kSelBins * k;
+    double m[3] = {0.0, 0.0, 0.0};
+    if (k == 3)
+        for (int j = 0; j < 3; ++j) m[j] = key_value(sel[2 * j]);
+    unsigned long long rank = (unsigned long long)(np / 2), prefix = 0;
+    if (PASS < 2)
+        for (int i = t; i < kSelBins; i += kSelBlock) h[i] = 0;
+    if (PASS >= 1) prefix = (unsigned long long)sel_pick(hk, &rank) << kSelShift0;
+    if (PASS >= 2) prefix |= (unsigned long long)sel_pick(hk + kSelBins, &rank) << kSelShift1;
+    __syncthreads();
+    if (PASS == 2 && blockIdx.x == 0 && t == 0) {
+        sel[2 * k] = prefix;
+        sel[2 * k + 1] = rank;
+    }
+    const int shift = PASS == 0 ? kSelShift0 : kSelShift1;
+    for (int i = blockIdx.x * kSelBlock + t; i < np; i += gridDim.x * kSelBlock) {
+        const double* p = pt + 4 * (int64_t)i;
+        const unsigned long long key = order_key(k < 3 ? p[k] : norm_dist(p, m));
+        if (PASS == 0) {
+            atomicAdd(&h[key >> kSelShift0], 1u);
+        } else if (PASS == 1) {
+            if ((key >> kSelShift0) == (prefix >> kSelShift0)) atomicAdd(&h[(key >> shift) & (kSelBins - 1)], 1u);
+        } else if ((key >> kSelShift1) == (prefix >> kSelShift1)) {
+            keys[(size_t)(k % 3) * np + atomicAdd(&count[k], 1u)] = key;
+        }
+    }
+    if (PASS < 2) {
+        __syncthreads();
+        // integer counts: the sum does not depend on the order the blocks add in
+        for (int i = t; i < kSelBins; i += kSelBlock)
+            if (h[i]) atomicAdd(&hk[PASS * kSelBins + i], h[i]);
     }
 }
 
-// BALProblem.cpp:274-281: L1 distance of each point to the per-axis medians
-__global__ void k_norm_dist(const double* __restrict__ pt, int np, const unsigned long long* __restrict__ sel,
-                            double* __restrict__ dist) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    const double* p = pt + 4 * (int64_t)i;
-    dist[i] = fabs(p[0] - key_value(sel[0])) + fabs(p[1] - key_value(sel[3])) + fabs(p[2] - key_value(sel[6]));
+// The remaining bits over the collected keys, one block per selection; their order does not matter.
+__global__ void __launch_bounds__(256) k_sel_finish(int np, int first, unsigned long long* __restrict__ sel,
+                                                    const unsigned int* __restrict__ count,
+                                                    const unsigned long long* __restrict__ keys) {
+    __shared__ unsigned int h[kSelBins];
+    const int k = first + (int)blockIdx.x, t = threadIdx.x;
+    const unsigned int n = count[k];
+    const unsigned long long* mine = keys + (size_t)(k % 3) * np;
+    unsigned long long prefix = sel[2 * k], rank = sel[2 * k + 1];
+    for (int top = kSelShift1; top > 0; top -= kSelBits) {  // bits [shift, top) of the keys
+        const int shift = top > kSelBits ? top - kSelBits : 0;
+        for (int i = t; i < kSelBins; i += 256) h[i] = 0;
+        __syncthreads();
+        for (unsigned int i = t; i < n; i += 256) {
+            const unsigned long long key = mine[i];
+            if ((key >> top) == (prefix >> top)) atomicAdd(&h[(key >> shift) & ((1ull << (top - shift)) - 1)], 1u);
+        }
+        __syncthreads();
+        prefix |= (unsigned long long)sel_pick(h, &rank) << shift;
+        __syncthreads();
+    }
+    if (t == 0) sel[2 * k] = prefix;
 }
 
 // BALProblem.cpp:283-302: X <- s (X - m), camera centres likewise, s = 100 / MAD
 __global__ void k_norm_apply(double* __restrict__ pt, int np, double* __restrict__ cam, int nc,
                              const unsigned long long* __restrict__ sel) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const double m[3] = {key_value(sel[0]), key_value(sel[3]), key_value(sel[6])};
-    const double scale = 100.0 / key_value(sel[9]);
+    const double m[3] = {key_value(sel[0]), key_value(sel[2]), key_value(sel[4])};
+    const double scale = 100.0 / key_value(sel[6]);
     if (i < np)
         for (int j = 0; j < 3; ++j) pt[4 * (int64_t)i + j] = scale * (pt[4 * (int64_t)i + j] - m[j]);
     if (i < nc) {
@@ -391,28 +483,28 @@ int ensure(DevBuf<T>& b, size_t n) {
 
 }  // namespace
 
-int draw_normals(int64_t n_normals, uint32_t seed, PrepScratch* w, hipStream_t s);
+int64_t first_pairs(int64_t n_normals);
+int draw_normals(int64_t n_normals, int64_t n_pairs, uint32_t seed, PrepScratch* w, hipStream_t s);
 
 int device_normalize(const DeviceParams& p, PrepScratch* w, hipStream_t s) {
     if (p.np == 0) return BA_OK;  // BALProblem.cpp:263-303 leaves an empty problem as it is
     const int np = p.np;
     const int nblocks = std::max(1, std::min(256, div_up(np, kSelBlock * 8)));
-    BA_TRY(ensure(w->sel_state, 12));
-    BA_TRY(ensure(w->hist, (size_t)4 * 256));
-    BA_TRY(ensure(w->dist, (size_t)np));
-    hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, s, w->sel_state.p, (unsigned long long)(np / 2), w->hist.p);
-    for (int pass = 0; pass < 8; ++pass) {
-        const int shift = 56 - 8 * pass;
-        hipLaunchKernelGGL(k_sel_hist, dim3(nblocks, 3), dim3(kSelBlock), 0, s, p.pt, w->dist.p, np, w->sel_state.p, 0,
-                           shift, w->hist.p);
-        hipLaunchKernelGGL(k_sel_pick, dim3(3), dim3(256), 0, s, w->sel_state.p, w->hist.p, 0, shift);
-    }
-    hipLaunchKernelGGL(k_norm_dist, dim3(div_up(np, 256)), dim3(256), 0, s, p.pt, np, w->sel_state.p, w->dist.p);
-    for (int pass = 0; pass < 8; ++pass) {
-        const int shift = 56 - 8 * pass;
-        hipLaunchKernelGGL(k_sel_hist, dim3(nblocks, 1), dim3(kSelBlock), 0, s, p.pt, w->dist.p, np, w->sel_state.p, 3,
-                           shift, w->hist.p);
-        hipLaunchKernelGGL(k_sel_pick, dim3(1), dim3(256), 0, s, w->sel_state.p, w->hist.p, 3, shift);
+    BA_TRY(ensure(w->sel_state, 8));
+    BA_TRY(ensure(w->hist, (size_t)4 * 2 * kSelBins + 4));
+    BA_TRY(ensure(w->keys, 3 * (size_t)np));
+    unsigned int* count = w->hist.p + 4 * 2 * kSelBins;
+    hipLaunchKernelGGL(k_sel_init, dim3(4 * 2 * kSelBins / 256), dim3(256), 0, s, w->hist.p, count);
+    for (int first : {0, 3}) {  // the axes together, then the distances to their medians
+        const int n = first == 0 ? 3 : 1;
+        hipLaunchKernelGGL(k_sel_pass<0>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
+                           count, w->keys.p);
+        hipLaunchKernelGGL(k_sel_pass<1>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
+                           count, w->keys.p);
+        hipLaunchKernelGGL(k_sel_pass<2>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
+                           count, w->keys.p);
+        hipLaunchKernelGGL(k_sel_finish, dim3(n), dim3(256), 0, s, np, first, w->sel_state.p, (const unsigned int*)count,
+                           (const unsigned long long*)w->keys.p);
     }
     hipLaunchKernelGGL(k_norm_apply, dim3(div_up(std::max(np, p.nc), 256)), dim3(256), 0, s, p.pt, np, p.cam, p.nc,
                        w->sel_state.p);
@@ -426,51 +518,55 @@ int device_perturb(const DeviceParams& p, uint32_t seed, double rs, double ts, d
     const int64_t n_normals = n_pt + (int64_t)p.nc * ((rs > 0.0 ? 3 : 0) + (ts > 0.0 ? 3 : 0));
     if (n_normals > (int64_t)1 << 30) return fail(BA_ERR_CAPACITY, "perturbation needs %lld normals (limit 2^30)",
                                                    (long long)n_normals);
-    if (n_normals > 0) BA_TRY(draw_normals(n_normals, seed, w, s));
-    if (ps > 0.0 && p.np > 0)
-        hipLaunchKernelGGL(k_perturb_points, dim3(div_up(p.np, 256)), dim3(256), 0, s, p.pt, p.pt_orig, p.np,
-                           (const double*)w->normals.p, ps);
-    // every camera goes through centre and back, as in the reference, also with both sigmas 0
-    if (p.nc > 0)
-        hipLaunchKernelGGL(k_perturb_cams, dim3(div_up(p.nc, 64)), dim3(64), 0, s, p.cam, p.nc,
-                           (const double*)w->normals.p, n_pt, rs, ts);
-    BA_HIP(hipGetLastError());
-    return BA_OK;
+    int64_t n_pairs = first_pairs(n_normals);
+    BA_TRY(ensure(w->total, 1));
+    for (;;) {
+        if (n_normals > 0) BA_TRY(draw_normals(n_normals, n_pairs, seed, w, s));
+        if (ps > 0.0 && p.np > 0)
+            hipLaunchKernelGGL(k_perturb_points, dim3(div_up(p.np, 256)), dim3(256), 0, s, p.pt, p.pt_orig, p.np,
+                               (const double*)w->normals.p, ps, (const int*)w->total.p, (int)n_normals);
+        // every camera goes through centre and back, as in the reference, also with both sigmas 0
+        if (p.nc > 0)
+            hipLaunchKernelGGL(k_perturb_cams, dim3(div_up(p.nc, 64)), dim3(64), 0, s, p.cam, p.nc,
+                               (const double*)w->normals.p, n_pt, rs, ts, (const int*)w->total.p, (int)n_normals);
+        BA_HIP(hipGetLastError());
+        if (n_normals == 0) return BA_OK;
+        int got = 0;
+        BA_HIP(hipMemcpyAsync(&got, w->total.p, sizeof(int), hipMemcpyDeviceToHost, s));
+        BA_HIP(hipStreamSynchronize(s));
+        if (got >= n_normals) return BA_OK;
+        n_pairs += n_pairs / 2;
+    }
 }
 
-// normals 0..n_normals-1 of the stream glibc's rand() gives after srand(seed), into w->normals
-int draw_normals(int64_t n_normals, uint32_t seed, PrepScratch* w, hipStream_t s) {
+// Pairs to draw for n normals: the acceptance rate is pi/4, so 1.3 per normal leaves a margin of many
+// standard deviations; a shortfall (read back by the caller) draws again with more.
+int64_t first_pairs(int64_t n_normals) { return n_normals + n_normals * 3 / 10 + 4096; }
+
+// Normals 0..n_normals-1 of the stream glibc's rand() gives after srand(seed), from n_pairs pairs of draws,
+// into w->normals; the number of accepted pairs into w->total.
+int draw_normals(int64_t n_normals, int64_t n_pairs, uint32_t seed, PrepScratch* w, hipStream_t s) {
     const std::vector<uint32_t>& tables = jump_tables();
     if (!w->table_chunks) {
         BA_TRY(w->tables.upload(tables.data(), tables.size(), s));
         w->table_chunks = 1;
     }
     const RandState start = glibc_seed_state(seed);
-    // pairs to draw: the acceptance rate is pi/4, so 1.3 per normal leaves a margin of many
-    // standard deviations; a shortfall (read back below) draws again with more
-    int64_t n_pairs = n_normals + n_normals * 3 / 10 + 4096;
+    const int64_t n_draws = 2 * n_pairs;
+    const int n_chunks = div_up(n_draws, kChunk);
+    if (n_chunks >= (1 << kJumps)) return fail(BA_ERR_CAPACITY, "random stream too long");
+    const int nb = div_up(n_pairs, kPairsPerBlock);
     BA_TRY(ensure(w->total, 1));
-    for (;;) {
-        const int64_t n_draws = 2 * n_pairs;
-        const int n_chunks = div_up(n_draws, kChunk);
-        if (n_chunks >= (1 << kJumps)) return fail(BA_ERR_CAPACITY, "random stream too long");
-        const int nb = div_up(n_pairs, kPairsPerBlock);
-        BA_TRY(ensure(w->draws, (size_t)n_draws));
-        BA_TRY(ensure(w->counts, (size_t)nb));
-        BA_TRY(ensure(w->normals, (size_t)n_normals));
-        hipLaunchKernelGGL(k_rand_generate, dim3(div_up(n_chunks, 64)), dim3(64), 0, s, start, w->tables.p, n_chunks,
-                           n_draws, w->draws.p);
-        hipLaunchKernelGGL(k_pairs_count, dim3(nb), dim3(kPairBlock), 0, s, w->draws.p, n_pairs, (int*)w->counts.p);
-        hipLaunchKernelGGL(k_pairs_scan, dim3(1), dim3(kPairBlock), 0, s, (int*)w->counts.p, nb, w->total.p);
-        hipLaunchKernelGGL(k_pairs_emit, dim3(nb), dim3(kPairBlock), 0, s, w->draws.p, n_pairs,
-                           (const int*)w->counts.p, (int)n_normals, w->normals.p);
-        BA_HIP(hipGetLastError());
-        int got = 0;
-        BA_HIP(hipMemcpyAsync(&got, w->total.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        BA_HIP(hipStreamSynchronize(s));
-        if (got >= n_normals) break;
-        n_pairs = n_pairs + n_pairs / 2;
-    }
+    BA_TRY(ensure(w->draws, (size_t)n_draws));
+    BA_TRY(ensure(w->counts, (size_t)nb));
+    BA_TRY(ensure(w->normals, (size_t)n_normals));
+    hipLaunchKernelGGL(k_rand_generate, dim3(div_up(n_chunks, kBlockChunks)), dim3(256), 0, s, start, w->tables.p, n_draws,
+                       w->draws.p);
+    hipLaunchKernelGGL(k_pairs_count, dim3(nb), dim3(kPairBlock), 0, s, w->draws.p, n_pairs, (int*)w->counts.p);
+    hipLaunchKernelGGL(k_pairs_scan, dim3(1), dim3(kPairBlock), 0, s, (int*)w->counts.p, nb, w->total.p);
+    hipLaunchKernelGGL(k_pairs_emit, dim3(nb), dim3(kPairBlock), 0, s, w->draws.p, n_pairs, (const int*)w->counts.p,
+                       (int)n_normals, w->normals.p);
+    BA_HIP(hipGetLastError());
     return BA_OK;
 }
 
