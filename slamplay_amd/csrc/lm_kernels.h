@@ -132,7 +132,7 @@ struct Dev {
     Real* VinvR;               // per point: 6 (same, in working precision)
     R4<Real>* qp;              // per point: Vinv S g_p
     double4* zs;               // per point: S_p z_p of the current PCG direction (FP64 in both precisions)
-    double4* pv;               // per slot, 3 records: J_p'J_p (sym 6), J_p'r (3), padding
+    R4<Real>* pv;              // per slot, 2 records: J_p row 0 and r_0, J_p row 1 and r_1
     R4<Real>* u;               // per slot: J_p'(J_c S_c v_c)
     double* cam_part;          // PS_COUNT * nc
     double* pt_part;           // PS_COUNT * n_pt_blocks
@@ -465,8 +465,10 @@ __global__ void __launch_bounds__(64) k_cam_prep(Dev<Real> d) {
 }
 
 // One workgroup per camera: diag(Jc'Jc) and g_c = Jc'r (unscaled, corrected) -- the column norms
-// for the Jacobi scaling and the LM diagonal -- plus each observation's point contributions
-// Jp'Jp and Jp'r for k_lin_pt.
+// for the Jacobi scaling and the LM diagonal -- plus each observation's Jp and r for k_lin_pt, in working
+// precision: 32 scattered bytes of an observation in mixed precision (64 in FP64) instead of the 96 of its
+// nine products, which the reader forms.  At 1500 cameras and 1.2 M observations, with k_lin_pt: 27 + 17 us
+// mixed (50 + 61 with the products stored), 43 + 41 FP64 (58 + 70); the scattered writes bound it.
 template <typename Real, int M>
 __global__ void __launch_bounds__(kWG) k_lin_cam(Dev<Real> d) {
     if (!d.st->need_lin) return;
@@ -497,17 +499,9 @@ __global__ void __launch_bounds__(kWG) k_lin_cam(Dev<Real> d) {
             acc[i] += (double)(Jc[i] * Jc[i] + Jc[9 + i] * Jc[9 + i]);
             acc[9 + i] += (double)(Jc[i] * r[0] + Jc[9 + i] * r[1]);
         }
-        // The point block's per-observation products are formed in FP64 from the (FP32 or FP64)
-        // Jacobian: products of FP32 values are exact in FP64, so each contribution is exactly
-        // positive semidefinite and V stays positive definite for nearly depth-free points.
-        const double q[6] = {Jp[0], Jp[1], Jp[2], Jp[3], Jp[4], Jp[5]};
-        const double r0 = r[0], r1 = r[1];
-        double4* pv = d.pv + 3 * (size_t)d.slot_of[j];
-        pv[0] = make_double4(q[0] * q[0] + q[3] * q[3], q[0] * q[1] + q[3] * q[4], q[0] * q[2] + q[3] * q[5],
-                             q[1] * q[1] + q[4] * q[4]);
-        pv[1] = make_double4(q[1] * q[2] + q[4] * q[5], q[2] * q[2] + q[5] * q[5], q[0] * r0 + q[3] * r1,
-                             q[1] * r0 + q[4] * r1);
-        pv[2] = make_double4(q[2] * r0 + q[5] * r1, 0.0, 0.0, 0.0);
+        R4<Real>* pv = d.pv + 2 * (size_t)d.slot_of[j];
+        pv[0] = R4<Real>{Jp[0], Jp[1], Jp[2], r[0]};
+        pv[1] = R4<Real>{Jp[3], Jp[4], Jp[5], r[1]};
     }
     block_sum<18>(acc, lds);
     const int t = threadIdx.x;
@@ -582,7 +576,9 @@ __device__ __forceinline__ void chunk_sum_r4(int len, size_t base, const R4<Real
             for (int w = 0; w < kWaves - 1; ++w) acc[i] += lds[(w * 3 + i) * 64 + lane];
 }
 
-// One workgroup per chunk: V_p = sum Jp'Jp, g_p = sum Jp'r per point.
+// One workgroup per chunk: V_p = sum Jp'Jp, g_p = sum Jp'r per point.  The per-observation products are
+// formed in FP64 from the (FP32 or FP64) Jacobian: products of FP32 values are exact in FP64, so each
+// contribution is exactly positive semidefinite and V stays positive definite for nearly depth-free points.
 template <typename Real>
 __global__ void __launch_bounds__(kWG) k_lin_pt(Dev<Real> d) {
     if (!d.st->need_lin) return;
@@ -592,17 +588,19 @@ __global__ void __launch_bounds__(kWG) k_lin_pt(Dev<Real> d) {
     double a[9];
     chunk_sum<9>(d.chunk_len[ch], (size_t)d.chunk_off[ch], a,
                  [&](size_t slot, double (&acc)[9]) {
-                     const double4* pv = d.pv + 3 * slot;
-                     const double4 x = pv[0], y = pv[1], z = pv[2];
-                     acc[0] += x.x;
-                     acc[1] += x.y;
-                     acc[2] += x.z;
-                     acc[3] += x.w;
-                     acc[4] += y.x;
-                     acc[5] += y.y;
-                     acc[6] += y.z;
-                     acc[7] += y.w;
-                     acc[8] += z.x;
+#pragma clang fp contract(off)  // each contribution is rounded by itself before it is added
+                     const R4<Real> x = d.pv[2 * slot], y = d.pv[2 * slot + 1];
+                     const double q[3] = {(double)x.x, (double)x.y, (double)x.z}, r0 = (double)x.w;
+                     const double s[3] = {(double)y.x, (double)y.y, (double)y.z}, r1 = (double)y.w;
+                     acc[0] += fma(q[0], q[0], s[0] * s[0]);
+                     acc[1] += fma(q[0], q[1], s[0] * s[1]);
+                     acc[2] += fma(q[0], q[2], s[0] * s[2]);
+                     acc[3] += fma(q[1], q[1], s[1] * s[1]);
+                     acc[4] += fma(q[1], q[2], s[1] * s[2]);
+                     acc[5] += fma(q[2], q[2], s[2] * s[2]);
+                     acc[6] += fma(q[0], r0, s[0] * r1);
+                     acc[7] += fma(q[1], r0, s[1] * r1);
+                     acc[8] += fma(q[2], r0, s[2] * r1);
                  },
                  lds);
     if (threadIdx.x >= 64) return;

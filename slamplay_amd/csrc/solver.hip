@@ -257,7 +257,7 @@ struct Solver final : SolverBase {
     DevBuf<Real> VinvR;
     DevBuf<R4<Real>> qp, u;
     DevBuf<double4> zs;
-    DevBuf<double4> pv;
+    DevBuf<R4<Real>> pv;
     DevBuf<double> cam_part, pt_part;
     DevBuf<LMState> st;
     DevBuf<ba_iteration> trace;
@@ -366,7 +366,7 @@ struct Solver final : SolverBase {
         BA_TRY(co_rec.alloc((size_t)std::max(no, 1)));
         // slot-order buffers: padding slots are never written and must read as zero
         const size_t nslots = (size_t)std::max(L.chunk_off[L.n_chunks], 1);
-        BA_TRY(pv.alloc(3 * nslots));
+        BA_TRY(pv.alloc(2 * nslots));
         BA_TRY(u.alloc(nslots));
         BA_HIP(hipMemsetAsync(pv.p, 0, pv.bytes(), s));
         BA_HIP(hipMemsetAsync(u.p, 0, u.bytes(), s));
