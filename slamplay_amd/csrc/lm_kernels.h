@@ -241,12 +241,66 @@ __device__ __forceinline__ T wave_sum(T v) {
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
-// Sum over each half-wave of 32 lanes (lanes 0-31 and 32-63 reduced separately).
-template <typename T>
-__device__ __forceinline__ T half_wave_sum(T v) {
-    v = row16_sum(v);
-    const T a = read_lane(v, 0) + read_lane(v, 16), b = read_lane(v, 32) + read_lane(v, 48);
-    return (threadIdx.x & 32) ? b : a;
+// Sums of several values at once, each lane left with the total of one: level b of a fold pairs the values,
+// lanes with bit b clear go on with the first, lanes with it set with the second, and each adds its
+// partner lane's part, so a level halves the values as it halves the terms.  Seven instructions a pair
+// and level, three at the last two, against 23 (eight of them v_readlane) a value for wave_sum: the 54
+// sums of k_rhs_cam were 14 of its 51 us at 1500 cameras, the 16 of k_jz_dir 2 of its 15.  The terms are
+// added in wave_sum's order: the totals are the same bits.  Every lane of the wave must be active.
+constexpr int kDppShl4 = 0x104, kDppShr4 = 0x114, kDppShl8 = 0x108, kDppShr8 = 0x118;  // lane + n, lane - n
+
+// Partner lane's a in lanes with bit BIT clear, its b in the others (BIT < 4).
+template <int BIT>
+__device__ __forceinline__ int fold_other(int a, int b, bool set) {
+    if constexpr (BIT < 2) {
+        return __builtin_amdgcn_update_dpp(0, set ? a : b, BIT == 0 ? kDppXor1 : kDppXor2, 0xF, 0xF, true);
+    } else {
+        constexpr int up = BIT == 2 ? kDppShl4 : kDppShl8, down = BIT == 2 ? kDppShr4 : kDppShr8;
+        const int low = __builtin_amdgcn_update_dpp(0, a, up, 0xF, 0xF, true);
+        return __builtin_amdgcn_update_dpp(low, b, down, 0xF, BIT == 2 ? 0xA : 0xC, false);
+    }
+}
+
+// Lanes with bit BIT clear: a's sum with the partner lane's; with it set: b's.
+template <int BIT>
+__device__ __forceinline__ double fold_pair(double a, double b) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    int lo, hi;
+    double keep;
+    if constexpr (BIT < 4) {
+        const bool set = threadIdx.x & (1 << BIT);
+        // BIT < 2 sends what the partner keeps: its first value to a lane with the bit clear
+        if constexpr (BIT < 2) {
+            lo = fold_other<BIT>((int)x, (int)y, set);
+            hi = fold_other<BIT>((int)(x >> 32), (int)(y >> 32), set);
+        } else {
+            lo = fold_other<BIT>((int)x, (int)y, false);
+            hi = fold_other<BIT>((int)(x >> 32), (int)(y >> 32), false);
+        }
+        keep = set ? b : a;
+        return keep + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    } else if constexpr (BIT == 4) {
+        const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        return __longlong_as_double((long long)((unsigned long long)h[0] << 32 | l[0])) +
+               __longlong_as_double((long long)((unsigned long long)h[1] << 32 | l[1]));
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        return __longlong_as_double((long long)((unsigned long long)h[0] << 32 | l[0])) +
+               __longlong_as_double((long long)((unsigned long long)h[1] << 32 | l[1]));
+    }
+}
+
+// v[0 .. N) folded over the lane bits [0, BITS): on return slot i >> BITS of lanes with low bits
+// i & (2^BITS - 1) holds value i's sum over the 2^BITS lanes (BITS 4: rows of 16, 6: the wave).
+template <int N, int BITS, int BIT = 0>
+__device__ __forceinline__ void lane_fold(double (&v)[N]) {
+    constexpr int n = (N + (1 << BIT) - 1) >> BIT;  // slots at this level
+#pragma unroll
+    for (int i = 0; i < n / 2; ++i) v[i] = fold_pair<BIT>(v[2 * i], v[2 * i + 1]);
+    if constexpr (n & 1) v[n / 2] = fold_pair<BIT>(v[n - 1], v[n - 1]);
+    if constexpr (BIT + 1 < BITS) lane_fold<N, BITS, BIT + 1>(v);
 }
 
 template <typename T>
@@ -287,12 +341,14 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ a, int 
 // lds[i * NW] holds the total of value i for every thread (a barrier is included).
 template <int N, typename T, int NW = kWaves>
 __device__ __forceinline__ void block_sum(T (&v)[N], T* lds) {
+    static_assert(N <= 64, "one total per lane");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const T s = wave_sum(v[i]);
-        if (lane == 0) lds[i * NW + wave] = s;
+    if constexpr (N == 1) {
+        v[0] = wave_sum(v[0]);
+    } else {
+        lane_fold<N, 6>(v);
     }
+    if (lane < N) lds[lane * NW + wave] = v[0];
     __syncthreads();
     for (int i = threadIdx.x; i < N; i += 64 * NW) {
         T s = lds[i * NW];
@@ -468,7 +524,7 @@ __global__ void __launch_bounds__(64) k_cam_prep(Dev<Real> d) {
 // for the Jacobi scaling and the LM diagonal -- plus each observation's Jp and r for k_lin_pt, in working
 // precision: 32 scattered bytes of an observation in mixed precision (64 in FP64) instead of the 96 of its
 // nine products, which the reader forms.  At 1500 cameras and 1.2 M observations, with k_lin_pt: 27 + 17 us
-// mixed (50 + 61 with the products stored), 43 + 41 FP64 (58 + 70); the scattered writes bound it.
+// mixed (50 + 61 with the products stored), 43 + 41 FP64 (58 + 70), before its sums were folded; the scattered writes bound it.
 template <typename Real, int M>
 __global__ void __launch_bounds__(kWG) k_lin_cam(Dev<Real> d) {
     if (!d.st->need_lin) return;

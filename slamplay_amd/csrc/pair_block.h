@@ -199,18 +199,19 @@ __device__ __forceinline__ void pair_block(const int4 bk_all, const int2* __rest
         pr = pr_next;
         pr_next = pr_far;
     }
+    // the 27 sums over each row's 16 lanes: lane q of a row gets numbers q and q + 16
+    double sum[27];
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
+    for (int e = 0; e < 27; ++e) sum[e] = acc[e / 3][e % 3];
+    lane_fold<27, 4>(sum);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const double v = row16_sum(acc[r][k]);
-            const int c = c0 + k;
-            if (q == 0 && k < nc) {
-                if (NW == 1)
-                    pair_entry(bk, r, c, v, dc2, S, ld);
-                else
-                    sums[81 * wave + 9 * r + c] = v;
-            }
+    for (int u = 0; u < 2; ++u) {
+        const int e = q + 16 * u, r = e / 3, k = e - 3 * r, c = c0 + k;
+        if (e < 27 && k < nc) {
+            if (NW == 1)
+                pair_entry(bk, r, c, sum[u], dc2, S, ld);
+            else
+                sums[81 * wave + 9 * r + c] = sum[u];
         }
     }
     if (NW > 1) {
