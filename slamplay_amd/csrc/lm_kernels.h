@@ -378,6 +378,14 @@ __device__ __forceinline__ double block_max1(double v, double* lds) {
 // Index of (i, k), i <= k, in a packed upper triangle of a 9x9 matrix (45 entries).
 __host__ __device__ __forceinline__ constexpr int sym9(int i, int k) { return i * 9 - (i * (i - 1)) / 2 + (k - i); }
 
+// The row and the column of entry e of that triangle.
+__host__ __device__ __forceinline__ constexpr int sym9_row(int e) {
+    int r = 0;
+    while (e >= 9 - r) e -= 9 - r++;
+    return r;
+}
+__host__ __device__ __forceinline__ constexpr int sym9_col(int e) { return sym9_row(e) + e - sym9(sym9_row(e), sym9_row(e)); }
+
 // ---------------------------------------------------------------------------------------------
 // Small dense FP64 algebra (per-thread)
 

@@ -4,7 +4,7 @@
 // byte offsets of its arrays.  Within a window:
 //   * observations in camera order (cam_off, co_pt local point index, co_uv64);
 //   * points in SELL-64 chunks (chunk_off / chunk_len), slot_of[j] = slot of observation j; the
-//     slot records pv are three double4 arrays of n_slots entries (component-major);
+//     slot records pv are two double4 arrays of n_slots entries (component-major);
 //   * the 9x9 blocks (a <= b) of the reduced camera system with their observation pairs
 //     (i, j) (camera(i) = a, camera(j) = b, same point), built once on the host and listed with
 //     the largest pair count first;

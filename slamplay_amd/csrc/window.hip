@@ -151,7 +151,7 @@ int build_window_image(const ba_problem_view* v, const ba_options& opt, WindowIm
     D.o_Vinv = take(48 * (int64_t)P);
     D.o_qp = take(32 * (int64_t)P);
     D.o_yp = take(24 * (int64_t)P);
-    D.o_pv = take(96 * (int64_t)slots);
+    D.o_pv = take(64 * (int64_t)slots);
     D.o_js = take(kWinJs * sizeof(Real) * (int64_t)No);
     D.o_S = take(sizeof(double) * (int64_t)n * n);  // zero: blocks without common points are never written
     D.o_L = take(sizeof(double) * (int64_t)small_system_doubles(n));  // the factor when it is not kept in LDS

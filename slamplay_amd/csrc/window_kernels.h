@@ -126,24 +126,25 @@ __device__ __forceinline__ void win_model_residual(const WinPtrs& w, const Camer
         snavely_residual<double>(P, X, u, v, r);
 }
 
-// Sum of N per-thread values over a workgroup of NT threads in a fixed order (wave butterflies,
-// then the waves in order by thread 0); the totals are returned to thread 0 only.
+// Sums of N per-thread values over a workgroup of NT threads in a fixed order (within each wave, then
+// the waves in order): thread t < N returns total t, the others zero.
 template <int N, int NT>
-__device__ __forceinline__ void wg_sum_fixed(double (&v)[N], double* lds) {
+__device__ __forceinline__ double wg_sums(double (&v)[N], double* lds) {
     constexpr int NW = NT / 64;
+    static_assert(N <= 64, "one total per lane");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const double s = wave_sum(v[i]);
-        if (lane == 0) lds[i * NW + wave] = s;
-    }
+    if constexpr (N == 1)
+        v[0] = wave_sum(v[0]);
+    else
+        lane_fold<N, 6>(v);
+    if (lane < N) lds[lane * NW + wave] = v[0];
     __syncthreads();
-    if (threadIdx.x == 0)
-        for (int i = 0; i < N; ++i) {
-            double s = lds[i * NW];
-            for (int k = 1; k < NW; ++k) s += lds[i * NW + k];
-            v[i] = s;
-        }
+    double s = 0.0;
+    if (threadIdx.x < N) {
+        s = lds[threadIdx.x * NW];
+        for (int k = 1; k < NW; ++k) s += lds[threadIdx.x * NW + k];
+    }
+    return s;
 }
 
 // Huber-corrected FP64 residual and Jacobians of observation j (point p) at the current parameters
@@ -182,7 +183,8 @@ __device__ __forceinline__ void win_scaled(const WinPtrs& w, const CameraPrep<do
     }
 }
 
-// Slot records: pv holds three double4 arrays of n_slots entries each (component-major).
+// Slot records: pv holds two double4 arrays of n_slots entries each (component-major): row 0 of J_p and r_0, row
+// 1 and r_1; after the linearization the first one's entries are the back-substitution's vectors.
 __device__ __forceinline__ double4& pv_at(const WinPtrs& w, int k, int slot) {
     return w.pv[(size_t)k * w.n_slots + slot];
 }
@@ -281,22 +283,17 @@ __global__ void __launch_bounds__(NT) k_wlin_cam(const WinDesc* __restrict__ des
             acc[9 + i] += Jc[i] * r[0] + Jc[9 + i] * r[1];
         }
         const int slot = w.slot_of[j];
-        pv_at(w, 0, slot) = make_double4(Jp[0] * Jp[0] + Jp[3] * Jp[3], Jp[0] * Jp[1] + Jp[3] * Jp[4],
-                                         Jp[0] * Jp[2] + Jp[3] * Jp[5], Jp[1] * Jp[1] + Jp[4] * Jp[4]);
-        pv_at(w, 1, slot) = make_double4(Jp[1] * Jp[2] + Jp[4] * Jp[5], Jp[2] * Jp[2] + Jp[5] * Jp[5],
-                                         Jp[0] * r[0] + Jp[3] * r[1], Jp[1] * r[0] + Jp[4] * r[1]);
-        pv_at(w, 2, slot) = make_double4(Jp[2] * r[0] + Jp[5] * r[1], 0.0, 0.0, 0.0);
+        pv_at(w, 0, slot) = make_double4(Jp[0], Jp[1], Jp[2], r[0]);
+        pv_at(w, 1, slot) = make_double4(Jp[3], Jp[4], Jp[5], r[1]);
     }
-    wg_sum_fixed<19, NT>(acc, lds);
-    if (threadIdx.x == 0) {
-        double gm = 0.0;
-        for (int i = 0; i < 9; ++i) {
-            w.udiag[9 * (size_t)c + i] = acc[i];
-            w.gc[9 * (size_t)c + i] = acc[9 + i];
-            gm = fmax(gm, fabs(acc[9 + i]));
-        }
-        w.cpart[WC_COUNT * (size_t)c + WC_GMAX] = gm;
-        w.cpart[WC_COUNT * (size_t)c + WC_COST] = acc[18];
+    const double total = wg_sums<19, NT>(acc, lds);
+    if (threadIdx.x < 64) {
+        const int i = threadIdx.x;
+        if (i < 9) w.udiag[9 * (size_t)c + i] = total;
+        if (i >= 9 && i < 18) w.gc[9 * (size_t)c + i - 9] = total;
+        const double gm = wave_max(i >= 9 && i < 18 ? fmax(0.0, fabs(total)) : 0.0);
+        if (i == 0) w.cpart[WC_COUNT * (size_t)c + WC_GMAX] = gm;
+        if (i == 18) w.cpart[WC_COUNT * (size_t)c + WC_COST] = total;
     }
 }
 
@@ -316,20 +313,27 @@ __global__ void __launch_bounds__(64) k_wlin_pt(const WinDesc* __restrict__ desc
         const int len = w.chunk_len[ch], base = w.chunk_off[ch];
         double a[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
         for (int r0 = 0; r0 < len; r0 += 4) {  // four rows' loads in flight, summed in row order
-            double4 x[4], y[4], z[4];
+            double4 x[4], y[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int slot = base + 64 * min(r0 + i, len - 1) + l;
                 x[i] = pv_at(w, 0, slot);
                 y[i] = pv_at(w, 1, slot);
-                z[i] = pv_at(w, 2, slot);
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (r0 + i < len) {
-                    a[0] += x[i].x; a[1] += x[i].y; a[2] += x[i].z; a[3] += x[i].w;
-                    a[4] += y[i].x; a[5] += y[i].y; a[6] += y[i].z; a[7] += y[i].w;
-                    a[8] += z[i].x;
+#pragma clang fp contract(off)  // an observation's term is rounded by itself before it is added
+                    const double4 q = x[i], s = y[i];
+                    a[0] += fma(q.x, q.x, s.x * s.x);
+                    a[1] += fma(q.x, q.y, s.x * s.y);
+                    a[2] += fma(q.x, q.z, s.x * s.z);
+                    a[3] += fma(q.y, q.y, s.y * s.y);
+                    a[4] += fma(q.y, q.z, s.y * s.z);
+                    a[5] += fma(q.z, q.z, s.z * s.z);
+                    a[6] += fma(q.x, q.w, s.x * s.w);
+                    a[7] += fma(q.y, q.w, s.y * s.w);
+                    a[8] += fma(q.z, q.w, s.z * s.w);
                 }
         }
         for (int i = 0; i < 6; ++i) w.V[6 * (size_t)p + i] = a[i];
@@ -437,7 +441,6 @@ __global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ des
     constexpr int NW = NT / 64;
     __shared__ double lds[9 * NW];
     __shared__ double dacc[NW][45];  // per wave: upper triangle of sum J~_c'(I - G)J~_c
-    __shared__ double red[NW][16][45];  // per wave: one round's terms summed over lane quads
     __shared__ CameraPrep<double> Psh;
     __shared__ StereoRig Gsh;
     const int t = blockIdx.x;
@@ -459,9 +462,9 @@ __global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ des
     double bacc[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) bacc[i] = 0.0;
-    for (int k = threadIdx.x; k < NW * 45; k += NT) (&dacc[0][0])[k] = 0.0;
+    double dsum = 0.0;  // lane e < 45: the wave's sum of term e
     __syncthreads();
-    // rounds of NT observations, every lane taking part in the per-round butterflies
+    // rounds of NT observations, every lane taking part in the per-round sums
     for (int j0r = j_beg; j0r < j_end; j0r += NT) {
         const int j = j0r + threadIdx.x;
         const int p = pn;
@@ -507,40 +510,35 @@ __global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ des
             t0[i] = g00 * Jd[i] + g01 * Jd[9 + i];
             t1[i] = g01 * Jd[i] + g11 * Jd[9 + i];
         }
-        // the 45 terms summed over lane quads by two DPP steps, the 16 quad sums of each term then
-        // added in order by lane e (an LDS transpose instead of 45 full-wave butterflies)
+        // the 45 terms, folded over rows of 16 lanes sixteen at a time (all at once they would take 90
+        // registers), then over the wave
+        double term[45], part[3][16];
         int e = 0;
 #pragma unroll
         for (int r = 0; r < 9; ++r)
 #pragma unroll
             for (int cc = r; cc < 9; ++cc, ++e) {
-                double v = Jd[r] * t0[cc] + Jd[9 + r] * t1[cc];
-                v += dpp_lane<kDppXor1>(v);
-                v += dpp_lane<kDppXor2>(v);
-                if ((lane & 3) == 0) red[wave][lane >> 2][e] = v;
+                part[e / 16][e % 16] = Jd[r] * t0[cc] + Jd[9 + r] * t1[cc];
+                if (e % 16 == 15) {
+                    lane_fold<16, 4>(part[e / 16]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
-        wave_sync_lds();
-        if (lane < 45) {
-            double v = red[wave][0][lane];
 #pragma unroll
-            for (int m = 1; m < 16; ++m) v += red[wave][m][lane];
-            dacc[wave][lane] += v;
-        }
-        wave_sync_lds();
+        for (int i = 13; i < 16; ++i) part[2][i] = 0.0;
+        lane_fold<16, 4>(part[2]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) term[i] = part[i][0];
+        lane_fold<45, 6, 4>(term);
+        dsum += term[0];
     }
-    wg_sum_fixed<9, NT>(bacc, lds);
-    if (threadIdx.x == 0)
-        for (int i = 0; i < 9; ++i) w.bc[9 * (size_t)c + i] = bacc[i];
+    if (lane < 45) dacc[wave][lane] = dsum;
+    const double b = wg_sums<9, NT>(bacc, lds);  // (its barrier covers dacc)
+    if (threadIdx.x < 9) w.bc[9 * (size_t)c + threadIdx.x] = b;
     // the diagonal block of S: D_c^2 + sum over the camera's observations (the waves in order);
     // the pair kernel writes the off-diagonal blocks only
     if (threadIdx.x < 45) {
-        const int k = threadIdx.x;
-        int r = 0, rem = k;
-        while (rem >= 9 - r) {
-            rem -= 9 - r;
-            ++r;
-        }
-        const int cc = r + rem;
+        const int k = threadIdx.x, r = sym9_row(k), cc = sym9_col(k);
         double v = dacc[0][k];
         for (int q = 1; q < NW; ++q) v += dacc[q][k];
         if (r == cc) v += w.dc2[9 * (size_t)c + r];
@@ -747,7 +745,7 @@ __global__ void __launch_bounds__(NT) k_wcand_cam(const WinDesc* __restrict__ de
         win_model_residual<M>(w, Psh, Gsh, j, X, r);
         acc[0] += half_rho(r[0] * r[0] + r[1] * r[1], o.loss, o.loss_a);
     }
-    wg_sum_fixed<1, NT>(acc, lds);
+    const double cost = wg_sums<1, NT>(acc, lds);
     if (threadIdx.x == 0) {
         double dx2 = 0.0, x2 = 0.0, model = 0.0;
         for (int i = 0; i < 9; ++i) {
@@ -759,7 +757,7 @@ __global__ void __launch_bounds__(NT) k_wcand_cam(const WinDesc* __restrict__ de
         }
         double* cp = w.cpart + WC_COUNT * (size_t)c;
         cp[WC_MODEL] = 0.5 * model;
-        cp[WC_CAND] = acc[0];
+        cp[WC_CAND] = cost;
         cp[WC_DX2] = dx2;
         cp[WC_X2] = x2;
     }
