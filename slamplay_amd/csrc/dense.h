@@ -152,17 +152,18 @@ __global__ void k_fill_S(double* __restrict__ S, int n, int ld, const double* __
 }
 
 // One 9x9 block of the reduced camera system per workgroup of NW waves (the blocks' pair lists, the
-// 36-value records of k_dense_store): pair_block in pair_block.h.  Bound by the products' instructions
-// and LDS reads (about 200 per 16 pairs) once the blocks of neighbouring cameras run on one XCD: 325 ->
-// 198 us at 250 cameras and 4.2M pairs (blocks in key order over all XCDs, the cameras' own blocks
-// among them), 78 -> 40 us at 49 cameras, 62 -> 9 us for a stereo window of 8.
+// 36-value records of k_dense_store): pair_block in pair_block.h.  Bound by LDS accesses and the products'
+// instructions once the blocks of neighbouring cameras run on one XCD; FP64 by its two wavefronts a SIMD
+// (238 registers) as well, FP32 is held to the three its 168 allow.  At 250 cameras and 4.2M pairs 325 us (blocks
+// in key order over all XCDs, the cameras' own blocks among them), 188 FP64 and 199 FP32 with sixteen
+// pairs a stage, 156 and 99 with 32; at 49 cameras 78, 37 and 29 us, for a window of 8 cameras 62, 5.5 and 5.8.
 template <typename Real, int NW>
 constexpr size_t schur_blocks_lds() {
     return (size_t)NW * pair_stage_bytes<Real, kRecDense>() + (NW > 1 ? NW * 81 * sizeof(double) : 0);
 }
 
 template <typename Real, int NW>
-__global__ void __launch_bounds__(64 * NW) k_schur_blocks(Dev<Real> d, const Real* __restrict__ js,
+__global__ void __launch_bounds__(64 * NW, sizeof(Real) == 4 ? 3 : 2) k_schur_blocks(Dev<Real> d, const Real* __restrict__ js,
                                                           const int4* __restrict__ blk, const int2* __restrict__ pairs,
                                                           double* __restrict__ S, int ld) {
     LMState* st = d.st;
@@ -608,7 +609,7 @@ struct DenseSchur {
     bool f64 = true;  // factor in FP64 (FP64 solver, or a small system)
     DevBuf<Real> js;
     DevBuf<int4> blk;
-    int schur_waves = 4;  // waves per block of the pair products
+    int schur_waves = 2;  // waves per block of the pair products
     DevBuf<int2> pairs;
     DevBuf<double> S, r, z, y;
     DevBuf<float> Af, Dinvf, Binvf, BinvTf;
@@ -653,11 +654,9 @@ struct DenseSchur {
             for (size_t k = 0; k < xq[x].size(); ++k) (*out)[k * kXcds + x] = xq[x][k];
         *n_pairs = total;
         // A workgroup of eight waves fills a CU's LDS with its staging areas, so it is taken only while
-        // every block still has a CU of its own (28 blocks of 380 pairs: 6.9 us against 7.8 with four
-        // waves and 15.9 with one; 1,130 blocks: 52 against 40).  Four waves otherwise: three such
-        // workgroups share a CU (1,130 blocks 70.8 -> 40 us and 8,856 blocks 205 -> 198 against one wave
-        // each; 193 with two).
-        schur_waves = (int)take.size() <= kCUs ? 8 : 4;
+        // every block still has a CU of its own (28 blocks of 380 pairs: 5.8 us against 6.5 with four
+        // waves).  Two waves otherwise: four such workgroups share a CU.
+        schur_waves = (int)take.size() <= kCUs ? 8 : 2;
         return BA_OK;
     }
 
@@ -777,7 +776,7 @@ struct DenseSchur {
         if (schur_waves == 8)
             enqueue_schur<8>(sv);
         else
-            enqueue_schur<4>(sv);
+            enqueue_schur<2>(sv);
         if (n <= kDenseSmallN) {
             sv.launch_shm("small_solve", k_dense_small, 1, kSmallThreads, small_system_doubles(n) * sizeof(double),
                           (const double*)S.p, ld, (const double*)d.bc, d.px, n, d.st);
