@@ -9,13 +9,13 @@
 // (pair_block.h, the products the batched windows use too).  A pair contributes
 // Jc~_i' (Hp_i Jp~_j') Jc~_j with Hp_i = Jp~_i Vinv_p, i.e. a 2x2 middle factor.
 //
-// The factorization is a tiled right-looking Cholesky (32 x 32 tiles): per step, the diagonal
-// tile is factored by one wave and its triangular inverse kept, the panel below is multiplied by
-// that inverse (TRSM as a small GEMM) and the trailing lower tiles are updated (SYRK/GEMM); both
-// products run on the matrix cores (v_mfma_f64_16x16x4f64, v_mfma_f32_16x16x4f32), and the
-// trailing update also factors the next diagonal tile, so a step is two launches.  The panel is
-// also stored transposed in the upper tiles (the factorization reads only the lower ones; in FP64
-// the factor overwrites S).  The triangular solves work on diagonal blocks of sixteen tiles whose
+// The factorization is a tiled right-looking Cholesky (32 x 32 tiles), two tile columns a step: a
+// diagonal tile is factored by one wave and its triangular inverse kept, the panel below is multiplied
+// by that inverse (TRSM as a small GEMM) and the trailing lower tiles are updated (SYRK/GEMM); the
+// products run on the matrix cores (v_mfma_f64_16x16x4f64, v_mfma_f32_16x16x4f32), and the trailing
+// update also factors the next pair of diagonal tiles, so a step is one launch.  The panel is stored
+// transposed in the upper tiles (the factorization reads only the lower ones; in FP64 the factor
+// overwrites S).  The triangular solves work on diagonal blocks of sixteen tiles whose
 // inverses are formed after the factorization: two launches per block and sweep, each a
 // matrix-vector product over many workgroups.  In mixed precision the factor is
 // FP32 and the step is refined in FP64 against the FP64 S (refine_steps iterations of
@@ -206,6 +206,12 @@ __device__ __forceinline__ typename Mfma<F>::acc tile_mma_nt(const F* __restrict
     return c;
 }
 
+// A lane's operand of such a product, loaded ahead of it.
+template <typename F>
+__device__ __forceinline__ void tile_operand(const F* __restrict__ Y, int ldy, int sj, F (&yv)[8]) {
+    Mfma<F>::load_row(Y + (size_t)(16 * sj + (threadIdx.x & 15)) * ldy, (threadIdx.x & 63) >> 4, yv);
+}
+
 // Factors the tile held in T (lower triangle used) with one wave and writes X = L^-1 (Dinv[k],
 // row-major, zero above the diagonal); L itself is not kept, nothing reads a factored diagonal tile.
 // Lane r < 32 keeps row r of the tile in registers, lane 32 + i row i of the identity: the column
@@ -213,100 +219,244 @@ __device__ __forceinline__ typename Mfma<F>::acc tile_mma_nt(const F* __restrict
 // turn the identity below it into L^-T, whose row i is column i of X, so the inverse costs no
 // instructions of its own (potrf_stacked).  Entries above the tile's diagonal are
 // updated with the rest and never read by another lane.  Returns false (and writes nothing) when a
-// pivot is not positive and finite.  Only one whole wave may call it.
+// pivot is not positive and finite.  Only one whole wave may call it.  T has rows of kTile + 1, X of ldx.
 template <typename F>
-__device__ __forceinline__ bool potrf_tile_wave(F (*T)[kTile + 1], F* __restrict__ X) {
+__device__ __forceinline__ bool potrf_tile_wave(const F* T, F* X, int ldx) {
     const int l = threadIdx.x & 63, r = l & 31;
     F a[kTile];
 #pragma unroll
     for (int c = 0; c < kTile; ++c) a[c] = l == kTile + c ? (F)1 : (F)0;
     if (l < kTile)
 #pragma unroll
-        for (int c = 0; c < kTile; ++c) a[c] = T[r][c];
+        for (int c = 0; c < kTile; ++c) a[c] = T[r * (kTile + 1) + c];
     if (!potrf_stacked<F>(a)) return false;
     if (l >= kTile)
 #pragma unroll
-        for (int m = 0; m < kTile; ++m) X[m * kTile + r] = a[m];
+        for (int m = 0; m < kTile; ++m) X[m * ldx + r] = a[m];
     return true;
 }
 
-// Diagonal tile k (used for the first tile; later ones are factored by the trailing update).
+// LDS tiles of the kernels below: rows start 16-byte aligned.
 template <typename F>
-__global__ void __launch_bounds__(64) k_potrf_tile(F* __restrict__ A, int ld, int k, F* __restrict__ Dinv, LMState* st) {
-    if (st->done || st->step_invalid) return;
-    __shared__ F T[kTile][kTile + 1];
-    const int l = threadIdx.x;
-    const size_t o = (size_t)(kTile * k) * ld + kTile * k;
-    for (int idx = l; idx < kTile * kTile; idx += 64) T[idx / kTile][idx % kTile] = A[o + (size_t)(idx / kTile) * ld + idx % kTile];
-    lds_barrier();
-    if (!potrf_tile_wave<F>(T, Dinv + (size_t)k * kTile * kTile) && l == 0) st->step_invalid = 1;
+constexpr int kLdsPitch = kTile + 16 / (int)sizeof(F);
+template <typename F>
+constexpr int kLdsTile = kTile * kLdsPitch<F>;
+constexpr int kStepThreads = 512;
+template <typename F>
+constexpr size_t step_pair_lds() {
+    return 8 * kLdsTile<F> * sizeof(F);
 }
 
-// Step k of the factorization in one launch, one workgroup per lower tile (i, j) of the trailing
-// matrix, k < j <= i, one 16 x 16 block per wave.  The panel tiles the update needs are formed in
-// the workgroup from the unscaled A_ik, A_jk and the kept inverse X_k = L_kk^-1 (L_ik = A_ik X_k',
-// the same matrix-core products in the same order as a separate panel launch would do), staged in
-// LDS, and A_ij -= L_ik L_jk' follows; so a step is one launch.  The workgroups of column k + 1
-// store L_ik' in the upper tile (k, i), which the factorization does not read; the lower tile
-// (i, k) still holds A_ik, which other workgroups of this launch read, and k_panel_down copies the
-// transposes into it once the factorization is done.  Block 0 (tile (k + 1, k + 1), dispatched
-// first) keeps its result in LDS and factors it, so the next step's diagonal factor costs no launch
-// of its own.
+// Factors the 64 x 64 diagonal block of tiles t, t + 1 from its tiles T00, T11 (rows of kTile + 1) and T10
+// (kLdsPitch) in LDS; X is one tile more.  Leaves X_t and X_t+1 in Dinv and L_t+1,t in the lower tile (t + 1, t),
+// transposed also in the upper one.  All kStepThreads threads call it, before a barrier on the tiles; all
+// but the first wave run idle() while that factors tile t.
+template <typename F, typename Idle>
+__device__ __forceinline__ void factor_pair(F* T00, F* T10, F* T11, F* X, F* __restrict__ A, int ld, int t,
+                                            F* __restrict__ Dinv, LMState* st, Idle idle) {
+    constexpr int PP = kLdsPitch<F>;
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, si = (w >> 1) & 1, sj = w & 1;
+    lds_barrier();
+    if (w > 0)
+        idle();
+    else if (!potrf_tile_wave<F>(T00, X, PP) && l == 0)
+        st->step_invalid = 1;
+    lds_barrier();
+    F* L = T00;  // L_t+1,t takes its place, rows of kLdsPitch
+    if (w < 4) {
+        typename Mfma<F>::acc p = {0, 0, 0, 0};
+        p = tile_mma_nt<F>(T10, PP, X, PP, si, sj, p, (F)1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) L[(16 * si + Mfma<F>::row(l, e)) * PP + 16 * sj + (l & 15)] = p[e];
+    } else {
+        for (int idx = threadIdx.x - 256; idx < kTile * kTile; idx += 256)
+            Dinv[(size_t)t * kTile * kTile + idx] = X[(idx / kTile) * PP + idx % kTile];
+    }
+    lds_barrier();
+    if (w >= 4) {
+        F* low = A + (size_t)(kTile * (t + 1)) * ld + kTile * t;
+        F* up = A + (size_t)(kTile * t) * ld + kTile * (t + 1);
+        for (int idx = threadIdx.x - 256; idx < kTile * kTile; idx += 256) {
+            const int a = idx / kTile, b = idx % kTile;
+            low[(size_t)a * ld + b] = L[a * PP + b];
+            up[(size_t)a * ld + b] = L[b * PP + a];
+        }
+    } else if (si >= sj) {
+        typename Mfma<F>::acc c = {0, 0, 0, 0};
+        F* mine = T11 + (16 * si) * (kTile + 1) + 16 * sj + (l & 15);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = mine[Mfma<F>::row(l, e) * (kTile + 1)];
+        c = tile_mma_nt<F>(L, PP, L, PP, si, sj, c, (F)-1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mine[Mfma<F>::row(l, e) * (kTile + 1)] = c[e];
+    }
+    lds_barrier();
+    if (w == 0 && !potrf_tile_wave<F>(T11, Dinv + (size_t)(t + 1) * kTile * kTile, kTile) && l == 0) st->step_invalid = 1;
+}
+
+// The first diagonal block (later ones are factored by the trailing update).
 template <typename F>
-__global__ void __launch_bounds__(256) k_step_tiles(F* __restrict__ A, int ld, int k, F* __restrict__ Dinv, LMState* st) {
+__global__ void __launch_bounds__(kStepThreads) k_potrf_pair(F* __restrict__ A, int ld, F* __restrict__ Dinv, LMState* st) {
     if (st->done || st->step_invalid) return;
-    constexpr int PP = kTile + 16 / (int)sizeof(F);  // LDS row pitch: rows start 16-byte aligned
-    __shared__ __align__(16) F P[2][kTile * PP];     // L_ik, L_jk
-    __shared__ F T[kTile][kTile + 1];
+    extern __shared__ __align__(16) unsigned char step_lds_mem[];
+    F* const lds = reinterpret_cast<F*>(step_lds_mem);
+    F *T00 = lds, *T10 = lds + kLdsTile<F>, *T11 = lds + 2 * kLdsTile<F>;
+    for (int idx = threadIdx.x; idx < kTile * kTile; idx += kStepThreads) {
+        const int a = idx / kTile, b = idx % kTile;
+        T00[a * (kTile + 1) + b] = A[(size_t)a * ld + b];
+        T10[a * kLdsPitch<F> + b] = A[(size_t)(kTile + a) * ld + b];
+        T11[a * (kTile + 1) + b] = A[(size_t)(kTile + a) * ld + kTile + b];
+    }
+    factor_pair<F>(T00, T10, T11, lds + 3 * kLdsTile<F>, A, ld, 0, Dinv, st, [] {});
+}
+
+// Step K of the factorization in one launch: tile columns k = 2 K and k + 1, one workgroup per lower 64 x 64
+// block (I, J) of the trailing matrix, K < J <= I.  The panel tiles the update needs are formed in the
+// workgroup from the unscaled A_ik, A_i,k+1 (rows of I and of J) and the kept inverses:
+//   L_ik = A_ik X_k',   L_i,k+1 = (A_i,k+1 - L_ik L_k+1,k') X_k+1',
+// staged in LDS, and A_ij -= L_ik L_jk' + L_i,k+1 L_j,k+1' follows, each wave on one 16 x 16 block of two
+// tiles: the products and sums of two steps of one tile column each, in their order.  The workgroups of
+// block column K + 1 store L' in the upper tiles, which the factorization does not read; the lower tiles of
+// columns k and k + 1 still hold what other workgroups of this launch read, and k_panel_down copies the
+// transposes into them once the factorization is done.  Block 0 (dispatched first) keeps its tiles in LDS
+// and factors them, so the next step's diagonal factors cost no launch of their own.  A step is bound by
+// that workgroup's chain, two tile factors (3 us each) behind two panels.  One launch per tile column paid the
+// launch, the first loads and the trailing matrix's read and write twice: at 2250 unknowns the factorization
+// took 832 us in FP64 and 552 in FP32, against 660 and 463; at 441, where the trailing matrix is small, 100
+// against 104.
+template <typename F>
+__global__ void __launch_bounds__(kStepThreads, 4) k_step_pair(F* __restrict__ A, int ld, int K, F* __restrict__ Dinv,
+                                                               LMState* st) {
+    if (st->done || st->step_invalid) return;
+    constexpr int PP = kLdsPitch<F>, TS = kLdsTile<F>;
+    extern __shared__ __align__(16) unsigned char step_lds_mem[];
+    F* const P = reinterpret_cast<F*>(step_lds_mem);  // tiles 0-3: L_.k of the rows of I, J; 4-7: L_.,k+1
     const int b = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
     int ii = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
     while ((ii + 1) * (ii + 2) / 2 <= b) ++ii;
     while (ii * (ii + 1) / 2 > b) --ii;
     const int jj = b - ii * (ii + 1) / 2;
-    const int i = k + 1 + ii, j = k + 1 + jj;
-    const int si = w >> 1, sj = w & 1;
-    const bool next_diag = b == 0;
-    const F* Xk = Dinv + (size_t)k * kTile * kTile;
-    F* Aij = A + (size_t)(kTile * i) * ld + kTile * j;
-    // the tile's own entries are requested before the panel products (a load after the barrier waits
-    // for memory once more)
-    typename Mfma<F>::acc c = {0, 0, 0, 0};
-    const bool own = !(i == j && si < sj);
-    if (own)
+    const int k = 2 * K, i0 = k + 2 + 2 * ii, j0 = k + 2 + 2 * jj;  // first tiles of the step, of I and of J
+    const bool diag = ii == jj;
+    const int half = w >> 2, si = (w >> 1) & 1, sj = w & 1;
+    // Panels: each wave a strip of 16 rows of I (waves 0-3) or of J (4-7, none on the diagonal), whose
+    // operands pass from product to product through the strip's LDS rows, between the wave's own lanes.
+    using Acc = typename Mfma<F>::acc;
+    const int l16 = l & 15;
+    if (w < 4 || !diag) {
+        const int tile = (w >> 1) & 1, strip = w & 1, slot = 2 * (w >> 2) + tile;
+        const F* row = A + (size_t)(kTile * ((w < 4 ? i0 : j0) + tile)) * ld + kTile * k;
+        F xv[8], y[2][8];
+        Acc p[2], a2[2];
+        tile_operand<F>(row, ld, strip, xv);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = Aij[(size_t)(16 * si + Mfma<F>::row(l, e)) * ld + 16 * sj + (l & 15)];
-    // panel tiles of rows i and j (one of them when i == j)
+        for (int sj = 0; sj < 2; ++sj) tile_operand<F>(Dinv + (size_t)k * kTile * kTile, kTile, sj, y[sj]);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        if (t == 1 && i == j) break;
-        const F* Ark = A + (size_t)(kTile * (t == 0 ? i : j)) * ld + kTile * k;
-        typename Mfma<F>::acc p = {0, 0, 0, 0};
-        p = tile_mma_nt<F>(Ark, ld, Xk, kTile, si, sj, p, (F)1);
+        for (int sj = 0; sj < 2; ++sj)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) P[t][(16 * si + Mfma<F>::row(l, e)) * PP + 16 * sj + (l & 15)] = p[e];
-    }
-    lds_barrier();
-    if (j == k + 1) {
-        F* Aki = A + (size_t)(kTile * k) * ld + kTile * i;
-        for (int idx = threadIdx.x; idx < kTile * kTile; idx += 256) {
-            const int cc = idx / kTile, rr = idx % kTile;
-            Aki[(size_t)cc * ld + rr] = P[0][rr * PP + cc];
+            for (int e = 0; e < 4; ++e) a2[sj][e] = row[(size_t)(16 * strip + Mfma<F>::row(l, e)) * ld + kTile + 16 * sj + l16];
+        F y2[2][8];
+#pragma unroll
+        for (int sj = 0; sj < 2; ++sj) tile_operand<F>(A + (size_t)(kTile * (k + 1)) * ld + kTile * k, ld, sj, y2[sj]);
+        F* out = P + slot * TS + 16 * strip * PP + l16;
+#pragma unroll
+        for (int sj = 0; sj < 2; ++sj) {
+            p[sj] = Acc{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) p[sj] = Mfma<F>::mma(xv[s], y[sj][s], p[sj]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[Mfma<F>::row(l, e) * PP + 16 * sj] = p[sj][e];
+        }
+#pragma unroll
+        for (int sj = 0; sj < 2; ++sj) tile_operand<F>(Dinv + (size_t)(k + 1) * kTile * kTile, kTile, sj, y[sj]);
+        wave_sync_lds();
+        tile_operand<F>(P + slot * TS, PP, strip, xv);
+        out += 4 * TS;
+#pragma unroll
+        for (int sj = 0; sj < 2; ++sj) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) a2[sj] = Mfma<F>::mma(-xv[s], y2[sj][s], a2[sj]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[Mfma<F>::row(l, e) * PP + 16 * sj] = a2[sj][e];
+        }
+        wave_sync_lds();
+        tile_operand<F>(P + (4 + slot) * TS, PP, strip, xv);
+        wave_sync_lds();
+#pragma unroll
+        for (int sj = 0; sj < 2; ++sj) {
+            p[sj] = Acc{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) p[sj] = Mfma<F>::mma(xv[s], y[sj][s], p[sj]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[Mfma<F>::row(l, e) * PP + 16 * sj] = p[sj][e];
         }
     }
-    if (own) {
-        c = tile_mma_nt<F>(P[0], PP, i == j ? P[0] : P[1], PP, si, sj, c, (F)-1);
+    // block (si, sj) of tile (i0 + u, j0 + v), less its products
+    const F* Pj = P + (diag ? 0 : 2) * TS;
+    auto load_block = [&](int u, int v, int si, int sj) {
+        Acc c;
+        const F* Aij = A + (size_t)(kTile * (i0 + u) + 16 * si) * ld + kTile * (j0 + v) + 16 * sj + l16;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int rr = 16 * si + Mfma<F>::row(l, e), cc = 16 * sj + (l & 15);
-            if (next_diag)
-                T[rr][cc] = c[e];
-            else
-                Aij[(size_t)rr * ld + cc] = c[e];
+        for (int e = 0; e < 4; ++e) c[e] = Aij[(size_t)Mfma<F>::row(l, e) * ld];
+        return c;
+    };
+    auto update_block = [&](int u, int v, int si, int sj, Acc c) {
+        c = tile_mma_nt<F>(P + u * TS, PP, Pj + v * TS, PP, si, sj, c, (F)-1);
+        return tile_mma_nt<F>(P + (4 + u) * TS, PP, Pj + (4 + v) * TS, PP, si, sj, c, (F)-1);
+    };
+    auto store_panel = [&](int first, int threads) {
+        for (int idx = first; idx < 4 * kTile * kTile; idx += threads) {
+            const int t = idx / (kTile * kTile), cc = idx / kTile % kTile, rr = idx % kTile;  // t: (column, row tile)
+            A[(size_t)(kTile * (k + (t >> 1)) + cc) * ld + kTile * (i0 + (t & 1)) + rr] =
+                P[(4 * (t >> 1) + (t & 1)) * TS + rr * PP + cc];
         }
+    };
+    if (b > 0) {
+        Acc c[2];
+        bool own[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            own[u] = !diag || u > half || (u == half && si >= sj);
+            if (own[u]) c[u] = load_block(u, half, si, sj);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (!own[u]) continue;
+            c[u] = update_block(u, half, si, sj, c[u]);
+            F* Aij = A + (size_t)(kTile * (i0 + u) + 16 * si) * ld + kTile * (j0 + half) + 16 * sj + l16;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Aij[(size_t)Mfma<F>::row(l, e) * ld] = c[u][e];
+        }
+        if (jj == 0) store_panel(threadIdx.x, kStepThreads);
+        return;
     }
-    if (!next_diag) return;
+    // The next diagonal block, in LDS tiles that a diagonal workgroup's panels do not use.  Tile (0, 0) first,
+    // by three waves; the others' blocks and the panel's store run while it is factored.
+    F *T00 = P + 2 * TS, *T10 = P + 3 * TS, *T11 = P + 6 * TS;
+    // waves 0-2: (0, 0) of tile (0, 0), then blocks (0, 0), (1, 0), (1, 1) of tile (1, 1) in waves 1-3; 4-7: tile (1, 0)
+    auto put = [&](F* T, int pitch, int bi, int bj, Acc c) {
+        F* out = T + 16 * bi * pitch + 16 * bj + l16;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[Mfma<F>::row(l, e) * pitch] = c[e];
+    };
+    const int bi0 = w > 0, bj0 = w > 1;  // wave's block of tile (0, 0)
+    const int bi1 = w > 1, bj1 = w > 2;  // and of tile (1, 1)
+    Acc c0 = {0, 0, 0, 0}, c1 = {0, 0, 0, 0};
+    if (w < 3) c0 = load_block(0, 0, bi0, bj0);
+    if (w > 3)
+        c1 = load_block(1, 0, si, sj);
+    else if (w > 0)
+        c1 = load_block(1, 1, bi1, bj1);
     lds_barrier();
-    if (w == 0 && !potrf_tile_wave<F>(T, Dinv + (size_t)(k + 1) * kTile * kTile) && l == 0) st->step_invalid = 1;
+    if (w < 3) put(T00, kTile + 1, bi0, bj0, update_block(0, 0, bi0, bj0, c0));
+    factor_pair<F>(T00, T10, T11, P + 7 * TS, A, ld, k + 2, Dinv, st, [&] {
+        if (w > 3)
+            put(T10, PP, si, sj, update_block(1, 0, si, sj, c1));
+        else
+            put(T11, kTile + 1, bi1, bj1, update_block(1, 1, bi1, bj1, c1));
+        store_panel(threadIdx.x - 64, kStepThreads - 64);
+    });
 }
 
 // After the factorization: L_ik = (tile (k, i))' into the lower tile (i, k), i > k (one workgroup per
@@ -664,7 +814,7 @@ struct DenseSchur {
     int create(const Layout& L, const int* cam_off, const int* co_pt, const ba_options& o, hipStream_t s) {
         const int nc = L.nc;
         n = 9 * nc;
-        nt = std::max(1, (n + kTile - 1) / kTile);
+        nt = 2 * std::max(1, (n + 2 * kTile - 1) / (2 * kTile));  // whole 64 x 64 blocks
         ld = nt * kTile;
         nb = (nt + kSolveBlk - 1) / kSolveBlk;
         f64 = sizeof(Real) == sizeof(double) || n <= kDenseF64MaxN;
@@ -703,6 +853,8 @@ struct DenseSchur {
             BA_TRY(Binvd.alloc(binv));
             BA_TRY(BinvTd.alloc(binv));
             BA_TRY(allow_dynamic_lds((const void*)k_block_inverse<double>, (int)block_inverse_lds(nt)));
+            BA_TRY(allow_dynamic_lds((const void*)k_potrf_pair<double>, (int)step_pair_lds<double>()));
+            BA_TRY(allow_dynamic_lds((const void*)k_step_pair<double>, (int)step_pair_lds<double>()));
         } else {
             BA_TRY(Af.alloc((size_t)ld * ld));
             BA_TRY(Dinvf.alloc((size_t)nt * kTile * kTile));
@@ -740,12 +892,12 @@ struct DenseSchur {
     template <typename F, typename SolverT>
     void factor_and_solve(SolverT& sv, F* A, F* Dinv, F* Binv, F* BinvT) {
         auto& d = sv.d;
-        sv.launch("potrf", k_potrf_tile<F>, 1, 64, A, ld, 0, Dinv, d.st);
-        for (int k = 0; k + 1 < nt; ++k) {
-            const int m = nt - k - 1;
-            sv.launch("step", k_step_tiles<F>, m * (m + 1) / 2, 256, A, ld, k, Dinv, d.st);
+        sv.launch_shm("potrf", k_potrf_pair<F>, 1, kStepThreads, step_pair_lds<F>(), A, ld, Dinv, d.st);
+        for (int K = 0; K + 1 < nt / 2; ++K) {
+            const int m = nt / 2 - 1 - K;
+            sv.launch_shm("step", k_step_pair<F>, m * (m + 1) / 2, kStepThreads, step_pair_lds<F>(), A, ld, K, Dinv, d.st);
         }
-        if (nt > 1) sv.launch("panel_down", k_panel_down<F>, nt * (nt - 1) / 2, 256, A, ld, (const LMState*)d.st);
+        sv.launch("panel_down", k_panel_down<F>, nt * (nt - 1) / 2, 256, A, ld, (const LMState*)d.st);
         sv.launch_shm("block_inverse", k_block_inverse<F>, nb * kSolveRows / kInvCols, kInvThreads, block_inverse_lds(nt), (const F*)A, ld,
                       (const F*)Dinv, Binv, BinvT, nt, (const LMState*)d.st);
         solve<F>(sv, A, Binv, BinvT, (const double*)d.bc, d.px, 0);

@@ -103,7 +103,7 @@ __device__ __forceinline__ void factor_columns(F (&a)[kTile], F inv, bool* bad) 
 // updates as row-broadcast operands; the next column is updated first and its pivot's reciprocal root
 // started, so that chain runs under the other columns' updates.  Bound by instruction issue, 7,300
 // cycles a tile of which the chain alone takes 3,000 (multipliers by v_readlane: 11,700; through LDS: 10,900).
-// A step of the 2250 x 2250 factorization, whose time it sets: 17.9 -> 7.0 us in FP64 (late steps), 15.1 -> 7.8 in FP32 (all),
+// A step of one tile column of the 2250 x 2250 factorization, whose time it set: 17.9 -> 7.0 us in FP64 (late steps), 15.1 -> 7.8 in FP32 (all),
 // against masked updates with v_readlane and an inverse by forward substitution afterwards.  Returns
 // false when a pivot is not positive and finite.
 template <typename F>
