@@ -359,10 +359,11 @@ __global__ void __launch_bounds__(NT) k_wdamp(const WinDesc* __restrict__ descs,
     const WinDesc D = descs[wtask[t]];
     const WinPtrs w = win_ptrs(D, arena);
     WinState* st = w.st;
-    if (st->done) return;
+    const int done = st->done, need_lin = st->need_lin, first = st->first_lin;
+    __syncthreads();  // every wave has read them before the first thread changes them
+    if (done) return;
     const int K = w.K, P = w.P, n = 9 * K, tid = threadIdx.x;
-    if (st->need_lin) {
-        const int first = st->first_lin;
+    if (need_lin) {
         if (first)
             for (int k = tid; k < n; k += NT) w.sc[k] = o.jacobi_scaling ? 1.0 / (1.0 + sqrt(w.udiag[k])) : 1.0;
         if (tid == 0) {
@@ -869,7 +870,9 @@ __global__ void __launch_bounds__(NT) k_wdecide(const WinDesc* __restrict__ desc
     const WinDesc D = descs[wtask[t]];
     const WinPtrs w = win_ptrs(D, arena);
     WinState* st = w.st;
-    if (st->done) return;
+    const int done = st->done;
+    __syncthreads();  // every wave has read it before the first thread changes the state
+    if (done) return;
     if (threadIdx.x == 0) {
         accepted = 0;
         const bool have_step = st->have_step != 0;
