@@ -37,35 +37,63 @@ namespace mba {
 constexpr int kJs = 36;  // per-observation stride of Jc~ (18, by columns), Jp~ (6), Hp (6), I - G (3)
 static_assert(kJs == RecLayout<kRecDense>::stride, "the dense record is pair_block's kRecDense");
 
+// The pair products' records (kRecDense).  `parts` workgroups share a camera's observations: with one, 49
+// cameras of 640 observations leave most of the chip idle (28 us against 10.5).  Bound by the stores: by the
+// lanes that form the records, 48 us in FP64 and 32 in FP32 at 250 cameras and 1M observations, through LDS
+// 40 and 18.
 template <typename Real, int M>
-__global__ void __launch_bounds__(kWG) k_dense_store(Dev<Real> d, Real* __restrict__ js) {
+__global__ void __launch_bounds__(kWG, 4) k_dense_store(Dev<Real> d, Real* __restrict__ js, int parts) {
     LMState* st = d.st;
     if (st->done || st->step_invalid) return;
-    const int c = xcd_remap(blockIdx.x, d.nc);
+    __shared__ Unit16 lds[kWaves][64 * kRecordRow];
+    constexpr bool f64 = sizeof(Real) == 8;  // a record is two rows then, J~_c and the rest, else one
+    const int per_part = gridDim.x / parts, part = blockIdx.x / per_part;
+    const int c = xcd_remap(blockIdx.x - part * per_part, d.nc);
     if (c >= d.nc) return;
     const CameraPrep<Real> P = d.prep[c];
     Real sc[9];
     for (int i = 0; i < 9; ++i) sc[i] = (Real)d.sc[9 * (size_t)c + i];
-    for (int j = d.cam_off[c] + threadIdx.x; j < d.cam_off[c + 1]; j += kWG) {
-        int p;
-        Real r[2], Jc[18], Jp[6];
-        corrected_jacobian<Real, M>(d, P, j, p, r, Jc, Jp);
-        Real* o = js + kJs * (size_t)j;
-        for (int i = 0; i < 9; ++i) {  // J~_c by columns: the two residual rows of column i adjacent
-            o[2 * i] = Jc[i] * sc[i];
-            o[2 * i + 1] = Jc[9 + i] * sc[i];
+    const int end = d.cam_off[c + 1], wave = threadIdx.x >> 6;
+    // rounds of a workgroup's observations, every lane taking part in the stores
+    for (int j0 = d.cam_off[c] + kWG * part + 64 * wave; j0 < end; j0 += kWG * parts) {
+        const int j = j0 + (threadIdx.x & 63);
+        Real Jc[18];
+#pragma unroll
+        for (int i = 0; i < 18; ++i) Jc[i] = (Real)0;
+        if (j < end) {
+            int p;
+            Real r[2], Jp[6], h[6], ig[3];
+            corrected_jacobian<Real, M>(d, P, j, p, r, Jc, Jp);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                Jc[i] *= sc[i];
+                Jc[9 + i] *= sc[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const Real s = (Real)d.sp[3 * (size_t)p + i];
+                Jp[i] *= s;
+                Jp[3 + i] *= s;
+            }
+            sym3_mul<Real>(d.VinvR + 6 * (size_t)p, Jp, h);
+            sym3_mul<Real>(d.VinvR + 6 * (size_t)p, Jp + 3, h + 3);
+            point_complement<Real, Real>(d, p, Jp, ig[0], ig[1], ig[2]);
+            const int at = f64 ? 0 : 9;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                stage_pair<Real>(lds[wave], at + i, Jp[2 * i], Jp[2 * i + 1]);
+                stage_pair<Real>(lds[wave], at + 3 + i, h[2 * i], h[2 * i + 1]);
+            }
+            stage_pair<Real>(lds[wave], at + 6, ig[0], ig[1]);
+            stage_pair<Real>(lds[wave], at + 7, ig[2], (Real)0);
+            stage_pair<Real>(lds[wave], at + 8, (Real)0, (Real)0);
         }
-        for (int i = 0; i < 3; ++i) {
-            const Real s = (Real)d.sp[3 * (size_t)p + i];
-            Jp[i] *= s;
-            Jp[3 + i] *= s;
-        }
-        for (int i = 0; i < 6; ++i) o[18 + i] = Jp[i];
-        Real h[6];
-        sym3_mul<Real>(d.VinvR + 6 * (size_t)p, Jp, h);
-        sym3_mul<Real>(d.VinvR + 6 * (size_t)p, Jp + 3, h + 3);
-        for (int i = 0; i < 6; ++i) o[24 + i] = h[i];
-        point_complement<Real, Real>(d, p, Jp, o[30], o[31], o[32]);
+        const int n = min(64, end - j0);
+        Real* out = js + kJs * (size_t)j0;
+        if (f64) flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 9, n);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) stage_pair<Real>(lds[wave], i, Jc[i], Jc[9 + i]);  // the rows of column i adjacent
+        flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 0, n);
     }
 }
 
@@ -759,6 +787,7 @@ struct DenseSchur {
     bool f64 = true;  // factor in FP64 (FP64 solver, or a small system)
     DevBuf<Real> js;
     DevBuf<int4> blk;
+    int store_parts = 1;  // workgroups of k_dense_store per camera
     int schur_waves = 2;  // waves per block of the pair products
     DevBuf<int2> pairs;
     DevBuf<double> S, r, z, y;
@@ -817,6 +846,10 @@ struct DenseSchur {
         nt = 2 * std::max(1, (n + 2 * kTile - 1) / (2 * kTile));  // whole 64 x 64 blocks
         ld = nt * kTile;
         nb = (nt + kSolveBlk - 1) / kSolveBlk;
+        // two workgroups a CU, while a camera has rounds to share
+        int most = 0;
+        for (int c = 0; c < nc; ++c) most = std::max(most, L.cam_off[c + 1] - L.cam_off[c]);
+        store_parts = std::max(1, std::min((2 * kCUs + nc - 1) / std::max(nc, 1), (most + kWG - 1) / kWG));
         f64 = sizeof(Real) == sizeof(double) || n <= kDenseF64MaxN;
         refine = f64 ? 0 : std::max(0, o.refine_steps);
         if (nc > 0) {
@@ -921,7 +954,7 @@ struct DenseSchur {
         sv.launch("dense_store",
                   pick_model(d.model, k_dense_store<Real, kModelSnavely>, k_dense_store<Real, kModelSnavelyG2o>,
                              k_dense_store<Real, kModelStereo>),
-                  xcd_grid(nc), kWG, d, js.p);
+                  xcd_grid(nc) * store_parts, kWG, d, js.p, store_parts);
         const size_t nn = (size_t)ld * ld;
         sv.launch("fill_S", k_fill_S, (int)((nn + 255) / 256), 256, S.p, n, ld, (const double*)d.M,
                   (const LMState*)d.st);

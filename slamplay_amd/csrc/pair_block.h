@@ -56,6 +56,29 @@ struct RecLayout<kRecDense> {
     __device__ static int chunk(int e) { return e < ci ? (e < 5 ? e : e + 1) : e - ci; }
 };
 
+// A wave's records on their way to memory go through LDS, so that neighbouring lanes write neighbouring
+// 16-byte units: stored by the lanes that form them, each store instruction touches 64 records' lines, a
+// part of a line at a time.  stage_pair puts two values of the lane's record, at pair `at` of its row of
+// kRecordRow units; flush_records stores `step` units of every row, units u0 .. of the first n records at out.
+typedef unsigned int Unit16 __attribute__((ext_vector_type(4)));
+constexpr int kRecordRow = 9;  // odd: neighbouring rows start in different banks
+template <typename Real>
+__device__ __forceinline__ void stage_pair(Unit16* lds, int at, Real x, Real y) {
+    reinterpret_cast<R2v<Real>*>(lds + kRecordRow * (threadIdx.x & 63))[at] = R2v<Real>{x, y};
+}
+template <int units, int step, typename Real>
+__device__ __forceinline__ void flush_records(const Unit16* lds, Real* __restrict__ out, int u0, int n) {
+    static_assert(step <= kRecordRow && step <= units, "a row's units");
+    const int lane = threadIdx.x & 63;
+    wave_sync_lds();
+#pragma unroll 4
+    for (int s = 0; s < step; ++s) {
+        const int e = 64 * s + lane, rec = e / step, u = e - step * rec;
+        if (rec < n) reinterpret_cast<Unit16*>(out)[(size_t)units * rec + u0 + u] = lds[kRecordRow * rec + u];
+    }
+    wave_sync_lds();
+}
+
 // The staging area holds 16-byte units (a slot in FP32, half a slot in FP64), unit u of pair k at
 // u (32 + 1) + k: neighbouring pairs' units are adjacent for the reads, and a pair's units, which
 // neighbouring lanes store, lie in different banks.  FP64 keeps the slots' second halves after all first ones.

@@ -435,13 +435,15 @@ __global__ void __launch_bounds__(NT) k_wdamp(const WinDesc* __restrict__ descs,
     }
 }
 
-// Per (window, camera): records of the reduced system and b_c.
+// Per (window, camera): records of the reduced system and b_c.  Bound by the records' stores, 256 bytes an
+// observation, which go through LDS (56 -> 47 us a launch of 32 windows).
 template <typename Real, int NT, int M>
-__global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ descs, char* __restrict__ arena,
+__global__ void __launch_bounds__(NT, 4) k_wrec_cam(const WinDesc* __restrict__ descs, char* __restrict__ arena,
                                                  const int2* __restrict__ ctask, int ntask, Opts o) {
     constexpr int NW = NT / 64;
     __shared__ double lds[9 * NW];
     __shared__ double dacc[NW][45];  // per wave: upper triangle of sum J~_c'(I - G)J~_c
+    __shared__ Unit16 rlds[NW][64 * kRecordRow];
     __shared__ CameraPrep<double> Psh;
     __shared__ StereoRig Gsh;
     const int t = blockIdx.x;
@@ -481,18 +483,15 @@ __global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ des
             double h0[3], h1[3];
             sym3_mul<double>(Vi, j0, h0);
             sym3_mul<double>(Vi, j1, h1);
-            Real* out = js + kWinJs * (size_t)j;
+            // the record's second half: column 8 of J~_c, H, J~_p
+            const int at = sizeof(Real) == 8 ? 0 : 8;
+            stage_pair<Real>(rlds[wave], at, (Real)Jc[8], (Real)Jc[17]);
+            stage_pair<Real>(rlds[wave], at + 1, (Real)h0[0], (Real)h0[1]);
+            stage_pair<Real>(rlds[wave], at + 2, (Real)h0[2], (Real)h1[0]);
+            stage_pair<Real>(rlds[wave], at + 3, (Real)h1[1], (Real)h1[2]);
 #pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                out[2 * i] = (Real)Jc[i];
-                out[2 * i + 1] = (Real)Jc[9 + i];
-            }
-            for (int i = 0; i < 3; ++i) {
-                out[18 + i] = (Real)h0[i];
-                out[21 + i] = (Real)h1[i];
-            }
-#pragma unroll
-            for (int i = 0; i < 6; ++i) out[24 + i] = (Real)Jp[i];
+            for (int i = 0; i < 3; ++i) stage_pair<Real>(rlds[wave], at + 4 + i, (Real)Jp[2 * i], (Real)Jp[2 * i + 1]);
+            stage_pair<Real>(rlds[wave], at + 7, (Real)0, (Real)0);
             g00 = 1.0 - (j0[0] * h0[0] + j0[1] * h0[1] + j0[2] * h0[2]);
             g01 = -(j0[0] * h1[0] + j0[1] * h1[1] + j0[2] * h1[2]);
             g11 = 1.0 - (j1[0] * h1[0] + j1[1] * h1[1] + j1[2] * h1[2]);
@@ -504,6 +503,13 @@ __global__ void __launch_bounds__(NT) k_wrec_cam(const WinDesc* __restrict__ des
 #pragma unroll
             for (int i = 0; i < 18; ++i) Jd[i] = Jc[i];
         }
+        const int jw = j0r + 64 * wave, nw = min(64, j_end - jw);  // the wave's observations (possibly none)
+        constexpr int units = kWinJs * (int)sizeof(Real) / 16;
+        Real* out = js + kWinJs * (size_t)jw;
+        if (sizeof(Real) == 8) flush_records<units, 8>(rlds[wave], out, 8, nw);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) stage_pair<Real>(rlds[wave], i, (Real)Jd[i], (Real)Jd[9 + i]);
+        flush_records<units, 8>(rlds[wave], out, 0, nw);
         // the observation's own term of the camera's diagonal block: J~_c'(I - G)J~_c
         double t0[9], t1[9];
 #pragma unroll
