@@ -255,7 +255,8 @@ struct Solver final : SolverBase {
     DevBuf<double> U, gc, sc, dc2, M, Minv, bc, px, pr, pz, pp, qc;
     DevBuf<double> V, gp, sp, dp2, Vinv64, upd_part, rz_hist;
     DevBuf<Real> VinvR;
-    DevBuf<R4<Real>> qp, u;
+    DevBuf<R4<Real>> qp;
+    DevBuf<R3<Real>> u;
     DevBuf<double4> zs;
     DevBuf<R4<Real>> pv;
     DevBuf<double> cam_part, pt_part;
