@@ -720,14 +720,14 @@ struct Solver final : SolverBase {
         // point index and the point's FP64 zs (jz); per camera its prep and the 9-vectors read and
         // written
         const double prep_b = sizeof(CameraPrep<Real>);
-        if (n == "jtx" && dir) return no * (4 * R + 4 + 4 * R) + nc * (prep_b + 9 * 8 * 4 + 2 * 8 * d.n_upd);
+        if (n == "jtx" && dir) return no * (4 * R + 4 + 3 * R) + nc * (prep_b + 9 * 8 * 4 + 2 * 8 * d.n_upd);
         if (n == "jz" && dir) return no * (4 * R + 4) + np * 32 + nc * (prep_b + 9 * 8 * 5);
-        if (n == "jtx" || n == "jtx_y") return no * (4 + 4 + 2 * R + 4 * R) + np * 4 * 8 + nc * 9 * 8 * 3;
+        if (n == "jtx" || n == "jtx_y") return no * (4 + 4 + 2 * R + 3 * R) + np * 4 * 8 + nc * 9 * 8 * 3;
         if (n == "jz") return no * (4 + 2 * R) + np * (4 * 8 + 4 * R) + nc * 9 * 8 * 8;
         // u by slot; per point its scale, FP64 V*^-1 (6), D_p^2, and the FP64 zs written
-        if (n == "pt_z") return no * 4 * R + np * (3 * 8 + 6 * 8 + 3 * 8 + 32);
-        if (n == "lin_cam") return no * (4 + 4 + 2 * R + 12 * 8) + np * 4 * 8 + nc * 18 * 8;
-        if (n == "lin_pt") return no * 12 * 8 + np * 9 * 8;
+        if (n == "pt_z") return no * 3 * R + np * (3 * 8 + 6 * 8 + 3 * 8 + 32);
+        if (n == "lin_cam") return no * (4 + 4 + 2 * R + 8 * R) + np * 4 * 8 + nc * 18 * 8;
+        if (n == "lin_pt") return no * 8 * R + np * 9 * 8;
         if (n == "rhs_cam") return no * (4 + 2 * R) + np * (3 * 8 + 3 * 8 + 6 * R + 3 * R) + nc * (81 * 3 + 9 * 3) * 8;
         if (n == "model_cand") return no * (4 + 2 * R + 16) + np * 3 * 8 * 3 + nc * 9 * 8;
         return 0.0;
