@@ -37,17 +37,37 @@ namespace mba {
 constexpr int kJs = 36;  // per-observation stride of Jc~ (18, by columns), Jp~ (6), Hp (6), I - G (3)
 static_assert(kJs == RecLayout<kRecDense>::stride, "the dense record is pair_block's kRecDense");
 
+// S <- the cameras' Schur-Jacobi blocks M_c (k_rhs_cam: D_c^2 plus every observation with itself) on the
+// diagonal, zero elsewhere, an identity tail on the padding diagonal: kFillPerBlock entries a workgroup, in the
+// launch of the records (a launch of its own, and one that wrote the solve's iteration count, were 15 us of a
+// four-iteration solve of 8 cameras in 485).
+constexpr int kFillPerBlock = 16 * kWG;
+__device__ __forceinline__ void fill_S(double* __restrict__ S, int n, int ld, const double* __restrict__ M, int block) {
+    const size_t end = std::min((size_t)ld * ld, (size_t)(block + 1) * kFillPerBlock);
+    for (size_t i = (size_t)block * kFillPerBlock + threadIdx.x; i < end; i += kWG) {
+        const int r = (int)(i / ld), c = (int)(i % ld);
+        double v = (r == c && r >= n) ? 1.0 : 0.0;
+        if (r < n && c < n && r / 9 == c / 9) v = M[81 * (size_t)(r / 9) + 9 * (r % 9) + c % 9];
+        S[i] = v;
+    }
+}
+
 // The pair products' records (kRecDense).  `parts` workgroups share a camera's observations: with one, 49
 // cameras of 640 observations leave most of the chip idle (28 us against 10.5).  Bound by the stores: by the
 // lanes that form the records, 48 us in FP64 and 32 in FP32 at 250 cameras and 1M observations, through LDS
 // 40 and 18.
 template <typename Real, int M>
-__global__ void __launch_bounds__(kWG, 4) k_dense_store(Dev<Real> d, Real* __restrict__ js, int parts) {
+__global__ void __launch_bounds__(kWG, 4) k_dense_store(Dev<Real> d, Real* __restrict__ js, int parts, int n_store,
+                                                        double* __restrict__ S, int n, int ld) {
     LMState* st = d.st;
     if (st->done || st->step_invalid) return;
     __shared__ Unit16 lds[kWaves][64 * kRecordRow];
     constexpr bool f64 = sizeof(Real) == 8;  // a record is two rows then, J~_c and the rest, else one
-    const int per_part = gridDim.x / parts, part = blockIdx.x / per_part;
+    if ((int)blockIdx.x >= n_store) {  // the workgroups after the records' fill S
+        fill_S(S, n, ld, d.M, (int)blockIdx.x - n_store);
+        return;
+    }
+    const int per_part = n_store / parts, part = blockIdx.x / per_part;
     const int c = xcd_remap(blockIdx.x - part * per_part, d.nc);
     if (c >= d.nc) return;
     const CameraPrep<Real> P = d.prep[c];
@@ -88,12 +108,12 @@ __global__ void __launch_bounds__(kWG, 4) k_dense_store(Dev<Real> d, Real* __res
             stage_pair<Real>(lds[wave], at + 7, ig[2], (Real)0);
             stage_pair<Real>(lds[wave], at + 8, (Real)0, (Real)0);
         }
-        const int n = min(64, end - j0);
+        const int rows = min(64, end - j0);
         Real* out = js + kJs * (size_t)j0;
-        if (f64) flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 9, n);
+        if (f64) flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 9, rows);
 #pragma unroll
         for (int i = 0; i < 9; ++i) stage_pair<Real>(lds[wave], i, Jc[i], Jc[9 + i]);  // the rows of column i adjacent
-        flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 0, n);
+        flush_records<kJs * (int)sizeof(Real) / 16, 9>(lds[wave], out, 0, rows);
     }
 }
 
@@ -165,18 +185,6 @@ __global__ void __launch_bounds__(kWG) k_pair_emit(const int* __restrict__ cam_o
             if (out + before + k < bk.w) pairs[out + before + k] = make_int2(i, first + k);
         out += total;
     }
-}
-
-// S <- the cameras' Schur-Jacobi blocks M_c (k_rhs_cam: D_c^2 plus every observation with itself) on the
-// diagonal, zero elsewhere, an identity tail on the padding diagonal.
-__global__ void k_fill_S(double* __restrict__ S, int n, int ld, const double* __restrict__ M, const LMState* st) {
-    if (st->done || st->step_invalid) return;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)ld * ld) return;
-    const int r = (int)(i / ld), c = (int)(i % ld);
-    double v = (r == c && r >= n) ? 1.0 : 0.0;
-    if (r < n && c < n && r / 9 == c / 9) v = M[81 * (size_t)(r / 9) + 9 * (r % 9) + c % 9];
-    S[i] = v;
 }
 
 // One 9x9 block of the reduced camera system per workgroup of NW waves (the blocks' pair lists, the
@@ -702,8 +710,9 @@ __global__ void __launch_bounds__(kWG) k_fwd_rows(const F* __restrict__ A, int l
 template <typename F>
 __global__ void __launch_bounds__(kWG) k_bwd_solve(const F* __restrict__ BinvT, int nt, int K, const double* __restrict__ y,
                                                    double* __restrict__ t, double* __restrict__ x, int n, int accumulate,
-                                                   const LMState* st) {
+                                                   int solves, LMState* st) {
     if (st->done || st->step_invalid) return;
+    if (K == 0 && blockIdx.x == 0 && threadIdx.x == 0) st->pcg_iters = solves;  // linear solver iterations
     const int rows = kTile * solve_block_tiles(K, nt), kb = kSolveRows * K;
     const int r0 = kSweepRows * (blockIdx.x * kWaves + (threadIdx.x >> 6));
     if (r0 >= rows) return;
@@ -765,11 +774,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_dense_small(const double* __r
     }
     small_backward<kSmallThreads, false>(small_lds, n);
     for (int k = threadIdx.x; k < n; k += kSmallThreads) x[k] = small_lds[tri(n) + k];
-}
-
-__global__ void k_set_linear_iters(LMState* st, int iters) {
-    if (st->done || st->step_invalid) return;
-    st->pcg_iters = iters;
+    if (threadIdx.x == 0) st->pcg_iters = 1;  // linear solver iterations
 }
 
 // Reduced systems up to this size are factored in FP64 in both precisions: the factor costs a few
@@ -916,7 +921,7 @@ struct DenseSchur {
         }
         for (int K = nb - 1; K >= 0; --K) {
             sv.launch("bwd_solve", k_bwd_solve<F>, div_up(kTile * solve_block_tiles(K, nt), per), kWG, BinvT, nt, K,
-                      (const double*)y.p, z.p, x, n, accumulate, st);
+                      (const double*)y.p, z.p, x, n, accumulate, 1 + refine, sv.d.st);
             if (K > 0)
                 sv.launch("bwd_rows", k_bwd_rows<F>, div_up(kSolveRows * K, per), kWG, A, ld, nt, K, (const double*)z.p, y.p, st);
         }
@@ -951,13 +956,12 @@ struct DenseSchur {
     void enqueue_solve(SolverT& sv) {
         auto& d = sv.d;
         const int nc = d.nc;
+        const size_t nn = (size_t)ld * ld;
+        const int n_store = xcd_grid(nc) * store_parts;
         sv.launch("dense_store",
                   pick_model(d.model, k_dense_store<Real, kModelSnavely>, k_dense_store<Real, kModelSnavelyG2o>,
                              k_dense_store<Real, kModelStereo>),
-                  xcd_grid(nc) * store_parts, kWG, d, js.p, store_parts);
-        const size_t nn = (size_t)ld * ld;
-        sv.launch("fill_S", k_fill_S, (int)((nn + 255) / 256), 256, S.p, n, ld, (const double*)d.M,
-                  (const LMState*)d.st);
+                  n_store + (int)((nn + kFillPerBlock - 1) / kFillPerBlock), kWG, d, js.p, store_parts, n_store, S.p, n, ld);
         if (schur_waves == 8)
             enqueue_schur<8>(sv);
         else
@@ -972,7 +976,6 @@ struct DenseSchur {
                       (const LMState*)d.st);
             factor_and_solve<float>(sv, Af.p, Dinvf.p, Binvf.p, BinvTf.p);
         }
-        sv.launch("set_iters", k_set_linear_iters, 1, 1, d.st, 1 + refine);
     }
 };
 
