@@ -525,15 +525,18 @@ __device__ __forceinline__ void corrected_jacobian(const Dev<Real>& d, const Cam
 // Linearization
 
 template <typename Real>
-__global__ void __launch_bounds__(64) k_cam_prep(Dev<Real> d) {
-    if (!d.st->need_lin) return;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= d.nc) return;
+__device__ __forceinline__ void cam_prep(const Dev<Real>& d, const double* __restrict__ cams, int c) {
     double cam[9];
-    for (int i = 0; i < 9; ++i) cam[i] = d.cam_x[(size_t)i * d.nc + c];
+    for (int i = 0; i < 9; ++i) cam[i] = cams[(size_t)i * d.nc + c];
     CameraPrep<Real> P;
     camera_prep<Real>(cam, P);
     d.prep[c] = P;
+}
+template <typename Real>
+__global__ void __launch_bounds__(64) k_cam_prep(Dev<Real> d) {
+    if (!d.st->need_lin) return;
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < d.nc) cam_prep<Real>(d, d.cam_x, c);
 }
 
 // One workgroup per camera: diag(Jc'Jc) and g_c = Jc'r (unscaled, corrected) -- the column norms
@@ -1512,15 +1515,60 @@ __global__ void __launch_bounds__(kWG) k_cam_update(Dev<Real> d, int it) {
     }
 }
 
+// One thread per camera: delta_c = -S_c y_c, candidate camera and its FP64 prep.
+template <typename Real, int M>
+__device__ __forceinline__ void cam_step(const Dev<Real>& d, int c) {
+    double cam[9], dx2 = 0.0, x2 = 0.0;
+    for (int i = 0; i < 9; ++i) {
+        const double dl = -d.sc[9 * (size_t)c + i] * d.px[9 * (size_t)c + i];
+        const double x = d.cam_x[(size_t)i * d.nc + c];
+        d.dcam[(size_t)i * d.nc + c] = dl;
+        cam[i] = x + dl;
+        dx2 += dl * dl;
+        x2 += x * x;
+    }
+    if constexpr (M == kModelStereo) {
+        // pose <- exp(xi) pose, xi = (rho, phi) in the first six slots
+        double xi[6], w[3], t[3];
+        for (int i = 0; i < 6; ++i) xi[i] = d.dcam[(size_t)i * d.nc + c];
+        for (int i = 0; i < 3; ++i) {
+            w[i] = d.cam_x[(size_t)i * d.nc + c];
+            t[i] = d.cam_x[(size_t)(3 + i) * d.nc + c];
+        }
+        se3_left_update(xi, w, t, cam, cam + 3);
+    } else if constexpr (M == kModelSnavelyG2o) {
+        // rotation <- exp(delta) rotation, read back as angle-axis
+        double dd[3], w[3];
+        for (int i = 0; i < 3; ++i) {
+            dd[i] = d.dcam[(size_t)i * d.nc + c];
+            w[i] = d.cam_x[(size_t)i * d.nc + c];
+        }
+        so3_left_update(dd, w, cam);
+    }
+    for (int i = 0; i < 9; ++i) d.cam_c[(size_t)i * d.nc + c] = cam[i];
+    CameraPrep<double> P;
+    camera_prep<double>(cam, P);
+    d.prep_c[c] = P;
+    d.cam_part[PS_DX2 * (size_t)d.nc + c] = dx2;
+    d.cam_part[PS_X2 * (size_t)d.nc + c] = x2;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Step, candidate and decision
 
 // One workgroup per chunk: y_p = Vinv S_p sum u_j (u_j = Jp'(r~ - Jc S_c y_c)),
 // delta_p = -S_p y_p, candidate = x + delta.
-template <typename Real>
-__global__ void __launch_bounds__(kWG) k_pt_backsub(Dev<Real> d) {
+// The workgroups after the first n_pt take 64 cameras' candidates each: both wait only for the camera step and the
+// slot vectors, and a launch of its own for the cameras cost 6 us an iteration.
+template <typename Real, int M>
+__global__ void __launch_bounds__(kWG) k_backsub(Dev<Real> d, int n_pt) {
     LMState* st = d.st;
     if (st->done || st->step_invalid) return;
+    if ((int)blockIdx.x >= n_pt) {
+        const int c = ((int)blockIdx.x - n_pt) * 64 + (int)threadIdx.x;
+        if (threadIdx.x < 64 && c < d.nc) cam_step<Real, M>(d, c);
+        return;
+    }
     __shared__ double lds[(kWaves - 1) * 3 * 64];
     const int ch = xcd_remap(blockIdx.x, d.n_chunks);
     if (ch >= d.n_chunks) return;
@@ -1560,48 +1608,6 @@ __global__ void __launch_bounds__(kWG) k_pt_backsub(Dev<Real> d) {
         d.pt_part[PS_DX2 * (size_t)d.n_pt_blocks + ch] = dx2;
         d.pt_part[PS_X2 * (size_t)d.n_pt_blocks + ch] = x2;
     }
-}
-
-// One thread per camera: delta_c = -S_c y_c, candidate camera and its FP64 prep.
-template <typename Real, int M>
-__global__ void __launch_bounds__(64) k_cam_step(Dev<Real> d) {
-    LMState* st = d.st;
-    if (st->done || st->step_invalid) return;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= d.nc) return;
-    double cam[9], dx2 = 0.0, x2 = 0.0;
-    for (int i = 0; i < 9; ++i) {
-        const double dl = -d.sc[9 * (size_t)c + i] * d.px[9 * (size_t)c + i];
-        const double x = d.cam_x[(size_t)i * d.nc + c];
-        d.dcam[(size_t)i * d.nc + c] = dl;
-        cam[i] = x + dl;
-        dx2 += dl * dl;
-        x2 += x * x;
-    }
-    if constexpr (M == kModelStereo) {
-        // pose <- exp(xi) pose, xi = (rho, phi) in the first six slots
-        double xi[6], w[3], t[3];
-        for (int i = 0; i < 6; ++i) xi[i] = d.dcam[(size_t)i * d.nc + c];
-        for (int i = 0; i < 3; ++i) {
-            w[i] = d.cam_x[(size_t)i * d.nc + c];
-            t[i] = d.cam_x[(size_t)(3 + i) * d.nc + c];
-        }
-        se3_left_update(xi, w, t, cam, cam + 3);
-    } else if constexpr (M == kModelSnavelyG2o) {
-        // rotation <- exp(delta) rotation, read back as angle-axis
-        double dd[3], w[3];
-        for (int i = 0; i < 3; ++i) {
-            dd[i] = d.dcam[(size_t)i * d.nc + c];
-            w[i] = d.cam_x[(size_t)i * d.nc + c];
-        }
-        so3_left_update(dd, w, cam);
-    }
-    for (int i = 0; i < 9; ++i) d.cam_c[(size_t)i * d.nc + c] = cam[i];
-    CameraPrep<double> P;
-    camera_prep<double>(cam, P);
-    d.prep_c[c] = P;
-    d.cam_part[PS_DX2 * (size_t)d.nc + c] = dx2;
-    d.cam_part[PS_X2 * (size_t)d.nc + c] = x2;
 }
 
 // One WG per camera: model cost change -(J~ s).(r~ + J~ s / 2) with J, r at x (working
@@ -1792,9 +1798,16 @@ __global__ void __launch_bounds__(kWG) k_decide(Dev<Real> d) {
 }
 
 // Accepted step: x <- candidate (cameras then points, one thread per parameter).
+// An accepted step: the candidate becomes the parameters (workgroups of the first n_copy), and the next
+// linearization's camera preps, from the candidate (the others, 64 cameras each).
 template <typename Real>
-__global__ void __launch_bounds__(kWG) k_apply(Dev<Real> d) {
+__global__ void __launch_bounds__(kWG) k_apply(Dev<Real> d, int n_copy) {
     if (!d.st->accepted) return;
+    if ((int)blockIdx.x >= n_copy) {
+        const int c = ((int)blockIdx.x - n_copy) * 64 + (int)threadIdx.x;
+        if (d.st->need_lin && threadIdx.x < 64 && c < d.nc) cam_prep<Real>(d, d.cam_c, c);
+        return;
+    }
     const size_t i = (size_t)blockIdx.x * kWG + threadIdx.x;
     const size_t ncam = 9 * (size_t)d.nc, npt = 4 * (size_t)d.np;
     if (i < ncam) d.cam_x[i] = d.cam_c[i];

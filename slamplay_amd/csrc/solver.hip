@@ -523,9 +523,9 @@ struct Solver final : SolverBase {
         launch_shm(name, kernel, grid, block, 0, args...);
     }
 
+    // (the camera preps are formed: by the step that was applied, or at the start)
     void enqueue_linearize() {
-        const int nc = L.nc, gpt = xcd_grid(d.n_pt_blocks), gcam = xcd_grid(nc);
-        launch("cam_prep", k_cam_prep<Real>, div_up(nc, 64), 64, d);
+        const int gpt = xcd_grid(d.n_pt_blocks), gcam = xcd_grid(L.nc);
         launch("lin_cam", BA_MODEL_KERNEL(k_lin_cam), gcam, kWG, d);
         launch("lin_pt", k_lin_pt<Real>, gpt, kWG, d);
     }
@@ -560,11 +560,11 @@ struct Solver final : SolverBase {
                 launch("jtx", BA_MODEL_KERNEL(k_jtx), gcam, kWG, d, 1, opt.pcg_max_iterations + 1, (const double*)d.pp);
         }
         launch("jtx_y", BA_MODEL_KERNEL(k_jtx), gcam, kWG, d, 0, 0, (const double*)d.px);
-        launch("pt_backsub", k_pt_backsub<Real>, gpt, kWG, d);
-        launch("cam_step", BA_MODEL_KERNEL(k_cam_step), div_up(nc, 64), 64, d);
+        launch("pt_backsub", BA_MODEL_KERNEL(k_backsub), gpt + div_up(nc, 64), kWG, d, gpt);
         launch("model_cand", BA_MODEL_KERNEL(k_model_cand), gcam, kWG, d);
         launch("decide", k_decide<Real>, 1, kWG, d);
-        launch("apply", k_apply<Real>, div_up(9 * (int64_t)nc + 4 * (int64_t)np, kWG), kWG, d);
+        const int copies = div_up(9 * (int64_t)nc + 4 * (int64_t)np, kWG);
+        launch("apply", k_apply<Real>, copies + div_up(nc, 64), kWG, d, copies);
         enqueue_linearize();
         launch("post_lin", k_post_lin<Real>, 1, kWG, d);
     }
@@ -607,6 +607,7 @@ struct Solver final : SolverBase {
             if (summary) fill_empty(summary);
             return BA_OK;
         }
+        launch("cam_prep", k_cam_prep<Real>, div_up(nc, 64), 64, d);
         enqueue_linearize();
         launch("prep_x", k_prep_from<Real>, div_up(nc, 64), 64, d, (const double*)d.cam_x);
         launch("cost_x", BA_MODEL_KERNEL(k_cost_cam), xcd_grid(nc), kWG, d, (const double*)d.pt_x);
