@@ -955,6 +955,7 @@ struct Batch final : BatchBase {
     // copies, waits and host permutations of 38 us each.)
     int download(int w, double* cams, double* pts) override {
         if (w < 0 || w >= (int)imgs.size()) return fail(BA_ERR_INVALID_ARGUMENT, "window %d out of range", w);
+        std::lock_guard<std::mutex> lock(download_mutex);  // threads may read their windows side by side
         if (large_index[w] >= 0) return large_solvers[large_index[w]]->download(cams, pts);
         if (downloads++ == 0) return lanes[lane_of[w]]->download(w, imgs[w].pt_perm, cams, pts);
         if (!fetched) BA_TRY(fetch_all());
@@ -973,6 +974,7 @@ struct Batch final : BatchBase {
     DevBuf<double> dparams;
     std::vector<double> host_params;
     int64_t n_params = 0;
+    std::mutex download_mutex;
     int downloads = 0;     // since the parameters last changed
     bool fetched = false;  // host_params holds them
 

@@ -1,5 +1,7 @@
 """Batch results read one window at a time (the first download after a change fetches its window alone,
 later ones a packed copy of all): every order of reading gives the parameters the batch holds now."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -43,4 +45,20 @@ def test_batch_downloads_follow_the_parameters(sizes):
     b.reset()
     for w in some:
         same(b.download(w), start[w])  # not the fetched solution
+    b.close()
+
+
+# windows of the batched kernels beside one of the single-problem solver (36 cameras)
+def test_batch_downloads_from_several_threads():
+    probs = [S.synthetic(4, seed=i + 1, num_cameras=c, num_points=60 + i, max_track=min(c, 6))
+             for i, c in enumerate([5, 36, 8, 6, 7, 5, 36, 9])]
+    start = [(p.cameras().copy(), p.points().copy()) for p in probs]
+    b = S.Batch(probs, **FIXED)
+    b.run()
+    b.reset()
+    with ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(b.download, range(len(probs))))
+    for x, y in zip(got, start):
+        np.testing.assert_array_equal(x[0], y[0])
+        np.testing.assert_array_equal(x[1], y[1])
     b.close()
