@@ -1797,9 +1797,9 @@ __global__ void __launch_bounds__(kWG) k_decide(Dev<Real> d) {
         lm_finish(st, BA_CONVERGENCE, BA_REASON_MIN_RADIUS, st->radius);
 }
 
-// Accepted step: x <- candidate (cameras then points, one thread per parameter).
-// An accepted step: the candidate becomes the parameters (workgroups of the first n_copy), and the next
-// linearization's camera preps, from the candidate (the others, 64 cameras each).
+// Accepted step: x <- candidate (the first n_copy workgroups: cameras then points, one thread per parameter), and
+// the next linearization's camera preps from the candidate (the others, 64 cameras each; a launch of its own kept
+// one workgroup's worth of cameras 4.6 us an iteration).
 template <typename Real>
 __global__ void __launch_bounds__(kWG) k_apply(Dev<Real> d, int n_copy) {
     if (!d.st->accepted) return;
