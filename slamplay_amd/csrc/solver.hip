@@ -484,6 +484,7 @@ struct Solver final : SolverBase {
     // against staging vectors and a permutation on the host.
     int download(double* cams, double* pts) override {
         const int nc = L.nc, np = L.np;
+        BA_TRY(use_device(device));  // a launch, unlike a copy, needs the stream's device to be the thread's current one
         hipLaunchKernelGGL(k_params_out, dim3(std::max(1, div_up(std::max(9 * (int64_t)nc, 3 * (int64_t)np), kWG))), dim3(kWG),
                            0, s, (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, dcam.p, dpt.p);
         BA_HIP(hipGetLastError());
