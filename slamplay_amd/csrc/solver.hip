@@ -263,6 +263,7 @@ struct Solver final : SolverBase {
     DevBuf<LMState> st;
     DevBuf<ba_iteration> trace;
     DevBuf<int> pt_orig;  // internal point -> caller point
+    DevBuf<double> params_out;  // download: cameras and points in the caller's layout
     PrepScratch prep_w;
     LMState* st_host = nullptr;  // pinned
     double wait_timeout_s = 0.0;
@@ -293,7 +294,7 @@ struct Solver final : SolverBase {
         int64_t b = 0;
         b += cam_off.bytes() + co_pt.bytes() + chunk_off.bytes() + chunk_len.bytes() + slot_of.bytes();
         b += co_uv64.bytes() + co_uvr.bytes() + co_rec.bytes();
-        b += cam_x.bytes() * 4 + pt_x.bytes() * 4 + dcam.bytes() + dpt.bytes();
+        b += cam_x.bytes() * 4 + pt_x.bytes() * 4 + dcam.bytes() + dpt.bytes() + params_out.bytes();
         b += prep.bytes() + prep_c.bytes();
         b += M.bytes() * 2 + gc.bytes() * 10 + upd_part.bytes() + rz_hist.bytes() + dp2.bytes();
         b += V.bytes() + gp.bytes() + sp.bytes() + Vinv64.bytes();
@@ -349,6 +350,7 @@ struct Solver final : SolverBase {
         BA_TRY(pt_c.alloc(4 * (size_t)np));
         BA_TRY(dcam.alloc(9 * (size_t)nc));
         BA_TRY(dpt.alloc(4 * (size_t)np));
+        BA_TRY(params_out.alloc(9 * (size_t)nc + 3 * (size_t)np));
         BA_TRY(prep.alloc(nc));
         BA_TRY(prep_c.alloc(nc));
         for (DevBuf<double>* b : {&M, &Minv}) BA_TRY(b->alloc(81 * (size_t)nc));
@@ -479,17 +481,19 @@ struct Solver final : SolverBase {
         return BA_OK;
     }
 
-    // The caller's layouts are formed on the device (into the step buffers, which hold nothing between
-    // runs) and copied straight into the caller's arrays: 370 -> 200 us for 1,500 cameras and 100k points,
-    // against staging vectors and a permutation on the host.
+    // The caller's layouts are formed on the device and copied straight into the caller's arrays: 370 -> 200 us for
+    // 1,500 cameras and 100k points, against staging vectors and a permutation on the host.  They have a
+    // buffer of their own: another thread may run the solver meanwhile, and the step buffers are in use between
+    // the launches of an iteration.
     int download(double* cams, double* pts) override {
         const int nc = L.nc, np = L.np;
         BA_TRY(use_device(device));  // a launch, unlike a copy, needs the stream's device to be the thread's current one
+        double *const out_c = params_out.p, *const out_p = params_out.p + 9 * (size_t)nc;
         hipLaunchKernelGGL(k_params_out, dim3(std::max(1, div_up(std::max(9 * (int64_t)nc, 3 * (int64_t)np), kWG))), dim3(kWG),
-                           0, s, (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, dcam.p, dpt.p);
+                           0, s, (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, out_c, out_p);
         BA_HIP(hipGetLastError());
-        if (cams && nc) BA_HIP(hipMemcpyAsync(cams, dcam.p, 9 * (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, s));
-        if (pts && np) BA_HIP(hipMemcpyAsync(pts, dpt.p, 3 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (cams && nc) BA_HIP(hipMemcpyAsync(cams, out_c, 9 * (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (pts && np) BA_HIP(hipMemcpyAsync(pts, out_p, 3 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, s));
         BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }
