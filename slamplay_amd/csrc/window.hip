@@ -260,22 +260,19 @@ __global__ void __launch_bounds__(256) k_window_place(const char* __restrict__ s
         dst[i] = i < n_in ? src[i] : make_uint4(0, 0, 0, 0);
 }
 
-// The windows' parameters in the caller's order, packed: 9 K camera values, then 3 P point values at
-// out_off; inv holds each window's internal index of every caller point.
+// The parameters of windows in the caller's order, packed, one workgroup each: 9 K camera values, then 3 P
+// point values at out_off; inv holds each window's internal index of every caller point.
 struct PackTask {
-    int slot, K, P, pad;
+    const double *cam_x, *pt_x;
     int64_t inv_off, out_off;
+    int K, P;
 };
-__global__ void __launch_bounds__(256) k_window_pack(const WinDesc* __restrict__ descs, char* __restrict__ arena,
-                                                     const PackTask* __restrict__ tasks, const int* __restrict__ inv,
+__global__ void __launch_bounds__(256) k_window_pack(const PackTask* __restrict__ tasks, const int* __restrict__ inv,
                                                      double* __restrict__ out) {
     const PackTask t = tasks[blockIdx.x];
-    const WinDesc D = descs[t.slot];
-    const double* cx = at<double>(arena, D.o_cam_x);
-    const double* px = at<double>(arena, D.o_pt_x);
     double* o = out + t.out_off;
-    for (int k = threadIdx.x; k < 9 * t.K; k += 256) o[k] = cx[k];
-    for (int e = threadIdx.x; e < 3 * t.P; e += 256) o[9 * t.K + e] = px[4 * (size_t)inv[t.inv_off + e / 3] + e % 3];
+    for (int k = threadIdx.x; k < 9 * t.K; k += 256) o[k] = t.cam_x[k];
+    for (int e = threadIdx.x; e < 3 * t.P; e += 256) o[9 * t.K + e] = t.pt_x[4 * (size_t)inv[t.inv_off + e / 3] + e % 3];
 }
 
 // Gathers the LM states of the listed windows into out (one thread per window).
@@ -649,6 +646,8 @@ struct BatchBase {
     virtual int run(ba_summary* summaries) = 0;
     virtual int reset() = 0;
     virtual int download(int w, double* cams, double* pts) = 0;
+    // Every window will be downloaded before the parameters change again.
+    virtual void expect_all() = 0;
     virtual int set_threads(int t) = 0;
     virtual void info(int* threads, int64_t* bytes) = 0;
     virtual int get_schedule(ba_batch_schedule* out) = 0;
@@ -949,58 +948,112 @@ struct Batch final : BatchBase {
         return BA_OK;
     }
 
-    // The first download after the windows' parameters changed fetches its window alone; the second
-    // one, so a caller that reads several, fetches all of them packed by one kernel per lane, and
-    // later ones read that copy until the parameters change again.  (512 windows one by one: 19.3 ms of
-    // copies, waits and host permutations of 38 us each.)
+    // A window read alone costs 37 us of copies, a wait and a permutation on the host; one of a range that one
+    // kernel packs costs 1.6 us (26 KB), so kPackedPerRead of them are fetched at the price of one read
+    // alone.  A caller may read one window or all of them, so what is fetched ahead grows with what has been
+    // read: after two reads, as long as every window fetched ahead has been read since, kAheadPerRead
+    // windows for each read so far come with the next one, in the direction of reading (a third more than the
+    // reads alone, should the caller stop there); and in whatever order, once the windows read alone have cost as
+    // much as all the remaining ones would, these come with the next.  512 windows: two of them 75 us, 64 at random
+    // 1.9 ms (2.3 one by one), all in order 3.3 ms, all at random 3.8 (18.6).  With all fetched by the second read
+    // two took 840 us, all 3.1 ms.
+    static constexpr int kPackedPerRead = 20;
+    static constexpr int kAheadPerRead = 8;
+
     int download(int w, double* cams, double* pts) override {
         if (w < 0 || w >= (int)imgs.size()) return fail(BA_ERR_INVALID_ARGUMENT, "window %d out of range", w);
         std::lock_guard<std::mutex> lock(download_mutex);  // threads may read their windows side by side
         if (large_index[w] >= 0) return large_solvers[large_index[w]]->download(cams, pts);
-        if (downloads++ == 0) return lanes[lane_of[w]]->download(w, imgs[w].pt_perm, cams, pts);
-        if (!fetched) BA_TRY(fetch_all());
+        if (held[w] < kUnread) {
+            const int n = (int)imgs.size();
+            int want = 1;
+            if (alone * (int64_t)kPackedPerRead >= untouched)
+                want = n;
+            else if (reads >= 2 && unread == 0)
+                want = (int)std::min<int64_t>(n, (int64_t)kAheadPerRead * reads);
+            const bool down = last_alone > w;
+            last_alone = w;
+            if (want == 1 || !can_pack()) {
+                ++alone;
+                ++reads;
+                if (held[w] == kNone) --untouched;
+                held[w] = kAlone;
+                return lanes[lane_of[w]]->download(w, imgs[w].pt_perm, cams, pts);
+            }
+            const int first = want == n ? 0 : down ? std::max(0, w - want + 1) : w;
+            BA_TRY(fetch(first, want == n ? n : down ? w + 1 : std::min(n, w + want)));
+        }
+        ++reads;
+        if (held[w] == kUnread) {
+            held[w] = kRead;
+            --unread;
+        }
         const double* src = host_params.data() + pack[pack_of[w]].out_off;
         if (cams) std::copy(src, src + 9 * (size_t)imgs[w].K, cams);
         if (pts) std::copy(src + 9 * (size_t)imgs[w].K, src + 9 * (size_t)imgs[w].K + 3 * (size_t)imgs[w].P, pts);
         return BA_OK;
     }
 
-    // Results on the host: the pack tasks lane after lane (lane l's are [pack_first[l], pack_first[l + 1])).
+    // Results on the host: a task for each batched window, in the windows' order.
     std::vector<PackTask> pack;
-    std::vector<int> pack_of;  // window -> its task
-    std::vector<size_t> pack_first;
+    std::vector<int> pack_of;  // window -> its task, or that of the next batched window (one entry more than windows)
     DevBuf<PackTask> dpack;
     DevBuf<int> dinv;
     DevBuf<double> dparams;
     std::vector<double> host_params;
     int64_t n_params = 0;
     std::mutex download_mutex;
-    int downloads = 0;     // since the parameters last changed
-    bool fetched = false;  // host_params holds them
+    // since the parameters last changed:
+    enum : char { kNone, kAlone, kUnread, kRead };  // never read, read alone; in host_params, not read from there or read
+    std::vector<char> held;      // per window
+    int untouched = 0, unread = 0;  // windows in kNone, in kUnread
+    int64_t alone = 0, reads = 0;   // reads of a window alone; all reads
+    int last_alone = -1;            // the window of the last read that host_params could not answer
 
     void params_changed() {
-        downloads = 0;
-        fetched = false;
+        std::lock_guard<std::mutex> lock(download_mutex);
+        held.assign(imgs.size(), kNone);
+        untouched = (int)pack.size();
+        unread = 0;
+        alone = reads = 0;
+        last_alone = -1;
+    }
+
+    void expect_all() override {
+        std::lock_guard<std::mutex> lock(download_mutex);
+        if (pack.size() > 1) alone = (int64_t)pack.size();  // the first read fetches all
+    }
+
+    // Room for the packed copies; without it every window is read alone.
+    bool can_pack() {
+        if (use_device(opt.device) != BA_OK) return false;
+        if (!dparams.p && dparams.alloc((size_t)n_params) != BA_OK) {
+            (void)hipGetLastError();
+            clear_error();
+        }
+        return dparams.p != nullptr;
     }
 
     int prepare_packing() {
         pack.clear();
-        pack_of.assign(imgs.size(), -1);
-        pack_first.assign(1, 0);
-        std::vector<int> inv;
+        pack_of.clear();
         n_params = 0;
-        for (const auto& order : lane_order) {
-            for (int w : order) {
-                const WindowImage& im = imgs[w];
-                pack_of[w] = (int)pack.size();
-                pack.push_back(PackTask{w, im.K, im.P, 0, (int64_t)inv.size(), n_params});
-                n_params += 9 * (int64_t)im.K + 3 * (int64_t)im.P;
-                const size_t o = inv.size();
-                inv.resize(o + im.P);
-                for (int ip = 0; ip < im.P; ++ip) inv[o + im.pt_perm[ip]] = ip;
-            }
-            pack_first.push_back(pack.size());
+        std::vector<int> inv;
+        for (size_t w = 0; w < imgs.size(); ++w) {
+            pack_of.push_back((int)pack.size());
+            if (lane_of[w] < 0) continue;
+            const WindowImage& im = imgs[w];
+            const WindowEngine<Real>& e = *lanes[lane_of[w]];
+            pack.push_back(PackTask{reinterpret_cast<const double*>(e.arena.p + e.hdesc[w].o_cam_x),
+                                    reinterpret_cast<const double*>(e.arena.p + e.hdesc[w].o_pt_x), (int64_t)inv.size(), n_params,
+                                    im.K, im.P});
+            n_params += 9 * (int64_t)im.K + 3 * (int64_t)im.P;
+            const size_t o = inv.size();
+            inv.resize(o + im.P);
+            for (int ip = 0; ip < im.P; ++ip) inv[o + im.pt_perm[ip]] = ip;
         }
+        pack_of.push_back((int)pack.size());
+        params_changed();
         if (pack.empty()) return BA_OK;
         hipStream_t s = lanes[0]->s;
         BA_TRY(dpack.upload(pack.data(), pack.size(), s));
@@ -1009,21 +1062,33 @@ struct Batch final : BatchBase {
         return BA_OK;
     }
 
-    int fetch_all() {
-        BA_TRY(use_device(opt.device));
-        if (!dparams.p) BA_TRY(dparams.alloc((size_t)n_params));
+    // The batched windows of [first, end) into host_params (after can_pack).
+    int fetch(int first, int end) {
         host_params.resize((size_t)n_params);
-        for (size_t l = 0; l < lanes.size(); ++l) {
-            const size_t n = pack_first[l + 1] - pack_first[l];
-            if (n)
-                hipLaunchKernelGGL(k_window_pack, dim3((unsigned)n), dim3(256), 0, lanes[l]->s, (const WinDesc*)lanes[l]->ddesc.p,
-                                   lanes[l]->arena.p, (const PackTask*)dpack.p + pack_first[l], (const int*)dinv.p, dparams.p);
-        }
+        // the lanes are idle between runs; one that an error left busy is waited for
+        for (auto& e : lanes)
+            if (hipStreamQuery(e->s) != hipSuccess) {
+                (void)hipGetLastError();  // "not ready" is no error here
+                BA_TRY(e->sync("window results"));
+            }
+        const int t0 = pack_of[first], t1 = pack_of[end];
+        const int64_t p0 = pack[t0].out_off, p1 = t1 < (int)pack.size() ? pack[t1].out_off : n_params;
+        hipStream_t s = lanes[0]->s;
+        hipLaunchKernelGGL(k_window_pack, dim3((unsigned)(t1 - t0)), dim3(256), 0, s, (const PackTask*)dpack.p + t0,
+                           (const int*)dinv.p, dparams.p);
         BA_HIP(hipGetLastError());
-        for (auto& e : lanes) BA_TRY(e->sync("window results"));
-        BA_HIP(hipMemcpyAsync(host_params.data(), dparams.p, (size_t)n_params * sizeof(double), hipMemcpyDeviceToHost, lanes[0]->s));
+        BA_HIP(hipMemcpyAsync(host_params.data() + p0, dparams.p + p0, (size_t)(p1 - p0) * sizeof(double), hipMemcpyDeviceToHost, s));
         BA_TRY(lanes[0]->sync("window results"));
-        fetched = true;
+        for (int w = first; w < end; ++w)
+            if (lane_of[w] >= 0 && held[w] < kUnread) {
+                if (held[w] == kNone) {
+                    --untouched;
+                    ++unread;
+                    held[w] = kUnread;
+                } else {
+                    held[w] = kRead;
+                }
+            }
         return BA_OK;
     }
 };
@@ -1738,6 +1803,7 @@ int ba_batch_solve(const ba_problem_view* windows, int32_t count, const ba_optio
     BA_TRY(ba_batch_create(windows, count, options, &b));
     std::unique_ptr<ba_batch> guard(b);
     BA_TRY(b->impl->run(summaries));
+    b->impl->expect_all();
     for (int w = 0; w < count; ++w) BA_TRY(b->impl->download(w, windows[w].cameras, windows[w].points));
     return BA_OK;
 }
@@ -1766,6 +1832,7 @@ int ba_stereo_batch_solve(const ba_stereo_view* windows, int32_t count, const ba
     std::unique_ptr<BatchBase> b;
     BA_TRY(make_batch(views.data(), count, o, &b, in.data(), false));
     BA_TRY(b->run(summaries));
+    b->expect_all();
     for (int w = 0; w < count; ++w) {
         BA_TRY(b->download(w, sp[w].cams.data(), windows[w].points));
         stereo_finish(&windows[w], sp[w], o.loss_scale, outliers ? outliers[w] : nullptr,

@@ -1,5 +1,6 @@
 """Batch results read one window at a time (the first download after a change fetches its window alone,
 later ones a packed copy of all): every order of reading gives the parameters the batch holds now."""
+import time
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -62,3 +63,54 @@ def test_batch_downloads_from_several_threads():
         np.testing.assert_array_equal(x[0], y[0])
         np.testing.assert_array_equal(x[1], y[1])
     b.close()
+
+
+def _orders(n):
+    rng = np.random.default_rng(n)
+    yield "up", list(range(n))
+    yield "down", list(range(n))[::-1]
+    yield "every third", list(range(0, n, 3))
+    yield "a few, then up", [n - 1, 0, n // 2] + list(range(n))
+    yield "random", list(rng.permutation(n))
+    yield "random, repeated", list(rng.integers(0, n, 3 * n))
+    yield "one again and again", [n // 3] * (n + 4)
+    yield "down from the middle, then up", list(range(n // 2, -1, -1)) + list(range(n))
+
+
+# how many windows come with a read depends on what was read before (from the third read on, eight for each
+# read so far; all, once the reads of one window have cost as much)
+@pytest.mark.parametrize("n", [1, 2, 3, 20, 45, 130])
+def test_batch_downloads_in_any_order(n):
+    # every eighth window is solved by the single-problem solver (36 cameras)
+    probs = [S.synthetic(4, seed=i + 1, num_cameras=36 if i % 8 == 5 else 5 + i % 3, num_points=40 + i % 70, max_track=5)
+             for i in range(n)]
+    b = S.Batch(probs, **FIXED)
+    b.run()
+    ref = [b.download(w) for w in range(n)]
+    for name, order in _orders(n):
+        b.reset()
+        b.run()
+        for w in order:
+            got = b.download(w)
+            np.testing.assert_array_equal(got[0], ref[w][0], err_msg=f"{name}: window {w}")
+            np.testing.assert_array_equal(got[1], ref[w][1], err_msg=f"{name}: window {w}")
+    b.close()
+
+
+def test_reading_two_windows_does_not_fetch_all():
+    b = S.Batch(S.local_ba_windows(256, seed=2), max_num_iterations=1)
+
+    def median_ms(windows):
+        t = []
+        for _ in range(15):
+            b.reset()
+            start = time.perf_counter()
+            for w in windows:
+                b.download(w)
+            t.append(time.perf_counter() - start)
+        return 1e3 * float(np.median(t))
+
+    one, two = median_ms([3]), median_ms([3, 200])
+    b.close()
+    # two reads of one window each are twice one; all 256 would be more than ten times
+    assert two < 5 * one, (one, two)
