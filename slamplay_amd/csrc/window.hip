@@ -872,6 +872,8 @@ struct Batch final : BatchBase {
         if (bytes) {
             *bytes = 0;
             for (auto& e : lanes) *bytes += e->arena_cap;
+            std::lock_guard<std::mutex> lock(download_mutex);
+            *bytes += (int64_t)(dpack.bytes() + dinv.bytes() + dparams.bytes());
         }
     }
 

@@ -114,3 +114,13 @@ def test_reading_two_windows_does_not_fetch_all():
     b.close()
     # two reads of one window each are twice one; all 256 would be more than ten times
     assert two < 5 * one, (one, two)
+
+
+def test_info_counts_the_packed_copy():
+    b = S.Batch([S.synthetic(4, seed=i + 1, num_cameras=5, num_points=40, max_track=5) for i in range(4)], **FIXED)
+    before = b.info()["device_bytes"]
+    for w in range(4):
+        b.download(w)
+    values = 4 * (9 * 5 + 3 * 40)
+    assert b.info()["device_bytes"] >= before + 8 * values
+    b.close()
