@@ -18,9 +18,9 @@ struct DeviceParams {
 
 // Scratch owned by the caller's handle, grown on demand and kept between calls.
 struct PrepScratch {
-    DevBuf<unsigned long long> sel_state;  // 4 selections x (key, rank)
-    DevBuf<unsigned int> hist;             // digit counts of the four selections' two passes, collected keys
-    DevBuf<unsigned long long> keys;       // keys that share a selection's first digits (three selections at once)
+    DevBuf<unsigned long long> sel_state;  // 4 selections x 7 states, then their keys and ranges
+    DevBuf<unsigned int> hist;             // digit counts of the passes' four selections, collected keys
+    DevBuf<unsigned long long> keys;       // keys that share a selection's digits so far (three selections at once)
     DevBuf<unsigned int> draws;            // glibc rand() outputs
     DevBuf<unsigned int> tables;           // jump-ahead matrices
     DevBuf<unsigned int> counts;           // accepted pairs per block, then their exclusive scan

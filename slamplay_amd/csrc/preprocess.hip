@@ -320,15 +320,31 @@ __global__ void k_perturb_cams(double* __restrict__ cam, int nc, const double* _
 // ---------------------------------------------------------------------------------------------
 // Upper median (nth_element at n/2, BALProblem.cpp:71-76) by radix selection over the IEEE bit
 // patterns mapped to order-preserving keys, from the top.  Selection k: 0..2 a point axis, 3 the L1
-// distances.  Two histograms of 11 bits over all keys (every block picks the digits found so far from
-// the previous counts itself, so a pass is one launch), then the keys that share those 22 bits -- a
-// thousandth of the range around the median, a few hundred of 100,000 -- are collected and one block
-// finishes on them (on all keys, if all are alike).  Bound by launches, 5 us each: four a selection, 43 us
-// for both selections of 100,000 points; eight passes of eight bits, with a launch each to pick the
-// digit, took 93 us.
+// distances.  Histograms of 11 bits over all keys (every block picks the digit found last from the previous
+// counts itself, so a pass is one launch), then the keys that share the digits so far are collected and one
+// block finishes on them.  Two histograms leave a thousandth of the range around the median, a few hundred of
+// 100,000 points in general position; bound by launches, 5 us each, both selections take 60 us with the wait
+// for them (eight passes of eight bits, with a launch each to pick the digit: 113).  But a map may lie in a
+// plane or far from the origin: most keys share 22 bits then, and the one block has them all.  At 100,000 points it
+// takes 65 us so for a plane and 122 for a map a thousand extents away; what it takes grows with the points,
+// so beyond kSelSpread four more histograms, which return at once when at most kSelCap keys are left, take the
+// digits down to the last over the whole chip: a million points in a plane 152 us, in general position 118
+// (eight passes 190 and 173; with all keys left to a block of 256 threads 4,900, and 446 for the plane of 100,000).
 constexpr int kSelBits = 11;
 constexpr int kSelBins = 1 << kSelBits;
-constexpr int kSelShift0 = 64 - kSelBits, kSelShift1 = kSelShift0 - kSelBits;
+constexpr int kSelPasses = 6;            // digits of a key: five of kSelBits, one of the last nine bits
+constexpr int kSelSpread = 1 << 17;
+constexpr unsigned int kSelCap = 1 << 14;
+constexpr int kFinishBlock = 1024;
+constexpr int kFinishList = 4096;        // keys the last block keeps in LDS
+
+// A selection with its first `bits` bits found: they are the prefix's, `count` keys share them and the one looked
+// for has rank `rank` among these.
+struct SelState {
+    unsigned long long prefix, rank;
+    unsigned int count, bits;
+};
+
 __device__ __forceinline__ unsigned long long order_key(double x) {
     const unsigned long long u = (unsigned long long)__double_as_longlong(x);
     return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
@@ -339,19 +355,23 @@ __device__ __forceinline__ double key_value(unsigned long long k) {
     return __longlong_as_double((long long)u);
 }
 
-// hist: [selection][pass 0, 1][kSelBins]; count: collected keys per selection
-__global__ void __launch_bounds__(256) k_sel_init(unsigned int* __restrict__ hist, unsigned int* __restrict__ count) {
+// hist: [pass][selection][kSelBins], n words in all; count: collected keys per selection, range: the smallest and
+// the largest of them
+__global__ void __launch_bounds__(256) k_sel_init(unsigned int* __restrict__ hist, int n, unsigned int* __restrict__ count,
+                                                  unsigned long long* __restrict__ range) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < 4 * 2 * kSelBins) hist[i] = 0;
+    if (i < n) hist[i] = 0;
     if (i < 4) count[i] = 0;
+    if (i < 8) range[i] = i & 1 ? 0 : ~0ull;
 }
 
-// The bin of counts h (kSelBins of them) that holds rank *r, by a block of 256 threads: its number is
-// returned in every thread and *r becomes the rank inside it.
-__device__ __forceinline__ unsigned int sel_pick(const unsigned int* __restrict__ h, unsigned long long* r) {
-    constexpr int per = kSelBins / 256;
-    __shared__ unsigned long long wsum[4], rank_in;
-    __shared__ unsigned int digit;
+// The bin of counts h (kSelBins of them) that holds rank *rank, by a block of NT threads: its number is returned
+// in every thread, *rank becomes the rank inside it and *count its count.
+template <int NT>
+__device__ __forceinline__ unsigned int sel_pick(const unsigned int* __restrict__ h, unsigned long long* rank, unsigned int* count) {
+    constexpr int per = kSelBins / NT, waves = NT / 64;
+    __shared__ unsigned long long wsum[waves], rank_in;
+    __shared__ unsigned int digit, count_in;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     unsigned int v[per];
     unsigned long long x = 0;
@@ -371,16 +391,36 @@ __device__ __forceinline__ unsigned int sel_pick(const unsigned int* __restrict_
     __syncthreads();
     unsigned long long excl = x - own;
     for (int w = 0; w < wave; ++w) excl += wsum[w];
-    if (excl <= *r && *r < excl + own) {
-        unsigned long long left = *r - excl;
+    if (excl <= *rank && *rank < excl + own) {
+        unsigned long long left = *rank - excl;
         int i = 0;
         while (i + 1 < per && left >= v[i]) left -= v[i++];
         digit = per * t + i;
+        count_in = v[i];
         rank_in = left;
     }
     __syncthreads();
-    *r = rank_in;
+    *rank = rank_in;
+    *count = count_in;
     return digit;
+}
+
+// Few enough keys are left for one block (the first two digits are always taken by the whole chip).
+__device__ __forceinline__ bool sel_small(const SelState& s) { return s.bits >= 2 * kSelBits && s.count <= kSelCap; }
+
+// Selection k as pass `pass` finds it: the state its predecessor left, with the digit that one counted.
+// Block 0 leaves it for the next pass.
+__device__ __forceinline__ SelState sel_state(SelState* __restrict__ states, const unsigned int* __restrict__ hist, int k, int pass,
+                                              int np, bool first_block) {
+    SelState s{0, (unsigned long long)(np / 2), (unsigned int)np, 0};
+    if (pass > 1) s = states[(kSelPasses + 1) * k + pass - 1];
+    if (pass > 0 && !sel_small(s)) {
+        const unsigned int digit = sel_pick<kSelBlock>(hist + (size_t)(4 * (pass - 1) + k) * kSelBins, &s.rank, &s.count);
+        s.bits = min(64u, s.bits + kSelBits);
+        s.prefix |= (unsigned long long)digit << (64 - s.bits);
+    }
+    if (pass > 0 && first_block && threadIdx.x == 0) states[(kSelPasses + 1) * k + pass] = s;
+    return s;
 }
 
 // BALProblem.cpp:274-281: L1 distance of a point to the per-axis medians
@@ -388,79 +428,235 @@ __device__ __forceinline__ double norm_dist(const double* __restrict__ p, const 
     return fabs(p[0] - m[0]) + fabs(p[1] - m[1]) + fabs(p[2] - m[2]);
 }
 
-// Pass 0 or 1 of selections first .. first + gridDim.y - 1, or (PASS 2) the collection of the keys that
-// share both digits.  sel[k] receives the selection's key so far and its rank among the collected ones.
-// Selection 3 forms the distances from the points and the medians in sel[0..2].
-template <int PASS>
-__global__ void __launch_bounds__(kSelBlock) k_sel_pass(const double* __restrict__ pt, int np, int first,
-                                                        unsigned long long* __restrict__ sel, unsigned int* __restrict__ hist,
-                                                        unsigned int* __restrict__ count, unsigned long long* __restrict__ keys) {
-    __shared__ unsigned int h[PASS < 2 ? kSelBins : 1];
+// The key of point i in selection k: its coordinate on axis k, or its distance to the medians m.
+__device__ __forceinline__ unsigned long long sel_key(const double* __restrict__ pt, int i, int k, const double m[3]) {
+    const double* p = pt + 4 * (int64_t)i;
+    return order_key(k < 3 ? p[k] : norm_dist(p, m));
+}
+
+// A round of kSelRound keys of a block: thread t has those of points i0 + t, i0 + kSelBlock + t, ... below np, all
+// loads in flight together (past the last point its key again).
+constexpr int kSelUnroll = 8;
+constexpr int kSelRound = kSelUnroll * kSelBlock;
+__device__ __forceinline__ void sel_round(const double* __restrict__ pt, int64_t i0, int np, int k, const double m[3],
+                                          unsigned long long (&key)[kSelUnroll]) {
+#pragma unroll
+    for (int u = 0; u < kSelUnroll; ++u)
+        key[u] = sel_key(pt, (int)min(i0 + u * kSelBlock + (int)threadIdx.x, (int64_t)np - 1), k, m);
+}
+
+// Counts of digit `pass` of selections first .. first + gridDim.y - 1.  Selection 3 forms the distances from
+// the points and the medians, the found keys 0..2.
+__global__ void __launch_bounds__(kSelBlock) k_sel_hist(const double* __restrict__ pt, int np, int first, int pass,
+                                                        const unsigned long long* __restrict__ found, SelState* __restrict__ states,
+                                                        unsigned int* __restrict__ hist) {
+    __shared__ unsigned int h[kSelBins];
     const int k = first + (int)blockIdx.y, t = threadIdx.x;
-    unsigned int* hk = hist + 2 * kSelBins * k;
+    const SelState s = sel_state(states, hist, k, pass, np, blockIdx.x == 0);
+    if (sel_small(s)) return;  // the same in every thread
     double m[3] = {0.0, 0.0, 0.0};
     if (k == 3)
-        for (int j = 0; j < 3; ++j) m[j] = key_value(sel[2 * j]);
-    unsigned long long rank = (unsigned long long)(np / 2), prefix = 0;
-    if (PASS < 2)
-        for (int i = t; i < kSelBins; i += kSelBlock) h[i] = 0;
-    if (PASS >= 1) prefix = (unsigned long long)sel_pick(hk, &rank) << kSelShift0;
-    if (PASS >= 2) prefix |= (unsigned long long)sel_pick(hk + kSelBins, &rank) << kSelShift1;
+        for (int j = 0; j < 3; ++j) m[j] = key_value(found[j]);
+    for (int i = t; i < kSelBins; i += kSelBlock) h[i] = 0;
     __syncthreads();
-    if (PASS == 2 && blockIdx.x == 0 && t == 0) {
-        sel[2 * k] = prefix;
-        sel[2 * k + 1] = rank;
+    const int top = 64 - (int)s.bits, shift = max(0, top - kSelBits);  // bits [shift, top) of the keys
+    const unsigned int mask = (1u << (top - shift)) - 1;
+    for (int64_t i0 = (int64_t)blockIdx.x * kSelRound; i0 < np; i0 += (int64_t)gridDim.x * kSelRound) {
+        unsigned long long key[kSelUnroll];
+        sel_round(pt, i0, np, k, m, key);
+#pragma unroll
+        for (int u = 0; u < kSelUnroll; ++u)
+            if (i0 + u * kSelBlock + t < np && (pass == 0 || ((key[u] ^ s.prefix) >> top) == 0))
+                atomicAdd(&h[(unsigned int)(key[u] >> shift) & mask], 1u);
     }
-    const int shift = PASS == 0 ? kSelShift0 : kSelShift1;
-    for (int i = blockIdx.x * kSelBlock + t; i < np; i += gridDim.x * kSelBlock) {
-        const double* p = pt + 4 * (int64_t)i;
-        const unsigned long long key = order_key(k < 3 ? p[k] : norm_dist(p, m));
-        if (PASS == 0) {
-            atomicAdd(&h[key >> kSelShift0], 1u);
-        } else if (PASS == 1) {
-            if ((key >> kSelShift0) == (prefix >> kSelShift0)) atomicAdd(&h[(key >> shift) & (kSelBins - 1)], 1u);
-        } else if ((key >> kSelShift1) == (prefix >> kSelShift1)) {
-            keys[(size_t)(k % 3) * np + atomicAdd(&count[k], 1u)] = key;
+    __syncthreads();
+    // integer counts: the sum does not depend on the order the blocks add in
+    unsigned int* out = hist + (size_t)(4 * pass + k) * kSelBins;
+    for (int i = t; i < kSelBins; i += kSelBlock)
+        if (h[i]) atomicAdd(&out[i], h[i]);
+}
+
+// After `passes` histograms: the keys that share the digits so far (at most `stride`: all points, or kSelCap after
+// all the passes) and their range.  None when the digits are the whole key.  A block reserves the places of a
+// round's keys with one addition, as all of them may be collected.
+__global__ void __launch_bounds__(kSelBlock) k_sel_collect(const double* __restrict__ pt, int np, int first, int passes,
+                                                           const unsigned long long* __restrict__ found,
+                                                           SelState* __restrict__ states, const unsigned int* __restrict__ hist,
+                                                           unsigned int* __restrict__ count,
+                                                           unsigned long long* __restrict__ range,
+                                                           unsigned long long* __restrict__ keys, int stride) {
+    constexpr int NW = kSelBlock / 64;
+    __shared__ unsigned int wave_n[NW], base;
+    const int k = first + (int)blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const SelState s = sel_state(states, hist, k, passes, np, blockIdx.x == 0);
+    if (s.bits == 64) return;  // the same in every thread
+    double m[3] = {0.0, 0.0, 0.0};
+    if (k == 3)
+        for (int j = 0; j < 3; ++j) m[j] = key_value(found[j]);
+    const int top = 64 - (int)s.bits;
+    unsigned long long lo = ~0ull, hi = 0;
+    for (int64_t i0 = (int64_t)blockIdx.x * kSelRound; i0 < np; i0 += (int64_t)gridDim.x * kSelRound) {
+        unsigned long long key[kSelUnroll], here[kSelUnroll];
+        sel_round(pt, i0, np, k, m, key);
+        unsigned int n = 0;  // the wave's keys
+#pragma unroll
+        for (int u = 0; u < kSelUnroll; ++u) {
+            here[u] = __ballot(i0 + u * kSelBlock + t < np && ((key[u] ^ s.prefix) >> top) == 0);
+            n += (unsigned int)__popcll(here[u]);
         }
-    }
-    if (PASS < 2) {
+        if (lane == 0) wave_n[wave] = n;
         __syncthreads();
-        // integer counts: the sum does not depend on the order the blocks add in
-        for (int i = t; i < kSelBins; i += kSelBlock)
-            if (h[i]) atomicAdd(&hk[PASS * kSelBins + i], h[i]);
+        if (t == 0) {
+            unsigned int all = 0;
+            for (int w = 0; w < NW; ++w) all += wave_n[w];
+            base = all ? atomicAdd(&count[k], all) : 0;
+        }
+        __syncthreads();
+        unsigned int at = base;
+        for (int w = 0; w < wave; ++w) at += wave_n[w];
+        if (n)
+#pragma unroll
+            for (int u = 0; u < kSelUnroll; ++u) {
+                if ((here[u] >> lane) & 1) {
+                    keys[(size_t)(k % 3) * stride + at + __popcll(here[u] & ((1ull << lane) - 1))] = key[u];
+                    lo = min(lo, key[u]);
+                    hi = max(hi, key[u]);
+                }
+                at += (unsigned int)__popcll(here[u]);
+            }
+        __syncthreads();  // wave_n and base have been read
+    }
+    if (__ballot(lo <= hi) == 0) return;  // most waves have none
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        lo = min(lo, __shfl_xor(lo, d, 64));
+        hi = max(hi, __shfl_xor(hi, d, 64));
+    }
+    if (lane == 0) {
+        atomicMin(&range[2 * k], lo);
+        atomicMax(&range[2 * k + 1], hi);
     }
 }
 
-// The remaining bits over the collected keys, one block per selection; their order does not matter.
-__global__ void __launch_bounds__(256) k_sel_finish(int np, int first, unsigned long long* __restrict__ sel,
-                                                    const unsigned int* __restrict__ count,
-                                                    const unsigned long long* __restrict__ keys) {
-    __shared__ unsigned int h[kSelBins];
-    const int k = first + (int)blockIdx.x, t = threadIdx.x;
-    const unsigned int n = count[k];
-    const unsigned long long* mine = keys + (size_t)(k % 3) * np;
-    unsigned long long prefix = sel[2 * k], rank = sel[2 * k + 1];
-    for (int top = kSelShift1; top > 0; top -= kSelBits) {  // bits [shift, top) of the keys
-        const int shift = top > kSelBits ? top - kSelBits : 0;
-        for (int i = t; i < kSelBins; i += 256) h[i] = 0;
-        __syncthreads();
-        for (unsigned int i = t; i < n; i += 256) {
-            const unsigned long long key = mine[i];
-            if ((key >> top) == (prefix >> top)) atomicAdd(&h[(key >> shift) & ((1ull << (top - shift)) - 1)], 1u);
+// The key of rank `rank` of the n collected ones at `mine`, which lie in [lo, hi], lo < hi, by NT threads.  From the
+// first bit they differ in, a histogram of kSelBits bits, and again on the keys of its bin, which are kept in
+// `list` once they are few; ended when they are one value.
+template <int NT>
+__device__ __forceinline__ unsigned long long sel_last_bits(const unsigned long long* __restrict__ mine, int n, unsigned long long rank,
+                                                            unsigned long long lo, unsigned long long hi, unsigned int* h,
+                                                            unsigned long long* list) {
+    constexpr int U = 8, NW = NT / 64;
+    __shared__ unsigned int listed;
+    __shared__ unsigned long long and_w[NW], or_w[NW];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int top = 64 - __clzll((long long)(lo ^ hi));  // at most 42: the keys share the passes' digits
+    unsigned long long prefix = lo >> top << top;
+    bool in_lds = false;
+    // f(key without the prefix) for every key that has it
+    auto each_key = [&](auto f) {
+        if (in_lds) {
+            for (int i = t; i < n; i += NT) {
+                const unsigned long long x = list[i] ^ prefix;
+                if (x < 1ull << top) f(x);
+            }
+            return;
+        }
+        for (int i0 = 0; i0 < n; i0 += U * NT) {
+            unsigned long long x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = mine[min(i0 + u * NT + t, n - 1)] ^ prefix;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * NT + t < n && x[u] < 1ull << top) f(x[u]);
+        }
+    };
+    for (unsigned int left = (unsigned int)n;;) {
+        for (int i = t; i < kSelBins; i += NT) h[i] = 0;
+        if (!in_lds && left <= kFinishList) {
+            if (t == 0) listed = 0;
+            __syncthreads();
+            each_key([&](unsigned long long x) {
+                const unsigned long long here = __ballot(1);
+                const int leader = __ffsll(here) - 1;
+                unsigned int at = 0;
+                if (lane == leader) at = atomicAdd(&listed, (unsigned int)__popcll(here));
+                list[__shfl(at, leader, 64) + __popcll(here & ((1ull << lane) - 1))] = x ^ prefix;
+            });
+            in_lds = true;
+            n = (int)left;
         }
         __syncthreads();
-        prefix |= (unsigned long long)sel_pick(h, &rank) << shift;
+        const int shift = max(0, top - kSelBits);
+        unsigned long long all_and = ~0ull, all_or = 0;
+        each_key([&](unsigned long long x) {
+            all_and &= x;
+            all_or |= x;
+            const unsigned int bin = (unsigned int)(x >> shift), bin0 = __builtin_amdgcn_readfirstlane(bin);
+            const unsigned long long same = __ballot(bin == bin0);
+            if (bin != bin0)
+                atomicAdd(&h[bin], 1u);
+            else if (lane == __ffsll(same) - 1)
+                atomicAdd(&h[bin], (unsigned int)__popcll(same));
+        });
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            all_and &= __shfl_xor(all_and, d, 64);
+            all_or |= __shfl_xor(all_or, d, 64);
+        }
+        if (lane == 0) {
+            and_w[wave] = all_and;
+            or_w[wave] = all_or;
+        }
+        __syncthreads();
+        for (int w = 0; w < NW; ++w) {
+            all_and &= and_w[w];
+            all_or |= or_w[w];
+        }
+        if (all_and == all_or) return prefix | all_or;  // one value; the same in every thread
+        prefix |= (unsigned long long)sel_pick<NT>(h, &rank, &left) << shift;
+        top = shift;
+        if (top == 0) return prefix;
         __syncthreads();
     }
-    if (t == 0) sel[2 * k] = prefix;
+}
+
+// The remaining bits over the collected keys, one block per selection; their order does not matter.  A few hundred
+// keys are work for four waves, whose barriers cost less than sixteen's.  With all of 100,000 keys collected it
+// is bound by one CU's instructions, hence all its threads, eight loads a thread in flight, and the lanes of a
+// wave whose key falls into its first lane's bin, often all of them, counted by one addition: 60 us (340 with a quarter
+// of the threads, a load at a time and an addition a key).
+__global__ void __launch_bounds__(kFinishBlock) k_sel_finish(int first, int passes, const SelState* __restrict__ states,
+                                                             const unsigned int* __restrict__ count,
+                                                             const unsigned long long* __restrict__ range,
+                                                             const unsigned long long* __restrict__ keys, int stride,
+                                                             unsigned long long* __restrict__ found) {
+    __shared__ unsigned int h[kSelBins];
+    __shared__ unsigned long long list[kFinishList];
+    const int k = first + (int)blockIdx.x;
+    const SelState s = states[(kSelPasses + 1) * k + passes];
+    const int n = (int)count[k];
+    const unsigned long long lo = range[2 * k], hi = range[2 * k + 1];
+    const unsigned long long* mine = keys + (size_t)(k % 3) * stride;
+    unsigned long long key;
+    if (s.bits == 64) {
+        key = s.prefix;
+    } else if (lo == hi) {
+        key = lo;
+    } else if (n <= kFinishList) {
+        if (threadIdx.x >= kSelBlock) return;
+        key = sel_last_bits<kSelBlock>(mine, n, s.rank, lo, hi, h, list);
+    } else {
+        key = sel_last_bits<kFinishBlock>(mine, n, s.rank, lo, hi, h, list);
+    }
+    if (threadIdx.x == 0) found[k] = key;
 }
 
 // BALProblem.cpp:283-302: X <- s (X - m), camera centres likewise, s = 100 / MAD
 __global__ void k_norm_apply(double* __restrict__ pt, int np, double* __restrict__ cam, int nc,
-                             const unsigned long long* __restrict__ sel) {
+                             const unsigned long long* __restrict__ found) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const double m[3] = {key_value(sel[0]), key_value(sel[2]), key_value(sel[4])};
-    const double scale = 100.0 / key_value(sel[6]);
+    const double m[3] = {key_value(found[0]), key_value(found[1]), key_value(found[2])};
+    const double scale = 100.0 / key_value(found[3]);
     if (i < np)
         for (int j = 0; j < 3; ++j) pt[4 * (int64_t)i + j] = scale * (pt[4 * (int64_t)i + j] - m[j]);
     if (i < nc) {
@@ -490,24 +686,30 @@ int device_normalize(const DeviceParams& p, PrepScratch* w, hipStream_t s) {
     if (p.np == 0) return BA_OK;  // BALProblem.cpp:263-303 leaves an empty problem as it is
     const int np = p.np;
     const int nblocks = std::max(1, std::min(256, div_up(np, kSelBlock * 8)));
-    BA_TRY(ensure(w->sel_state, 8));
-    BA_TRY(ensure(w->hist, (size_t)4 * 2 * kSelBins + 4));
-    BA_TRY(ensure(w->keys, 3 * (size_t)np));
-    unsigned int* count = w->hist.p + 4 * 2 * kSelBins;
-    hipLaunchKernelGGL(k_sel_init, dim3(4 * 2 * kSelBins / 256), dim3(256), 0, s, w->hist.p, count);
+    const int passes = np > kSelSpread ? kSelPasses : 2;
+    const int words = 4 * passes * kSelBins, stride = np > kSelSpread ? (int)kSelCap : np;
+    constexpr int kStateWords = sizeof(SelState) / sizeof(unsigned long long) * 4 * (kSelPasses + 1);
+    BA_TRY(ensure(w->sel_state, kStateWords + 12));
+    BA_TRY(ensure(w->hist, (size_t)words + 4));
+    BA_TRY(ensure(w->keys, 3 * (size_t)stride));
+    unsigned int* count = w->hist.p + words;
+    SelState* states = reinterpret_cast<SelState*>(w->sel_state.p);
+    unsigned long long *found = w->sel_state.p + kStateWords, *range = found + 4;
+    hipLaunchKernelGGL(k_sel_init, dim3(words / 256), dim3(256), 0, s, w->hist.p, words, count, range);
     for (int first : {0, 3}) {  // the axes together, then the distances to their medians
         const int n = first == 0 ? 3 : 1;
-        hipLaunchKernelGGL(k_sel_pass<0>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
-                           count, w->keys.p);
-        hipLaunchKernelGGL(k_sel_pass<1>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
-                           count, w->keys.p);
-        hipLaunchKernelGGL(k_sel_pass<2>, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, w->sel_state.p, w->hist.p,
-                           count, w->keys.p);
-        hipLaunchKernelGGL(k_sel_finish, dim3(n), dim3(256), 0, s, np, first, w->sel_state.p, (const unsigned int*)count,
-                           (const unsigned long long*)w->keys.p);
+        for (int pass = 0; pass < passes; ++pass)
+            hipLaunchKernelGGL(k_sel_hist, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, pass,
+                               (const unsigned long long*)found, states, w->hist.p);
+        hipLaunchKernelGGL(k_sel_collect, dim3(nblocks, n), dim3(kSelBlock), 0, s, p.pt, np, first, passes,
+                           (const unsigned long long*)found, states, (const unsigned int*)w->hist.p, count, range, w->keys.p,
+                           stride);
+        hipLaunchKernelGGL(k_sel_finish, dim3(n), dim3(kFinishBlock), 0, s, first, passes, (const SelState*)states,
+                           (const unsigned int*)count, (const unsigned long long*)range, (const unsigned long long*)w->keys.p, stride,
+                           found);
     }
     hipLaunchKernelGGL(k_norm_apply, dim3(div_up(std::max(np, p.nc), 256)), dim3(256), 0, s, p.pt, np, p.cam, p.nc,
-                       w->sel_state.p);
+                       (const unsigned long long*)found);
     BA_HIP(hipGetLastError());
     return BA_OK;
 }
