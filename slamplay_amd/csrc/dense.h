@@ -304,17 +304,17 @@ constexpr size_t step_pair_lds() {
 // Factors the 64 x 64 diagonal block of tiles t, t + 1 from its tiles T00, T11 (rows of kTile + 1) and T10
 // (kLdsPitch) in LDS; X is one tile more.  Leaves X_t and X_t+1 in Dinv and L_t+1,t in the lower tile (t + 1, t),
 // transposed also in the upper one.  All kStepThreads threads call it, before a barrier on the tiles; all
-// but the first wave run idle() while that factors tile t.
+// but the first wave run idle() while that factors tile t.  A pivot that fails sets step_invalid to `mark`.
 template <typename F, typename Idle>
 __device__ __forceinline__ void factor_pair(F* T00, F* T10, F* T11, F* X, F* __restrict__ A, int ld, int t,
-                                            F* __restrict__ Dinv, LMState* st, Idle idle) {
+                                            F* __restrict__ Dinv, LMState* st, int mark, Idle idle) {
     constexpr int PP = kLdsPitch<F>;
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, si = (w >> 1) & 1, sj = w & 1;
     lds_barrier();
     if (w > 0)
         idle();
     else if (!potrf_tile_wave<F>(T00, X, PP) && l == 0)
-        st->step_invalid = 1;
+        st->step_invalid = mark;
     lds_barrier();
     F* L = T00;  // L_t+1,t takes its place, rows of kLdsPitch
     if (w < 4) {
@@ -345,7 +345,7 @@ __device__ __forceinline__ void factor_pair(F* T00, F* T10, F* T11, F* X, F* __r
         for (int e = 0; e < 4; ++e) mine[Mfma<F>::row(l, e) * (kTile + 1)] = c[e];
     }
     lds_barrier();
-    if (w == 0 && !potrf_tile_wave<F>(T11, Dinv + (size_t)(t + 1) * kTile * kTile, kTile) && l == 0) st->step_invalid = 1;
+    if (w == 0 && !potrf_tile_wave<F>(T11, Dinv + (size_t)(t + 1) * kTile * kTile, kTile) && l == 0) st->step_invalid = mark;
 }
 
 // The first diagonal block (later ones are factored by the trailing update).
@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(kStepThreads) k_potrf_pair(F* __restrict__ A, 
         T10[a * kLdsPitch<F> + b] = A[(size_t)(kTile + a) * ld + b];
         T11[a * (kTile + 1) + b] = A[(size_t)(kTile + a) * ld + kTile + b];
     }
-    factor_pair<F>(T00, T10, T11, lds + 3 * kLdsTile<F>, A, ld, 0, Dinv, st, [] {});
+    factor_pair<F>(T00, T10, T11, lds + 3 * kLdsTile<F>, A, ld, 0, Dinv, st, 1, [] {});
 }
 
 // Step K of the factorization in one launch: tile columns k = 2 K and k + 1, one workgroup per lower 64 x 64
@@ -381,7 +381,10 @@ __global__ void __launch_bounds__(kStepThreads) k_potrf_pair(F* __restrict__ A, 
 template <typename F>
 __global__ void __launch_bounds__(kStepThreads, 4) k_step_pair(F* __restrict__ A, int ld, int K, F* __restrict__ Dinv,
                                                                LMState* st) {
-    if (st->done || st->step_invalid) return;
+    // Workgroup 0 may mark the step invalid while others start: the mark of this launch is left to later ones, so that
+    // every wave of a workgroup decides alike.
+    const int mark = K + 2, invalid = st->step_invalid;
+    if (st->done || (invalid != 0 && invalid != mark)) return;
     constexpr int PP = kLdsPitch<F>, TS = kLdsTile<F>;
     extern __shared__ __align__(16) unsigned char step_lds_mem[];
     F* const P = reinterpret_cast<F*>(step_lds_mem);  // tiles 0-3: L_.k of the rows of I, J; 4-7: L_.,k+1
@@ -504,7 +507,7 @@ __global__ void __launch_bounds__(kStepThreads, 4) k_step_pair(F* __restrict__ A
         c1 = load_block(1, 1, bi1, bj1);
     lds_barrier();
     if (w < 3) put(T00, kTile + 1, bi0, bj0, update_block(0, 0, bi0, bj0, c0));
-    factor_pair<F>(T00, T10, T11, P + 7 * TS, A, ld, k + 2, Dinv, st, [&] {
+    factor_pair<F>(T00, T10, T11, P + 7 * TS, A, ld, k + 2, Dinv, st, mark, [&] {
         if (w > 3)
             put(T10, PP, si, sj, update_block(1, 0, si, sj, c1));
         else

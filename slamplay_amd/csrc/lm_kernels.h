@@ -79,7 +79,7 @@ struct LMState {
     double step_norm, x_norm;
     double pcg_bb;
     int iteration, consecutive_invalid, done, termination;
-    int need_lin, first_lin, accepted, step_invalid;
+    int need_lin, first_lin, accepted, step_invalid;  // step_invalid: zero or not
     int num_successful, num_unsuccessful;
     int pcg_iters, pcg_done, total_pcg_iters, trace_len;
     int g2o_iter, g2o_trials;  // g2o mode: outer iterations done, rejected trials of the current one

@@ -52,3 +52,24 @@ def test_dense_pair_lists_match_oracle(oracle_mod, nc, repeats):
     # as above: at most 1e7 in condition times unit roundoff, per step
     assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-8 * ref["final_cost"]
     np.testing.assert_allclose(p.cameras(), ref["cams"], rtol=0, atol=1e-7 * np.abs(ref["cams"]).max())
+
+
+# A camera without observations and without damping: its pivots are exactly zero, in each step of the
+# factorization that its place can fall into.  Every step is refused, the parameters stay.
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("nc,unused", [(12, 5), (24, 23), (40, 0), (40, 9), (60, 31), (116, 110)])
+def test_dense_zero_pivots_refuse_the_step(oracle_mod, nc, unused, mixed):
+    p = S.synthetic(2, seed=nc, num_cameras=nc - 1, num_points=40 * nc, max_track=8)
+    ci = p.camera_index() + (p.camera_index() >= unused).astype(np.int32)
+    cams = np.insert(p.cameras().reshape(-1, 9), unused, p.cameras()[:9], axis=0)
+    q = S.BALProblem.from_arrays(ci, p.point_index(), p.observations().reshape(-1, 2), cams, p.points())
+    kw = dict(FIXED, max_num_iterations=20, min_lm_diagonal=1e-300, initial_trust_region_radius=1e60,
+              max_trust_region_radius=1e60)  # the damping of a zero column, 1e-360, is zero
+    ref = oracle_mod.solve(nc, q.num_points(), ci, p.point_index(), p.observations(), cams.reshape(-1), p.points(),
+                           oracle_mod.default_options(**kw))
+    assert not any(t["step_is_successful"] for t in ref["trace"][1:])
+    out = S.SolveBA(q, linear_solver=C.SOLVER_DENSE_SCHUR, precision=C.PRECISION_MIXED if mixed else C.PRECISION_FP64, **kw)
+    assert out["num_successful_steps"] == 0 and out["final_cost"] == out["initial_cost"]
+    assert len(out["trace"]) > 1 and not any(t["step_is_successful"] for t in out["trace"][1:])
+    np.testing.assert_array_equal(q.cameras(), cams.reshape(-1))
+    np.testing.assert_array_equal(q.points(), p.points())
