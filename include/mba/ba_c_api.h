@@ -283,7 +283,7 @@ int ba_solver_info(ba_solver* solver, int64_t* device_bytes, int32_t* linear_sol
  * state.  Every sum is formed in a fixed order, so a window's result does not depend on which other
  * windows share the launch nor on the schedule.  Windows compute in FP64 whatever options.precision
  * says (a reduced system of at most 288 unknowns is factored in FP64, as ba_solve does); it is
- * factored in the workgroup's LDS up to 21 cameras and in the window's own device buffer up to 32;
+ * factored in the workgroup's LDS up to 22 cameras and in the window's own device buffer up to 32;
  * larger windows are solved by the single-problem solver (ba_solver, with the requested precision)
  * and reported the same way. */
 typedef struct ba_batch ba_batch;
@@ -305,11 +305,11 @@ typedef struct ba_batch_schedule {
     int32_t solve_threads;       /* workgroup of the per-window factor and solve: 256 or 512 */
     int32_t blocks_per_wave;     /* 9x9 blocks of S per wave in one task of the Schur-product kernel: 1, 2, 4 or 8 */
     int32_t lds_cameras;         /* windows of at most this many cameras factor in LDS, larger ones in their device
-                                    buffer (capped at what the LDS holds, 21; the launch reserves the largest such
+                                    buffer (capped at what the LDS holds, 22; the launch reserves the largest such
                                     window's triangle for every workgroup) */
     int32_t candidates;          /* schedules the autotuner timed (0: set by the caller) */
     double iteration_ms;         /* one LM iteration of the batch with this schedule (0: not timed) */
-    double default_iteration_ms; /* the same with the default schedule 256 / 256 / 2 / 21 (0: not timed) */
+    double default_iteration_ms; /* the same with the default schedule 256 / 256 / 2 / 22 (0: not timed) */
     int32_t lanes;               /* output only: launch streams the windows are dealt to (largest work first, in
                                     turn) and run concurrently -- one per 32 windows, at most 4; the schedule
                                     applies to every lane and the timings are of all lanes launched together */

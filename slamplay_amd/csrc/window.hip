@@ -46,18 +46,31 @@ int64_t lds_per_block() {
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 
+// Static LDS of k_wsolve, by the compiled kernels (-1: not known).
+int64_t solve_static_lds() {
+    static const int64_t bytes = [] {
+        int64_t most = 0;
+        for (const void* kernel : {(const void*)k_wsolve<256>, (const void*)k_wsolve<512>}) {
+            hipFuncAttributes a{};
+            if (hipFuncGetAttributes(&a, kernel) != hipSuccess) {
+                (void)hipGetLastError();
+                return int64_t(-1);
+            }
+            most = std::max(most, (int64_t)a.sharedSizeBytes);
+        }
+        return most;
+    }();
+    return bytes;
+}
 
-// LDS of k_wsolve beside the packed triangle: its right-hand side row and flag, and room for alignment.
-int64_t solve_static_lds() { return 3 * kWinMaxN * 8 + 16 + 256; }
-
-// Largest reduced system (9 K) k_wsolve can factor in LDS (0: none).
+// Largest reduced system (9 K) k_wsolve can factor in LDS (0: none): its packed triangle with the right-hand side
+// row beside the static part.
 int max_window_n() {
+    if (solve_static_lds() < 0) return 0;
     const int64_t room = lds_per_block() - solve_static_lds();
-    if (room <= 0) return 0;
-    int n = (int)std::floor(std::sqrt(2.0 * (double)room / 8.0));  // packed: n (n + 1) / 2 doubles
-    while (n > 0 && (int64_t)n * (n + 1) / 2 * 8 > room) --n;
-    n = std::min(n, kWinMaxN);
-    return n - n % 9;
+    int n = kWinMaxN;
+    while (n > 0 && (int64_t)small_system_doubles(n) * 8 > room) n -= 9;
+    return n;
 }
 
 // Dynamic LDS of k_wschur: one staging area per wave.

@@ -406,3 +406,22 @@ def test_mixed_windows_38_final_cost(oracle_mod):
         ref = _oracle(oracle_mod, p, max_num_iterations=10, **FIXED)
         worst = max(worst, abs(s["final_cost"] - ref["final_cost"]) / ref["final_cost"])
     assert worst < 1e-6, worst
+
+
+def test_largest_windows_factored_in_lds():
+    """The packed triangle of 198 unknowns with its right-hand side row, 159,200 bytes, fits a workgroup's LDS beside
+    the kernel's own; 207 unknowns do not fit.  Where a window is factored does not change its bits."""
+    probs = [window(700 + k, k, 40 * k) for k in (20, 21, 22, 23)]
+    b = S.Batch(probs, precision=0, max_num_iterations=5)
+    b.set_schedule(256, 256, 2, 32)
+    assert b.schedule()["lds_cameras"] == 22
+    results = []
+    for threads, lds in ((256, 22), (512, 22), (256, 21), (256, 0)):
+        b.set_schedule(256, threads, 2, lds)
+        b.reset()
+        results.append((b.run(), [b.download(w) for w in range(len(probs))]))
+    for sums, params in results[1:]:
+        for w in range(len(probs)):
+            assert _same(sums[w], results[0][0][w])
+            np.testing.assert_array_equal(params[w][0], results[0][1][w][0])
+            np.testing.assert_array_equal(params[w][1], results[0][1][w][1])
