@@ -256,13 +256,16 @@ __global__ void k_window_reset(const WinDesc* __restrict__ descs, char* __restri
 }
 
 // Places the images of a lane's windows: window t's inputs from the staged copy into its region, the
-// rest of the region zeroed.  One upload and one launch per lane; a window used to take two copies and
-// a fill of its own, 20 us of runtime calls each (64 stereo windows: 4.5 ms).  gridDim.y workgroups per
+// rest of the region zeroed.  One upload and one launch for kStageBytes of inputs; a window used to take two copies
+// and a fill of its own, 20 us of runtime calls each (64 stereo windows: 4.5 ms).  gridDim.y workgroups per
 // window, 16 bytes per thread and turn (regions and staged inputs are 256-byte multiples).
 struct PlaceTask {
     int64_t src, dst, in_bytes, total;
 };
 constexpr int kPlaceSplit = 16;
+// The staged copy, on the host and on the device, is of so many windows' inputs at a time (or of one): a batch that
+// nearly fills the device needs no room for all of them again.
+constexpr int64_t kStageBytes = 64 << 20;
 __global__ void __launch_bounds__(256) k_window_place(const char* __restrict__ staged, char* __restrict__ arena,
                                                       const PlaceTask* __restrict__ tasks) {
     const PlaceTask t = tasks[blockIdx.x];
@@ -418,28 +421,45 @@ struct WindowEngine {
     int place_all(const std::vector<WindowImage>& imgs, const std::vector<int>& slots) {
         if (slots.empty()) return BA_OK;
         std::vector<PlaceTask> tasks;
-        int64_t base = 0, staged = 0;
+        int64_t base = 0, most = 0;
         for (int w : slots) {
             const int64_t in = (int64_t)imgs[w].bytes.size();
-            tasks.push_back(PlaceTask{staged, base, in, imgs[w].total});
+            tasks.push_back(PlaceTask{0, base, in, imgs[w].total});
             hdesc[w] = rebase(imgs[w].desc, base);
-            staged += in;
             base += imgs[w].total;
         }
         if (base > arena_cap) return fail(BA_ERR_CAPACITY, "windows do not fit the arena");
-        std::vector<char> host((size_t)staged);
-        for (size_t i = 0; i < slots.size(); ++i)
-            std::memcpy(host.data() + tasks[i].src, imgs[slots[i]].bytes.data(), (size_t)tasks[i].in_bytes);
+        std::vector<size_t> ends;  // of the groups that are staged together
+        int64_t staged = 0;
+        for (size_t i = 0; i < tasks.size(); ++i) {
+            if (staged > 0 && staged + tasks[i].in_bytes > kStageBytes) {
+                ends.push_back(i);
+                staged = 0;
+            }
+            tasks[i].src = staged;
+            staged += tasks[i].in_bytes;
+            most = std::max(most, staged);
+        }
+        ends.push_back(tasks.size());
+        std::vector<char> host((size_t)most);
         DevBuf<char> dstaged;
         DevBuf<PlaceTask> dtasks;
-        BA_TRY(dstaged.upload(host.data(), host.size(), s));
+        BA_TRY(dstaged.alloc((size_t)most));
         BA_TRY(dtasks.upload(tasks.data(), tasks.size(), s));
         BA_HIP(hipMemcpyAsync(ddesc.p, hdesc.data(), hdesc.size() * sizeof(WinDesc), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_window_place, dim3((unsigned)slots.size(), kPlaceSplit), dim3(256), 0, s, (const char*)dstaged.p,
-                           arena.p, (const PlaceTask*)dtasks.p);
-        BA_HIP(hipGetLastError());
+        size_t first = 0;
+        for (size_t end : ends) {
+            for (size_t i = first; i < end; ++i)
+                std::memcpy(host.data() + tasks[i].src, imgs[slots[i]].bytes.data(), (size_t)tasks[i].in_bytes);
+            const size_t bytes = (size_t)(tasks[end - 1].src + tasks[end - 1].in_bytes);
+            BA_HIP(hipMemcpyAsync(dstaged.p, host.data(), bytes, hipMemcpyHostToDevice, s));
+            hipLaunchKernelGGL(k_window_place, dim3((unsigned)(end - first), kPlaceSplit), dim3(256), 0, s, (const char*)dstaged.p,
+                               arena.p, (const PlaceTask*)dtasks.p + first);
+            BA_HIP(hipGetLastError());
+            BA_HIP(hipStreamSynchronize(s));
+            first = end;
+        }
         work_slots.clear();
-        BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }
 

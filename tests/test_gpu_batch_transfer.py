@@ -124,3 +124,24 @@ def test_info_counts_the_packed_copy():
     values = 4 * (9 * 5 + 3 * 40)
     assert b.info()["device_bytes"] >= before + 8 * values
     b.close()
+
+
+def test_windows_staged_in_several_groups():
+    """One lane's inputs beyond the 64 MB that are staged at a time (2.5 MB a window: 33,000 observations and their
+    pairs), a small window among them: every window is where and what it is in a batch of its own."""
+    probs = [S.synthetic(4, seed=i + 1, num_cameras=20, num_points=3000, max_track=20) for i in range(44)]
+    probs[25] = S.synthetic(4, seed=99, num_cameras=5, num_points=40, max_track=5)
+    start = [(p.cameras().copy(), p.points().copy()) for p in probs]
+    b = S.Batch(probs, **FIXED)
+    assert b.schedule()["lanes"] == 1
+    for w in range(len(probs)):
+        np.testing.assert_array_equal(b.download(w)[0], start[w][0])
+        np.testing.assert_array_equal(b.download(w)[1], start[w][1])
+    b.run()
+    for w in (0, 24, 25, 26, 43):
+        one = S.Batch(probs[w:w + 1], **FIXED)
+        one.run()
+        np.testing.assert_array_equal(b.download(w)[0], one.download(0)[0])
+        np.testing.assert_array_equal(b.download(w)[1], one.download(0)[1])
+        one.close()
+    b.close()
