@@ -55,9 +55,10 @@ __device__ __forceinline__ void fill_S(double* __restrict__ S, int n, int ld, co
 // The pair products' records (kRecDense).  `parts` workgroups share a camera's observations: with one, 49
 // cameras of 640 observations leave most of the chip idle (28 us against 10.5).  Bound by the stores: by the
 // lanes that form the records, 48 us in FP64 and 32 in FP32 at 250 cameras and 1M observations, through LDS
-// 40 and 18.
+// 40 and 18.  FP64 is held to three wavefronts a SIMD, not four: the g2o model's 134 registers then stay
+// registers (10.0 us at 49 cameras, 10.5 with six of 128 spilled); the others need no more than 128.
 template <typename Real, int M>
-__global__ void __launch_bounds__(kWG, 4) k_dense_store(Dev<Real> d, Real* __restrict__ js, int parts, int n_store,
+__global__ void __launch_bounds__(kWG, sizeof(Real) == 8 ? 3 : 4) k_dense_store(Dev<Real> d, Real* __restrict__ js, int parts, int n_store,
                                                         double* __restrict__ S, int n, int ld) {
     LMState* st = d.st;
     if (st->done || st->step_invalid) return;

@@ -436,9 +436,10 @@ __global__ void __launch_bounds__(NT) k_wdamp(const WinDesc* __restrict__ descs,
 }
 
 // Per (window, camera): records of the reduced system and b_c.  Bound by the records' stores, 256 bytes an
-// observation, which go through LDS (56 -> 47 us a launch of 32 windows).
+// observation, which go through LDS (56 -> 47 us a launch of 32 windows).  Three wavefronts a SIMD: at 166 registers
+// nothing is spilled; four, at 128 and 14 spilled, took 122 us instead of 102 in the launches of 512 windows.
 template <typename Real, int NT, int M>
-__global__ void __launch_bounds__(NT, 4) k_wrec_cam(const WinDesc* __restrict__ descs, char* __restrict__ arena,
+__global__ void __launch_bounds__(NT, 3) k_wrec_cam(const WinDesc* __restrict__ descs, char* __restrict__ arena,
                                                  const int2* __restrict__ ctask, int ntask, Opts o) {
     constexpr int NW = NT / 64;
     __shared__ double lds[9 * NW];
