@@ -55,8 +55,10 @@ __device__ __forceinline__ void spread_rows(double v, double* lo, double* hi) {
 }
 
 // acc += (lane LANE of each row of b) * x, one instruction.  The assembler form is needed because the
-// compiler does not fold a row broadcast into a multiply-add; b must have been written at least two
-// instructions earlier, which row_operands_ready guarantees.
+// compiler does not fold a row broadcast into a multiply-add.  b must have been written at least two
+// wait states earlier: row_operands_ready gives them to the values as they are formed; the compiler, which does
+// not know that the assembler form reads b by DPP, could only break it by copying b in between, and
+// tests/test_code_objects.py looks for that in the compiled kernels.
 template <int LANE>
 __device__ __forceinline__ void fma_row_lane(double& acc, double b, double x) {
     asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(x), "n"(LANE));
