@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 FIXED = dict(max_num_iterations=3, function_tolerance=0.0, gradient_tolerance=0.0, parameter_tolerance=0.0)
 
 
-# 9 nc unknowns: 27 (1 tile), 36, 63 (2 tiles), 180, 189, 198 (6 and 7 tiles), 288 (9 exact), 297,
-# 513 (17 tiles: block 2 of one tile), 1026 (33 tiles: block 3 of one tile)
+# 9 nc unknowns: 27, 36, 63, 180, 189, 198 (one workgroup, tiles of 32 columns), 288 and 297 (64 x 64 blocks: 4 and a
+# half, and a little more), 513 and 1026 (one and two 512-row blocks of the sweeps and the first of another)
 @pytest.mark.parametrize("nc", [3, 4, 7, 20, 21, 22, 32, 33, 57, 114])
 def test_dense_sizes_match_oracle(oracle_mod, nc):
     p = S.synthetic(2, seed=nc, num_cameras=nc, num_points=40 * nc, max_track=min(8, nc))
@@ -73,3 +73,38 @@ def test_dense_zero_pivots_refuse_the_step(oracle_mod, nc, unused, mixed):
     assert len(out["trace"]) > 1 and not any(t["step_is_successful"] for t in out["trace"][1:])
     np.testing.assert_array_equal(q.cameras(), cams.reshape(-1))
     np.testing.assert_array_equal(q.points(), p.points())
+
+
+def _against_oracle(oracle_mod, nc, mixed, **kw):
+    p = S.synthetic(2, seed=nc, num_cameras=nc, num_points=40 * nc, max_track=min(8, nc))
+    ref = oracle_mod.solve(p.num_cameras(), p.num_points(), p.camera_index(), p.point_index(), p.observations(),
+                           p.cameras(), p.points(), oracle_mod.default_options(**kw))
+    out = S.SolveBA(p, linear_solver=C.SOLVER_DENSE_SCHUR, precision=C.PRECISION_MIXED if mixed else C.PRECISION_FP64, **kw)
+    assert out["num_successful_steps"] == sum(t["step_is_successful"] for t in ref["trace"][1:])
+    return out, ref, p
+
+
+# Past one workgroup's 198 unknowns the system is padded to 64 x 64 blocks: 207 unknowns (the first), 576 and 1152 (9
+# and 18 blocks exactly), 639 (one short of 10); the sweeps' blocks of 512 rows end inside the first of them
+# and after 8 and 16 blocks.
+@pytest.mark.parametrize("nc", [23, 64, 71, 128])
+def test_dense_block_edges_match_oracle(oracle_mod, nc):
+    out, ref, p = _against_oracle(oracle_mod, nc, False, **FIXED)
+    # as above: at most 1e7 in condition times unit roundoff, per step
+    assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-8 * ref["final_cost"]
+    np.testing.assert_allclose(p.cameras(), ref["cams"], rtol=0, atol=1e-7 * np.abs(ref["cams"]).max())
+
+
+# The FP32 factor (from 289 unknowns on) at the same edges and at 297, 513 and 1026 (4, 8 and 16 blocks and
+# something).  Well damped, so that the steps are the factor's and not the rounding of the FP32 Jacobians along
+# weak directions: D^2 is the diagonal, a third and a ninth of it.
+@pytest.mark.parametrize("nc", [33, 57, 64, 71, 114, 128])
+def test_dense_mixed_block_edges_match_oracle(oracle_mod, nc):
+    start = S.synthetic(2, seed=nc, num_cameras=nc, num_points=40 * nc, max_track=min(8, nc)).cameras().copy().reshape(-1, 9)
+    out, ref, p = _against_oracle(oracle_mod, nc, True, **dict(FIXED, initial_trust_region_radius=1.0))
+    # FP32 Jacobian entries are right to 1e-5 (roundings of 6e-8 and the cancellation in a projection), the condition
+    # of the damped, scaled system is at most 100: 1e-3 of the step in each kind of parameter, and so of the
+    # decrease
+    step = np.abs(ref["cams"].reshape(-1, 9) - start).max(axis=0)
+    assert (np.abs(p.cameras().reshape(-1, 9) - ref["cams"].reshape(-1, 9)).max(axis=0) <= 1e-3 * step).all()
+    assert abs(out["final_cost"] - ref["final_cost"]) <= 1e-3 * (ref["initial_cost"] - ref["final_cost"])
