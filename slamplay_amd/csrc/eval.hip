@@ -3,7 +3,8 @@
 // utils/camera/SnavelyReprojectionError.h:42-92), and the FP64 cost 1/2 sum rho(|r|^2).
 //
 // Layout: observations in caller order; cameras AoS (9 doubles) as in BALProblem.  One thread per
-// observation, camera prep computed once per camera by k_camera_prep_aos.
+// observation.  The Jacobian entry's camera preps are computed once per camera by k_camera_prep_aos; the cost
+// has eleven terms per camera of its own (CostCam).
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -55,9 +56,9 @@ __global__ void k_eval_obs(int no, const int* __restrict__ ci, const int* __rest
 //   kCostPrep   up to 256 cameras: every block computes them into its LDS, one camera per thread, and no
 //               launch of its own is needed;
 //   kCostGather beyond: computed once by k_cost_cameras, gathered from memory, 88 contiguous bytes each.
-// 1.2M observations of 1,500 cameras: 40.1 -> 18.6 us a call (a copy of the whole table in every CU's
-// LDS, 132 KB: 19.4); 14.9k observations of 16 cameras: 12.7 -> 9.7 us, the rate the host issues two
-// launches at.
+// 1.2M observations of 1,500 cameras: 40 -> 22 us a call on inputs that the caches still hold, 49.5 -> 28.6 on
+// twelve sets of them in turn, 430 MB (a copy of the whole table in every CU's LDS, 132 KB, instead of the
+// gather: 1 us more); 14.9k observations of 16 cameras: 12.7 -> 9.7 us, the rate the host issues two launches at.
 struct CostCam {
     double u[3], c, s;   // R X = X c + (u x X) s + u (u.X)(1 - c)
     double t[3], f, k1, k2;

@@ -12,8 +12,9 @@ namespace mba {
 constexpr int kTile = 32;
 
 // 1 / sqrt(d) for the pivot chain: the hardware estimate r and one third-order step r (1 + e / 2 + 3 e^2 / 8),
-// e = 1 - d r^2 (four dependent operations; the 23 correct bits of the FP64 estimate become 69, the FP32
-// one's error is squared twice over).
+// e = 1 - d r^2, four dependent operations.  The step leaves out 5 e^3 / 16 and more: 2^-67 of the result for the
+// FP64 estimate's 23 bits (|e| < 2^-22), and less for the FP32 one's, so the result is as good as
+// the roundings of the step itself, about one unit in the last place.
 __device__ __forceinline__ double pivot_rsqrt(double d) {
     const double r = __builtin_amdgcn_rsq(d), e = fma(-d * r, r, 1.0);
     return fma(r * e, fma(e, 0.375, 0.5), r);
