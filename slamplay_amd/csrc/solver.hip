@@ -350,7 +350,7 @@ struct Solver final : SolverBase {
         BA_TRY(pt_c.alloc(4 * (size_t)np));
         BA_TRY(dcam.alloc(9 * (size_t)nc));
         BA_TRY(dpt.alloc(4 * (size_t)np));
-        BA_TRY(params_out.alloc(9 * (size_t)nc + 3 * (size_t)np));
+        BA_TRY(params_out.alloc(std::max(9 * (size_t)nc + 3 * (size_t)np, kLongCopyBytes / sizeof(double))));
         BA_TRY(prep.alloc(nc));
         BA_TRY(prep_c.alloc(nc));
         for (DevBuf<double>* b : {&M, &Minv}) BA_TRY(b->alloc(81 * (size_t)nc));
@@ -481,19 +481,32 @@ struct Solver final : SolverBase {
         return BA_OK;
     }
 
-    // The caller's layouts are formed on the device and copied straight into the caller's arrays: 370 -> 200 us for
-    // 1,500 cameras and 100k points, against staging vectors and a permutation on the host.  They have a
-    // buffer of their own: another thread may run the solver meanwhile, and the step buffers are in use between
-    // the launches of an iteration.
+    // The caller's layouts are formed on the device and copied: 370 -> 200 us for 1,500 cameras and 100k points,
+    // against staging vectors and a permutation on the host.  They have a buffer of their own: another thread may
+    // run the solver meanwhile, and the step buffers are in use between the launches of an iteration.  The copies'
+    // fixed cost is most of a small download, so up to kOneCopyBytes both arrays come in one, through a host
+    // vector; and behind a kernel the runtime copies up to 64 KB at 2.4 GB/s, beyond much faster, so above
+    // kShortCopyBytes kLongCopyBytes of the buffer are copied at least.  20 / 1,000 / 2,000 / 4,000 / 10,000 points
+    // 26 / 31 / 32 / 30 / 37 us (35, 45, 38, 40, 52 by the host; by two copies behind the kernel 38, 45, 55, 39, 44).
+    static constexpr size_t kOneCopyBytes = 256 << 10, kShortCopyBytes = 12 << 10, kLongCopyBytes = 66 << 10;
     int download(double* cams, double* pts) override {
         const int nc = L.nc, np = L.np;
         BA_TRY(use_device(device));  // a launch, unlike a copy, needs the stream's device to be the thread's current one
-        double *const out_c = params_out.p, *const out_p = params_out.p + 9 * (size_t)nc;
-        hipLaunchKernelGGL(k_params_out, dim3(std::max(1, div_up(std::max(9 * (int64_t)nc, 3 * (int64_t)np), kWG))), dim3(kWG),
-                           0, s, (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, out_c, out_p);
+        const size_t n_cam = 9 * (size_t)nc, n_pt = 3 * (size_t)np, bytes = (n_cam + n_pt) * sizeof(double);
+        double *const out_c = params_out.p, *const out_p = params_out.p + n_cam;
+        hipLaunchKernelGGL(k_params_out, dim3(std::max(1, div_up((int64_t)std::max(n_cam, n_pt), kWG))), dim3(kWG), 0, s,
+                           (const double*)cam_x.p, nc, (const double*)pt_x.p, (const int*)pt_orig.p, np, out_c, out_p);
         BA_HIP(hipGetLastError());
-        if (cams && nc) BA_HIP(hipMemcpyAsync(cams, out_c, 9 * (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, s));
-        if (pts && np) BA_HIP(hipMemcpyAsync(pts, out_p, 3 * (size_t)np * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (bytes > 0 && bytes <= kOneCopyBytes) {
+            std::vector<double> host((bytes <= kShortCopyBytes ? bytes : std::max(bytes, kLongCopyBytes)) / sizeof(double));
+            BA_HIP(hipMemcpyAsync(host.data(), params_out.p, host.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+            BA_HIP(hipStreamSynchronize(s));
+            if (cams) std::copy(host.begin(), host.begin() + n_cam, cams);
+            if (pts) std::copy(host.begin() + n_cam, host.begin() + n_cam + n_pt, pts);
+            return BA_OK;
+        }
+        if (cams && nc) BA_HIP(hipMemcpyAsync(cams, out_c, n_cam * sizeof(double), hipMemcpyDeviceToHost, s));
+        if (pts && np) BA_HIP(hipMemcpyAsync(pts, out_p, n_pt * sizeof(double), hipMemcpyDeviceToHost, s));
         BA_HIP(hipStreamSynchronize(s));
         return BA_OK;
     }

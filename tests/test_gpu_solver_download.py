@@ -2,6 +2,7 @@
 another thread runs the solver."""
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -58,3 +59,41 @@ def test_downloads_beside_a_run_do_not_change_it(solver):
         t.join()
     sv.close()
     assert reads[0] > 0
+
+
+def _points_only(n):
+    rng = np.random.default_rng(n)
+    cams = np.array([0.1, -0.2, 0.05, 0.3, -0.1, -5.0, 500.0, 0.0, 0.0])
+    pts = rng.normal(0, 3, 3 * n)
+    return cams, pts, S.BALProblem.from_arrays(np.zeros(n, np.int32), rng.permutation(n).astype(np.int32), np.zeros((n, 2)), cams, pts)
+
+
+# bytes below, at and above 12 KB (509 points), 66 KB (2,813) and 256 KB (10,919)
+@pytest.mark.parametrize("n", [1, 508, 509, 510, 2812, 2813, 2814, 10919, 10920, 20000])
+def test_download_sizes(n):
+    cams, pts, p = _points_only(n)
+    sv = S.Solver(p)
+    c, x = sv.download()
+    np.testing.assert_array_equal(c, cams)
+    np.testing.assert_array_equal(x, pts)
+    for which in (0, 1):  # one of the two arrays only
+        out = np.full(9 if which == 0 else 3 * n, np.nan)
+        ptr = out.ctypes.data_as(C.f64p)
+        C.check(C.lib().ba_solver_download(sv._h, ptr if which == 0 else None, ptr if which == 1 else None))
+        np.testing.assert_array_equal(out, (cams, pts)[which])
+    sv.close()
+
+
+def test_download_time_does_not_fall_with_size():
+    def median_us(n):
+        sv = S.Solver(_points_only(n)[2])
+        t = []
+        for _ in range(100):
+            start = time.perf_counter()
+            sv.download()
+            t.append(time.perf_counter() - start)
+        sv.close()
+        return 1e6 * float(np.median(t))
+
+    # as two copies behind the kernel, 2,000 points took half as long again as 3,000
+    assert median_us(2000) < 1.3 * median_us(3000)
