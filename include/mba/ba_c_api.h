@@ -245,7 +245,9 @@ int ba_stereo_batch_solve(const ba_stereo_view* windows, int32_t count, const ba
 
 /* Device-resident solver: create uploads the problem and builds the device layout once; run solves
  * from the parameters currently held on the device; reset restores the parameters given at create;
- * download copies the device parameters to host AoS arrays. */
+ * download copies the device parameters to host AoS arrays (either pointer may be NULL).  While another
+ * thread is inside run it may be called with launch_mode 1 only (the default mode records the stream's launches
+ * into a graph); it then returns the parameters some iteration holds and leaves the run as it is. */
 typedef struct ba_solver ba_solver;
 int ba_solver_create(const ba_problem_view* problem, const ba_options* options, ba_solver** out);
 int ba_solver_run(ba_solver* solver, ba_summary* summary);
@@ -293,6 +295,8 @@ int ba_batch_create(const ba_problem_view* windows, int32_t count, const ba_opti
  * is the time from the start of the run to the moment that window finished on the device. */
 int ba_batch_run(ba_batch* batch, ba_summary* summaries);
 int ba_batch_reset(ba_batch* batch);
+/* Threads may download side by side.  What is fetched ahead of a caller who reads on in order, and all windows
+ * once single reads have cost as much, is kept on the host until the parameters change. */
 int ba_batch_download(ba_batch* batch, int32_t window, double* cameras, double* points);
 int ba_batch_destroy(ba_batch* batch);
 /* One-shot: create, run, write every window's parameters back in place, destroy. */
