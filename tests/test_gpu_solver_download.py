@@ -95,5 +95,5 @@ def test_download_time_does_not_fall_with_size():
         sv.close()
         return 1e6 * float(np.median(t))
 
-    # as two copies behind the kernel, 2,000 points took half as long again as 3,000
-    assert median_us(2000) < 1.3 * median_us(3000)
+    # as two copies behind the kernel, 2,000 points took half as long again as 3,000; now 32 us against 29
+    assert median_us(2000) < 1.4 * median_us(3000)
